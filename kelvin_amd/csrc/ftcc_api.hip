@@ -921,10 +921,16 @@ void ensure_fixed_operands(ftcc_ctx *c) {
 }
 
 // Pairs of (lx, ly) grouped by class 2*lx + ly in `order`, each class padded
-// to a multiple of 256 (the product tile).
+// to a multiple of PAIR_PAD: the K slab of the split-bf16 product, the
+// coarsest alignment that a class range has to have (rows and columns past
+// the end of a tile are dropped by the products themselves).  Padding to
+// the 256 of the product tile multiplied the work of small systems: at
+// n = 38 the classes of 171 and 361 pairs ran as 256 and 512, 2.9 times the
+// products.
 // packed (lx and ly the same list): only x < y within a class of equal
 // spins, class 01 whole and class 10 empty -- one pair of each
 // antisymmetric couple.
+constexpr int PAIR_PAD = 32;
 PairSpace build_pairs(ftcc_ctx *c, const std::vector<int> &lx,
                       const std::vector<int> &ly, const int order[4],
                       bool packed = false) {
@@ -943,7 +949,7 @@ PairSpace build_pairs(ftcc_ctx *c, const std::vector<int> &lx,
           ++cnt;
         }
     }
-    while (map.size() % 256) map.push_back(-1);
+    while (map.size() % PAIR_PAD) map.push_back(-1);
     ps.count[cls] = cnt;
     ps.len[cls] = (int)map.size() - ps.start[cls];
   }

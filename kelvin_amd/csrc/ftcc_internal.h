@@ -115,7 +115,7 @@ struct SplitMat {
 // Spin-class ordering of a pair space (x, y), x from a set with spin labels
 // lx, y from a set with labels ly: pairs are grouped by class
 // c = 2*lx[x] + ly[y] in a chosen class order, lexicographic inside a class,
-// and each class is padded to a multiple of 256.  map[r] is the flat pair
+// and each class is padded to a multiple of 32.  map[r] is the flat pair
 // index x*ny + y of blocked position r (-1 for padding).
 struct PairSpace {
   int total = 0;

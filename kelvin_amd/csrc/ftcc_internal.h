@@ -84,10 +84,9 @@ struct Gemm {
   const int *mmap = nullptr, *nmap = nullptr;
   int mlvl = -1, nlvl = -1;
   int64_t sAk0 = 0, sAk1 = 0, sBk0 = 0, sBk1 = 0;
-  // launch plan: tile shape policy (0 by the shape: narrow tiles when one
-  // dimension is at most 64 or K is; 1 wide: 128x128 unless one dimension is
-  // at most 64; 2 narrow: 128x64 or 64x128 by the aspect) and the workgroup
-  // count below which K is split
+  // launch plan: tile shape policy (0 by the estimated time; 1 wide: 128x128
+  // unless one dimension is at most 64; 2 narrow: never 128x128) and the
+  // workgroup count up to which K may be split
   int tile_policy = 0;
   int split_target = 1024;
 };

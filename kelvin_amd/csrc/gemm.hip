@@ -1,9 +1,13 @@
 // Batched strided GEMM on the CDNA4 matrix cores.
 //
-// One workgroup = 4 wave64s computes a 128x128 tile of C; each wave owns a
-// 64x64 quadrant as 4x4 MFMA 16x16 blocks.  K advances in slabs of 16 staged
-// through LDS (double buffered, one barrier per slab) with the next slab
-// prefetched into registers while the current one feeds the MFMAs.
+// One workgroup = 4 wave64s computes a tile of C of 128x128 to 64x64; each
+// wave owns a quadrant as 16x16 MFMA blocks.  K advances in slabs of 16 staged
+// through LDS (the largest tile double buffered, one barrier per slab) with
+// the next slab prefetched into registers while the current one feeds the
+// MFMAs.  The tile and the splits of K are the pair of least estimated time
+// (plan_of).  Measured, FP64, K contiguous in both operands: 4096^3 52 to 55
+// TFLOP/s with every tile; 15 of 722^3 42 with 64x64, 30 with 128x128; one
+// 361x722x722 in 59 us with 64x64, 30 us with its K split as well.
 //
 // LDS holds both operands "K-inner": As[m][k], Bs[n][k], rows padded so the
 // 16 lanes that share a k-group hit distinct banks.  Inside a slab the
@@ -26,6 +30,7 @@
 #include "ftcc_internal.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace ftcc {
 namespace {
@@ -36,21 +41,10 @@ typedef double d2_t __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 16, NT = 256;
 
-// Output tile: 128x128, or 64 on the side of a dimension of at most 64
-// (products over one spin run of an orbital index)
+// Output tile: 128x128, 128x64, 64x128 or 64x64
 struct Tile {
   int m, n;
 };
-// Short K (the O(n^5) contractions over one index): the narrow,
-// single-buffered tiles (three workgroups per CU) stream the output faster
-// than 128x128 (3.5% on those launches at n = 114).
-inline Tile pick_tile(int M, int N, int K, int policy) {
-  if (M <= 64 && N > 64) return {64, 128};
-  if (N <= 64 && M > 64) return {128, 64};
-  if (policy == 2 || (policy == 0 && K <= 64))
-    return M >= N ? Tile{128, 64} : Tile{64, 128};
-  return {128, 128};
-}
 
 struct GemmDev {
   int M, N, K, nb1, nb2, splits, kchunk, tilesM, tilesN;
@@ -257,7 +251,7 @@ __device__ inline void load4(const T *src, T out[4]) {
   for (int s = 0; s < 4; ++s) out[s] = src[s];
 }
 
-// TM x TN output tile per workgroup (128x128, 64x128 or 128x64): the four
+// TM x TN output tile per workgroup (128x128 down to 64x64): the four
 // waves form a 2x2 grid, each owning (TM/2) x (TN/2) as RT x CT MFMA blocks.
 template <typename T, bool A_MFAST, bool B_NFAST, int TM, int TN, bool KL>
 __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmDev p) {
@@ -431,8 +425,29 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmDev p) {
   }
 }
 
-// C[b][m,n] = alpha * sum_r partial[r][b][m][n] + beta*C  (fixed order)
-// Sum of the R split-K partials of each output element, then the epilogue.
+// Epilogue of one element of a split product: C[b][m,n] = alpha * s + gamma
+// * D + beta * C through the scatter maps.
+__device__ inline void put_sum(const GemmDev &p, int64_t cb, int64_t mn,
+                               double s) {
+  const int m0 = (int)(mn / p.N), n0 = (int)(mn % p.N);
+  const int m = p.rmap ? p.rmap[m0] : m0, n = p.cmap ? p.cmap[n0] : n0;
+  if (m < 0 || n < 0) return;
+  const int64_t b1 = p.reduce_b2 ? cb : cb / p.nb2;
+  const int64_t b2 = p.reduce_b2 ? 0 : cb % p.nb2;
+  const Lvl lr = map_level(levels(m, p.M1, p.M2), p.mmap, p.mlvl),
+            lc = map_level(levels(n, p.N1, p.N2), p.nmap, p.nlvl);
+  double *c = p.C + b1 * p.sC1 + b2 * p.sC2 +
+              at(lr, p.sCm0, p.sCm1, p.sCm) + at(lc, p.sCn0, p.sCn1, p.sCn);
+  double y = p.alpha * s;
+  if (p.D)
+    y += p.gamma * p.D[b1 * p.sD1 + b2 * p.sD2 +
+                       at(lr, p.sDm0, p.sDm1, p.sDm) +
+                       at(lc, p.sDn0, p.sDn1, p.sDn)];
+  if (p.beta != 0.0) y += p.beta * *c;
+  *c = y;
+}
+
+// C[b][m,n] = alpha * sum_r partial[r][b][m][n] + beta*C  (fixed order).
 // A block of RG x 64 threads takes 64 consecutive elements (coalesced rows
 // of the partial buffer); its RG groups sum interleaved partials (several
 // loads in flight per thread) and combine in LDS, so that even a small
@@ -468,45 +483,92 @@ __global__ __launch_bounds__(64 * RG) void reduce_partial_kernel(GemmDev p,
       double s = 0.0;
 #pragma unroll
       for (int q = 0; q < RG; ++q) s += part[q][lane];
-      const int m0 = (int)(mn / p.N), n0 = (int)(mn % p.N);
-      const int m = p.rmap ? p.rmap[m0] : m0, n = p.cmap ? p.cmap[n0] : n0;
-      if (m >= 0 && n >= 0) {
-        int64_t b1, b2;
-        if (p.reduce_b2) {
-          b1 = cb;
-          b2 = 0;
-        } else {
-          b1 = cb / p.nb2;
-          b2 = cb % p.nb2;
-        }
-        const Lvl lr = map_level(levels(m, p.M1, p.M2), p.mmap, p.mlvl),
-                  lc = map_level(levels(n, p.N1, p.N2), p.nmap, p.nlvl);
-        double *c = p.C + b1 * p.sC1 + b2 * p.sC2 +
-                    at(lr, p.sCm0, p.sCm1, p.sCm) +
-                    at(lc, p.sCn0, p.sCn1, p.sCn);
-        double y = p.alpha * s;
-        if (p.D)
-          y += p.gamma * p.D[b1 * p.sD1 + b2 * p.sD2 +
-                             at(lr, p.sDm0, p.sDm1, p.sDm) +
-                             at(lc, p.sDn0, p.sDn1, p.sDn)];
-        if (p.beta != 0.0) y += p.beta * *c;
-        *c = y;
-      }
+      put_sum(p, cb, mn, s);
     }
     __syncthreads();
   }
 }
 
-int choose_splits(const Gemm &g, int tiles, int bk) {
-  // Few output tiles over a long K (the O(n^5) contractions onto n x n
-  // matrices) stream their operands from HBM once: split K until ~4
-  // workgroups per CU keep enough loads in flight; >= 8 slabs per split.
-  const int64_t blocks = (int64_t)tiles * g.nb1 * g.nb2;
-  const int64_t target = std::max(1, g.split_target);
-  if (blocks >= target) return 1;
-  const int maxs = std::max(1, g.K / (8 * bk));
-  int want = (int)((target + blocks - 1) / blocks);
-  return std::max(1, std::min(want, std::min(maxs, 2048)));
+// The same for few partials: one thread per element, which sums them in
+// order with all its loads in flight (the form above leaves RG - R of its
+// RG groups idle).
+constexpr int FEW = 12;
+__global__ __launch_bounds__(256) void reduce_few_kernel(GemmDev p, int R) {
+  const int64_t MN = (int64_t)p.M * p.N;
+  const int64_t total = MN * p.nbC;
+  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total;
+       idx += (int64_t)gridDim.x * 256) {
+    double v[FEW];
+#pragma unroll
+    for (int r = 0; r < FEW; ++r)
+      v[r] = p.partial[(int64_t)(r < R ? r : 0) * total + idx];
+    double s = v[0];
+#pragma unroll
+    for (int r = 1; r < FEW; ++r) s += r < R ? v[r] : 0.0;
+    put_sum(p, idx / MN, idx % MN, s);
+  }
+}
+
+// Tile shape and K splits of a product: the pair with the least estimated
+// time.  Per CU a workgroup's slab takes the time of its MFMAs, and a CU
+// works through its workgroups of a launch at that rate or at that of the
+// load latency of its resident ones, whichever is longer; splitting K adds
+// the partial sums' write and read.  (Splitting every launch of fewer than
+// 1024 workgroups, as this rule did before, spent half of an FP64 step at
+// n = 54 in the sums of partials: 7.4 of 14.4 ms.)
+struct Plan {
+  Tile t;
+  int splits;
+};
+double estimate_us(const Gemm &g, Tile t, int splits) {
+  const double tiles = (double)((g.M + t.m - 1) / t.m) *
+                       ((g.N + t.n - 1) / t.n) * g.nb1 * g.nb2;
+  const int occ = t.m * t.n >= 128 * 128 ? 2 : (t.m * t.n >= 8192 ? 3 : 4);
+  const double slabs = std::ceil(std::ceil(g.K / (double)BK) / splits);
+  // one slab of the tile on a CU's four matrix cores, us, and the time
+  // from a slab's loads to its use
+  const double ts = 1.9 * t.m * t.n / (128.0 * 128.0), lat = 1.2;
+  const double b = tiles * splits;
+  const double us =
+      (slabs + 2.0) * std::max(std::ceil(b / 256.0) * ts,
+                               std::ceil(b / (256.0 * occ)) * lat);
+  const double R = splits * (g.reduce_b2 ? (double)g.nb2 : 1.0);
+  const double out = (double)g.M * g.N * g.nb1 * g.nb2 * 8e-6;   // MB
+  const double sum = R > 1.0 ? 4.0 + out * (splits * 2.0 + 1.0) / 3.0 : 0.0;
+  return us + sum;
+}
+Plan plan_of(const Gemm &g) {
+  const int pol = g.tile_policy;
+  const Tile cand[4] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
+  Plan best{{128, 128}, 1};
+  double us = 1e300;
+  for (int q = 0; q < 4; ++q) {
+    const Tile t = cand[q];
+    // a side of at most 64 takes no 128-wide tile
+    if ((g.M <= 64 && t.m > 64) || (g.N <= 64 && t.n > 64)) continue;
+    if (pol == 1 && ((g.M > 64 && t.m < 128) || (g.N > 64 && t.n < 128)))
+      continue;
+    if (pol == 2 && t.m * t.n == 128 * 128) continue;
+    // short K (the O(n^5) contractions over one index): the single-buffered
+    // tiles (three or more workgroups per CU) stream the output faster than
+    // 128x128 (3.5% on those launches at n = 114)
+    if (pol == 0 && g.K <= 64 && t.m * t.n == 128 * 128) continue;
+    const int64_t blocks = (int64_t)((g.M + t.m - 1) / t.m) *
+                           ((g.N + t.n - 1) / t.n) * g.nb1 * g.nb2;
+    const int64_t want =
+        (std::max(1, g.split_target) + blocks - 1) / blocks;
+    const int maxs = (int)std::max<int64_t>(
+        1, std::min<int64_t>(std::min<int64_t>(want, 2048),
+                             g.K / (4 * BK)));
+    for (int sp = 1; sp <= maxs; sp += 1 + sp / 8) {
+      const double e = estimate_us(g, t, sp);
+      if (e < us * 0.98) {
+        us = e;
+        best = Plan{t, sp};
+      }
+    }
+  }
+  return best;
 }
 
 template <typename K3>
@@ -531,7 +593,8 @@ void launch_tile(bool amf, bool bnf, bool kl, const GemmDev &d,
 template <typename T>
 void launch_layout(Tile tl, bool amf, bool bnf, bool kl, const GemmDev &d,
                    hipStream_t s) {
-  if (tl.m == 64) launch_tile<T, 64, 128>(amf, bnf, kl, d, s);
+  if (tl.m == 64 && tl.n == 64) launch_tile<T, 64, 64>(amf, bnf, kl, d, s);
+  else if (tl.m == 64) launch_tile<T, 64, 128>(amf, bnf, kl, d, s);
   else if (tl.n == 64) launch_tile<T, 128, 64>(amf, bnf, kl, d, s);
   else launch_tile<T, 128, 128>(amf, bnf, kl, d, s);
 }
@@ -539,11 +602,7 @@ void launch_layout(Tile tl, bool amf, bool bnf, bool kl, const GemmDev &d,
 }  // namespace
 
 size_t gemm_partial_elems(const Gemm &g) {
-  const Tile tl = pick_tile(g.M, g.N, g.K, g.tile_policy);
-  const int tiles = ((g.M + tl.m - 1) / tl.m) * ((g.N + tl.n - 1) / tl.n);
-  const int bk = BK;  // conservative: smallest slab gives the most splits
-  const int splits = choose_splits(g, tiles, bk);
-  const int R = splits * (g.reduce_b2 ? g.nb2 : 1);
+  const int R = (g.K > 0 ? plan_of(g).splits : 1) * (g.reduce_b2 ? g.nb2 : 1);
   if (R <= 1) return 0;
   const int nbC = g.reduce_b2 ? g.nb1 : g.nb1 * g.nb2;
   return (size_t)R * nbC * g.M * g.N;
@@ -578,7 +637,8 @@ void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
   d.sCn = g.sCn;
   d.sC1 = g.sC1;
   d.sC2 = g.sC2;
-  const Tile tl = pick_tile(g.M, g.N, g.K, g.tile_policy);
+  const Plan pl = plan_of(g);
+  const Tile tl = pl.t;
   d.tilesM = (g.M + tl.m - 1) / tl.m;
   d.tilesN = (g.N + tl.n - 1) / tl.n;
   d.m_inner = d.tilesM < d.tilesN ? 1 : 0;
@@ -587,7 +647,7 @@ void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
     d.splits = 1;
     d.kchunk = 0;
   } else {
-    d.splits = choose_splits(g, d.tilesM * d.tilesN, BK);
+    d.splits = pl.splits;
     // round the chunk to whole slabs of the active precision
     int kc = (g.K + d.splits - 1) / d.splits;
     kc = ((kc + bk - 1) / bk) * bk;
@@ -664,9 +724,16 @@ void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
     launch_layout<float>(tl, amf, bnf, kl, d, s);
   if (R > 1) {
     const int64_t total = (int64_t)d.nbC * g.M * g.N;
-    const int blocks = (int)std::min<int64_t>((total + 63) / 64, 65536);
-    hipLaunchKernelGGL(reduce_partial_kernel, dim3(blocks), dim3(64 * RG), 0,
-                       s, d, R);
+    // few partials of a large output: a thread for each element
+    if (R <= FEW && total >= 32 * 1024) {
+      const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65536);
+      hipLaunchKernelGGL(reduce_few_kernel, dim3(blocks), dim3(256), 0, s, d,
+                         R);
+    } else {
+      const int blocks = (int)std::min<int64_t>((total + 63) / 64, 65536);
+      hipLaunchKernelGGL(reduce_partial_kernel, dim3(blocks), dim3(64 * RG),
+                         0, s, d, R);
+    }
     FTCC_CHECK_HIP(hipGetLastError());
   }
 }

@@ -107,11 +107,12 @@ __global__ void sum4_kernel(const double *partials, int nblocks,
 
 // tau = t2 + t1[a,i]t1[b,j] - t1[b,i]t1[a,j], taut = t2 + (...)/2,
 // ar = t2/2 + t1[a,i]t1[b,j] (the ring amplitude of Wmbej, [f,b,j,n])
-__global__ void tau_kernel(const double *t1, const double *t2, int V, int O,
-                           double *tau, double *taut, double *ar) {
+__global__ void tau_kernel(const double *t1s, const double *t2, int V, int O,
+                           int nb, double *tau, double *taut, double *ar) {
   const int64_t n = (int64_t)V * V * O * O;
-  ADJ_LOOP(e, n) {
-    int64_t r = e;
+  ADJ_LOOP(e, n * nb) {
+    const double *t1 = t1s + e / n * ((int64_t)V * O);
+    int64_t r = e % n;
     const int j = (int)(r % O);
     r /= O;
     const int i = (int)(r % O);
@@ -140,21 +141,22 @@ __device__ inline double proj(const double *x, int a, int b, int i, int j,
 // (the transposed residual is projected onto antisymmetric tensors) and
 // the adjoint of tau/taut for the t1 chain rule
 __global__ void assemble_kernel(const double *acc, const double *gtau,
-                                const double *gt, int V, int O, double *S,
-                                double *out2) {
+                                const double *gt, int V, int O, int nb,
+                                double *S, double *out2) {
   const int64_t n = (int64_t)V * V * O * O;
-  ADJ_LOOP(e, n) {
-    int64_t r = e;
+  ADJ_LOOP(e, n * nb) {
+    const int64_t y = e / n * n;
+    int64_t r = e - y;
     const int j = (int)(r % O);
     r /= O;
     const int i = (int)(r % O);
     r /= O;
     const int b = (int)(r % V);
     const int a = (int)(r / V);
-    const double pt = proj(gt, a, b, i, j, V, O);
-    const double s = proj(gtau, a, b, i, j, V, O) + 0.5 * pt;
+    const double pt = proj(gt + y, a, b, i, j, V, O);
+    const double s = proj(gtau + y, a, b, i, j, V, O) + 0.5 * pt;
     S[e] = s;
-    out2[e] = proj(acc, a, b, i, j, V, O) + 0.5 * pt + s;
+    out2[e] = proj(acc + y, a, b, i, j, V, O) + 0.5 * pt + s;
   }
 }
 
@@ -361,6 +363,7 @@ struct Ten {
   std::string l;
   std::vector<int64_t> st;
   std::string rule;   // spin rule: letters left of '|' sum to those right
+  int64_t bs = 0;     // stride between grid points (0: shared by all)
   int64_t stride(char x) const {
     const size_t k = l.find(x);
     return k == std::string::npos ? -1 : st[k];
@@ -397,6 +400,14 @@ Ten ten(const ftcc_ctx *c, const double *p, const char *letters,
   } else if (t.l.size() == 2) {
     t.rule = t.l.substr(0, 1) + "|" + t.l.substr(1, 1);
   }
+  return t;
+}
+
+// the same with one tensor per grid point, one after another
+Ten bten(const ftcc_ctx *c, const double *p, const char *letters,
+         const char *rule = nullptr) {
+  Ten t = ten(c, p, letters, rule);
+  t.bs = t.st[0] * letter_dim(c, t.l[0]);
   return t;
 }
 
@@ -526,10 +537,11 @@ Shape shape_of(const Extents &ext, const Ten &A0, const Ten &B0,
   return best;
 }
 
-// The GEMM of C = alpha A.B + beta C over the letter extents `ext`, or
-// false when no level order satisfies the engine's layout rules.
+// The GEMM of C = alpha A.B + beta C over the letter extents `ext` at nb
+// grid points, or false when no level order satisfies the engine's layout
+// rules.
 bool plan(const Extents &ext, double alpha, const Ten &A0, const Ten &B0,
-          double beta, const Ten &C, const Groups &G, Gemm &g) {
+          double beta, const Ten &C, const Groups &G, int nb, Gemm &g) {
   const Shape best = shape_of(ext, A0, B0, C, G);
   if (best.score < 0) return false;
   const Ten &A = best.swap ? B0 : A0, &B = best.swap ? A0 : B0;
@@ -539,7 +551,10 @@ bool plan(const Extents &ext, double alpha, const Ten &A0, const Ten &B0,
   g.A = A.p;
   g.B = B.p;
   g.C = const_cast<double *>(C.p);
-  g.nb1 = 1;
+  g.nb1 = nb;
+  g.sA1 = A.bs;
+  g.sB1 = B.bs;
+  g.sC1 = C.bs;
   auto prod = [](const std::vector<Level> &v) {
     int64_t s = 1;
     for (const Level &L : v) s *= L.dim;
@@ -634,11 +649,14 @@ __device__ inline int64_t pack_off(int x, const PackIdx &l) {
 }
 // dst[r][k] (row length K) = src(r, k): rows along the thread index when the
 // source is contiguous along rows (through a 32x32 LDS tile), else along k.
+// (slice blockIdx.z: src + z * sb into dst + z * R * K)
 __global__ __launch_bounds__(256) void pack_kernel(const double *src,
                                                    PackIdx rl, PackIdx kl,
                                                    int R, int K, double *dst,
-                                                   int along_r) {
+                                                   int along_r, int64_t sb) {
   __shared__ double tile[32][33];
+  src += blockIdx.z * sb;
+  dst += (int64_t)blockIdx.z * R * K;
   const int r0 = blockIdx.y * 32, k0 = blockIdx.x * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   if (along_r) {
@@ -673,10 +691,11 @@ PackIdx pack_levels(int n1, int n2, int64_t s0, int64_t s1, int64_t s) {
 // is left as it is (small, already contiguous, batched or level-mapped).
 bool pack_block(ftcc_ctx *c, Gemm &g) {
   const double flops = 2.0 * g.M * (double)g.N * g.K;
-  if (flops < 1e9 || g.nb1 != 1 || g.nb2 != 1 || g.mmap || g.nmap)
-    return false;
+  if (flops < 1e9 || g.nb2 != 1 || g.mmap || g.nmap) return false;
   if (g.sAk == 1 && g.sBk == 1 && g.K2 == 0) return false;
-  const int64_t need = ((int64_t)g.M + g.N) * g.K;
+  // an operand shared by the grid points is copied once
+  const int na = g.sA1 ? g.nb1 : 1, nbb = g.sB1 ? g.nb1 : 1;
+  const int64_t need = ((int64_t)g.M * na + (int64_t)g.N * nbb) * g.K;
   if (need > c->pack_elems) {
     FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
     dfree(c, c->pack_buf);
@@ -685,20 +704,21 @@ bool pack_block(ftcc_ctx *c, Gemm &g) {
     c->pack_buf = dalloc(c, need);
     c->pack_elems = need;
   }
-  double *pa = c->pack_buf, *pb = c->pack_buf + (int64_t)g.M * g.K;
+  double *pa = c->pack_buf, *pb = c->pack_buf + (int64_t)g.M * na * g.K;
   const PackIdx kA = pack_levels(g.K1, g.K2, g.sAk0, g.sAk1, g.sAk);
   const PackIdx kB = pack_levels(g.K1, g.K2, g.sBk0, g.sBk1, g.sBk);
   const PackIdx rA = pack_levels(g.M1, g.M2, g.sAm0, g.sAm1, g.sAm);
   const PackIdx rB = pack_levels(g.N1, g.N2, g.sBn0, g.sBn1, g.sBn);
   require(g.M < (1 << 30) && g.N < (1 << 30) && g.K < (1 << 30),
           "pack: operand too large");
-  const dim3 ga((g.K + 31) / 32, (g.M + 31) / 32), gb((g.K + 31) / 32,
-                                                     (g.N + 31) / 32);
-  require(ga.y < 65536 && gb.y < 65536, "pack: grid too large");
+  const dim3 ga((g.K + 31) / 32, (g.M + 31) / 32, na),
+      gb((g.K + 31) / 32, (g.N + 31) / 32, nbb);
+  require(ga.y < 65536 && gb.y < 65536 && g.nb1 < 65536,
+          "pack: grid too large");
   hipLaunchKernelGGL(pack_kernel, ga, dim3(256), 0, c->stream, g.A, rA, kA,
-                     g.M, g.K, pa, g.sAm == 1 ? 1 : 0);
+                     g.M, g.K, pa, g.sAm == 1 ? 1 : 0, g.sA1);
   hipLaunchKernelGGL(pack_kernel, gb, dim3(256), 0, c->stream, g.B, rB, kB,
-                     g.N, g.K, pb, g.sBn == 1 ? 1 : 0);
+                     g.N, g.K, pb, g.sBn == 1 ? 1 : 0, g.sB1);
   FTCC_CHECK_HIP(hipGetLastError());
   // the packed rows keep the levels of C: row m at m * K
   const int64_t K = g.K;
@@ -710,6 +730,8 @@ bool pack_block(ftcc_ctx *c, Gemm &g) {
   g.sBn = K;
   g.sBn1 = g.N2 > 0 ? (int64_t)g.N2 * K : 0;
   g.sBn0 = g.N2 > 0 ? (int64_t)g.N1 * g.N2 * K : 0;
+  g.sA1 = na > 1 ? (int64_t)g.M * K : 0;
+  g.sB1 = nbb > 1 ? (int64_t)g.N * K : 0;
   g.K1 = 1;
   g.K2 = 0;
   g.sAk = g.sBk = 1;
@@ -719,10 +741,14 @@ bool pack_block(ftcc_ctx *c, Gemm &g) {
 
 // dst_hi/dst_lo[r][k] (row length ld) = the split of src(r, k) for k < K,
 // zero for K <= k < ld (the split-bf16 GEMM reads whole 32-deep slabs)
+// (slice blockIdx.z: src + z * sb, R * ld further on in hi and lo)
 __global__ __launch_bounds__(256) void split_pack_kernel(
     const double *src, PackIdx rl, PackIdx kl, int R, int K, int ld,
-    __bf16 *hi, __bf16 *lo, int along_r) {
+    __bf16 *hi, __bf16 *lo, int along_r, int64_t sb) {
   __shared__ double tile[32][33];
+  src += blockIdx.z * sb;
+  hi += (int64_t)blockIdx.z * R * ld;
+  lo += (int64_t)blockIdx.z * R * ld;
   const int r0 = blockIdx.y * 32, k0 = blockIdx.x * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   auto put = [&](int r, int k, double v) {
@@ -775,19 +801,21 @@ int64_t level_extent(const PackIdx &l, int n) {
 
 // In the low-precision mode of the lambda iteration, a large block runs as a
 // split-bf16 product (lo*hi + hi*lo + hi*hi, FP32 accumulation).  False when
-// the block stays FP64 (the mode is off, the block is small, batched, mapped
-// or has an addend).
+// the block stays FP64 (the mode is off, the block of one grid point is
+// small, mapped or has an addend).
 bool lowp_ok(const ftcc_ctx *c, const Gemm &g) {
   if (c->adj_prec != FTCC_PREC_BF16X3) return false;
   const double flops = 2.0 * g.M * (double)g.N * g.K;
-  return flops >= c->adj_lowp_min_flops && g.nb1 == 1 && g.nb2 == 1 &&
-         !g.mmap && !g.nmap && !g.D && !g.rmap && !g.cmap && g.K >= 1;
+  return flops >= c->adj_lowp_min_flops && g.nb2 == 1 && !g.mmap && !g.nmap && !g.D && !g.rmap && !g.cmap && g.K >= 1;
 }
 
 // doubles of a block's split operands and of its offset tables in the
 // low-precision buffer, each rounded to 256 bytes
 int64_t lowp_split_doubles(const Gemm &g) {
-  const int64_t bf = 2 * ((int64_t)g.M + g.N) * split_ld(g.K);
+  const int64_t bf = 2 *
+                     ((int64_t)g.M * (g.sA1 ? g.nb1 : 1) +
+                      (int64_t)g.N * (g.sB1 ? g.nb1 : 1)) *
+                     split_ld(g.K);
   return ((bf + 3) / 4 + 31) / 32 * 32;
 }
 int64_t lowp_table_doubles(const Gemm &g) {
@@ -828,12 +856,14 @@ bool lowp_group(ftcc_ctx *c, const Gemm *const *gs, int n) {
     const Gemm &g = *gs[k];
     const int64_t ld = split_ld(g.K);
     SplitMat A, B;
+    const int na = g.sA1 ? g.nb1 : 1, nbb = g.sB1 ? g.nb1 : 1;
     A.ld = B.ld = ld;
-    A.bstride = B.bstride = 0;
+    A.bstride = na > 1 ? (int64_t)g.M * ld : 0;
+    B.bstride = nbb > 1 ? (int64_t)g.N * ld : 0;
     A.hi = (__bf16 *)p;
-    A.lo = A.hi + (int64_t)g.M * ld;
-    B.hi = A.lo + (int64_t)g.M * ld;
-    B.lo = B.hi + (int64_t)g.N * ld;
+    A.lo = A.hi + (int64_t)g.M * na * ld;
+    B.hi = A.lo + (int64_t)g.M * na * ld;
+    B.lo = B.hi + (int64_t)g.N * nbb * ld;
     p += lowp_split_doubles(g);
     int *rmap = (int *)p, *cmap = rmap + g.M;
     p += lowp_table_doubles(g);
@@ -841,15 +871,16 @@ bool lowp_group(ftcc_ctx *c, const Gemm *const *gs, int n) {
     const PackIdx kB = pack_levels(g.K1, g.K2, g.sBk0, g.sBk1, g.sBk);
     const PackIdx rA = pack_levels(g.M1, g.M2, g.sAm0, g.sAm1, g.sAm);
     const PackIdx rB = pack_levels(g.N1, g.N2, g.sBn0, g.sBn1, g.sBn);
-    const dim3 ga((unsigned)((ld + 31) / 32), (g.M + 31) / 32),
-        gb((unsigned)((ld + 31) / 32), (g.N + 31) / 32);
-    require(ga.y < 65536 && gb.y < 65536, "split pack: grid too large");
+    const dim3 ga((unsigned)((ld + 31) / 32), (g.M + 31) / 32, na),
+        gb((unsigned)((ld + 31) / 32), (g.N + 31) / 32, nbb);
+    require(ga.y < 65536 && gb.y < 65536 && g.nb1 < 65536,
+            "split pack: grid too large");
     hipLaunchKernelGGL(split_pack_kernel, ga, dim3(256), 0, c->stream, g.A,
                        rA, kA, g.M, g.K, (int)ld, A.hi, A.lo,
-                       g.sAm == 1 ? 1 : 0);
+                       g.sAm == 1 ? 1 : 0, g.sA1);
     hipLaunchKernelGGL(split_pack_kernel, gb, dim3(256), 0, c->stream, g.B,
                        rB, kB, g.N, g.K, (int)ld, B.hi, B.lo,
-                       g.sBn == 1 ? 1 : 0);
+                       g.sBn == 1 ? 1 : 0, g.sB1);
     hipLaunchKernelGGL(level_offsets_kernel, dim3((g.M + 255) / 256),
                        dim3(256), 0, c->stream, c_rows(g), g.M,
                        (int64_t)(g.C - base), rmap);
@@ -864,14 +895,15 @@ bool lowp_group(ftcc_ctx *c, const Gemm *const *gs, int n) {
     prob[k].B = B;
     prob[k].rmap = rmap;
     prob[k].cmap = cmap;
-    flops += 2.0 * g.M * (double)g.N * g.K;
+    flops += 2.0 * g.M * (double)g.N * g.K * g.nb1;
   }
   c->cur_M = g0.M;
   c->cur_N = g0.N;
   c->cur_K = g0.K;
-  c->cur_nb = n;
+  c->cur_nb = n * g0.nb1;
   const int tok = prof_begin(c, ftcc_ctx::PROF_PRODUCTS, flops, 0.0);
-  sbgemm_grouped(n, prob, 1, g0.alpha, g0.beta, base, 1, 1, 0, c->stream);
+  sbgemm_grouped(n, prob, g0.nb1, g0.alpha, g0.beta, base, 1, 1, g0.sC1,
+                 c->stream);
   prof_end(c, tok);
   return true;
 }
@@ -881,9 +913,10 @@ bool lowp_group(ftcc_ctx *c, const Gemm *const *gs, int n) {
 // spin blocks allowed by the three operands' rules are multiplied (a
 // forbidden block of A or B is zero, one of C stays zero); otherwise, or
 // when a block has no layout the engine takes, the whole product runs
-// dense.
+// dense.  The same at nb grid points in each launch: every tensor moves by
+// its own stride between them.
 void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
-         const Ten &C, int line = __builtin_LINE()) {
+         const Ten &C, int nb = 1, int line = __builtin_LINE()) {
   require(beta == 0.0 || beta == 1.0, "contraction: beta must be 0 or 1");
   // per-call-site timing: the GEMMs below belong to the caller's line
   struct Site {
@@ -942,7 +975,7 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
       b.p += off[1];
       cc.p += off[2];
       Block blk;
-      if (!plan(ext, alpha, a, b, 1.0, cc, G, blk.g)) ok = false;
+      if (!plan(ext, alpha, a, b, 1.0, cc, G, nb, blk.g)) ok = false;
       blk.ckey = 0;
       for (int k = 0; k < L; ++k)
         if (C.stride(letters[k]) >= 0 && sp[(unsigned char)letters[k]])
@@ -950,8 +983,10 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
       blocks.push_back(blk);
     }
     if (ok) {
-      if (beta == 0.0) fill(const_cast<double *>(C.p), elems(C, full), 0.0,
-                            c->stream);
+      require(nb == 1 || C.bs == elems(C, full),
+              "contraction: outputs of the grid points are not contiguous");
+      if (beta == 0.0) fill(const_cast<double *>(C.p), elems(C, full) * nb,
+                            0.0, c->stream);
       // split-bf16 blocks go out in groups of up to three with disjoint
       // outputs (a group's launch must not add twice into one element)
       std::vector<const Block *> group;
@@ -984,7 +1019,7 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
     }
   }
   Gemm g;
-  require(plan(full, alpha, A0, B0, beta, C, G, g),
+  require(plan(full, alpha, A0, B0, beta, C, G, nb, g),
           "contraction " + A0.l + "," + B0.l + "->" + C.l +
               ": no layout the GEMM engine takes");
   pack_block(c, g);
@@ -997,20 +1032,27 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
 // Workspace of the adjoint: per-grid-point fixed intermediates (a cache of
 // as many slices as the budget allows), and the buffers of one application.
 // ---------------------------------------------------------------------------
+// (each array holds `n` grid points, one after another)
 struct AdjSlice {
+  int n = 0;
   double *wmnij = nullptr, *wefab = nullptr, *wmbej = nullptr, *zt = nullptr,
-         *zv = nullptr, *f = nullptr;   // f: Fme Fae Fmi Fbe Fmj
+         *zv = nullptr;
+  double *me = nullptr, *ae = nullptr, *mi = nullptr, *be = nullptr,
+         *mj = nullptr;   // the Fock-type intermediates
 };
 
 struct Adjoint {
   const double *T1 = nullptr, *T2 = nullptr;   // the checkpoint
   int ng = 0;
-  std::vector<AdjSlice> cache;   // slices [0, cache.size()) are kept
-  AdjSlice work;                 // intermediates of an uncached slice
-  // application buffers
+  int nb = 1;                    // grid points of one application's launches
+  AdjSlice cache;                // grid points [0, cache.n) are kept
+  AdjSlice work;                 // intermediates of uncached grid points
+  // application buffers of nb grid points
   double *tau = nullptr, *taut = nullptr, *ar = nullptr, *vT = nullptr,
          *acc = nullptr, *gtau = nullptr, *gt = nullptr, *gw = nullptr,
-         *q = nullptr, *u = nullptr, *u2 = nullptr, *small = nullptr;
+         *q = nullptr, *u = nullptr, *u2 = nullptr;
+  double *gFmj = nullptr, *gFbe = nullptr, *gFae = nullptr, *gFmi = nullptr,
+         *gFme = nullptr;
   double *partials = nullptr;
   // lambda update: per-slice scales and weights (4 * ng on the device, the
   // host copy alive until the stream passes the upload), singles energy
@@ -1030,25 +1072,49 @@ double *aalloc(ftcc_ctx *c, Adjoint *A, int64_t n) {
   return p;
 }
 
-int64_t small_elems(const ftcc_ctx *c) {
+void alloc_slice(ftcc_ctx *c, Adjoint *A, AdjSlice &s, int n) {
   const int64_t O = c->no, V = c->nv;
-  return 3 * O * V + 2 * V * V + 2 * O * O;
+  s = AdjSlice();
+  if (n <= 0) return;
+  s.wmnij = aalloc(c, A, n * O * O * O * O);
+  s.wefab = aalloc(c, A, n * V * V * V * V);
+  s.wmbej = aalloc(c, A, n * O * V * V * O);
+  s.zt = aalloc(c, A, n * V * V * V * O);
+  s.zv = aalloc(c, A, n * V * O * O * O);
+  s.me = aalloc(c, A, n * (O * V + 2 * V * V + 2 * O * O));
+  s.ae = s.me + n * O * V;
+  s.mi = s.ae + n * V * V;
+  s.be = s.mi + n * O * O;
+  s.mj = s.be + n * V * V;
+  s.n = n;
 }
-
-void alloc_slice(ftcc_ctx *c, Adjoint *A, AdjSlice &s) {
+// the intermediates from grid point y of the block on
+AdjSlice at_point(const ftcc_ctx *c, const AdjSlice &b, int64_t y) {
   const int64_t O = c->no, V = c->nv;
-  s.wmnij = aalloc(c, A, O * O * O * O);
-  s.wefab = aalloc(c, A, V * V * V * V);
-  s.wmbej = aalloc(c, A, O * V * V * O);
-  s.zt = aalloc(c, A, V * V * V * O);
-  s.zv = aalloc(c, A, V * O * O * O);
-  s.f = aalloc(c, A, small_elems(c));
+  AdjSlice s = b;
+  s.n = b.n - (int)y;
+  s.wmnij += y * O * O * O * O;
+  s.wefab += y * V * V * V * V;
+  s.wmbej += y * O * V * V * O;
+  s.zt += y * V * V * V * O;
+  s.zv += y * V * O * O * O;
+  s.me += y * O * V;
+  s.ae += y * V * V;
+  s.mi += y * O * O;
+  s.be += y * V * V;
+  s.mj += y * O * O;
+  return s;
 }
 
 int64_t slice_bytes(const ftcc_ctx *c) {
   const int64_t O = c->no, V = c->nv;
   return 8 * (O * O * O * O + V * V * V * V + O * V * V * O + V * V * V * O +
-              V * O * O * O + small_elems(c));
+              V * O * O * O + O * V + 2 * V * V + 2 * O * O);
+}
+// application buffers of one grid point
+int64_t buffer_bytes(const ftcc_ctx *c) {
+  const int64_t O = c->no, V = c->nv;
+  return 8 * (9 * V * V * O * O + V * O * O * O + V * V * V * O);
 }
 
 // the adjoint's reduction buffers (allocated on first use)
@@ -1060,214 +1126,203 @@ Adjoint *adjoint_ws(ftcc_ctx *c) {
   return A;
 }
 
-// the buffers of one application of J^T (ftcc_adjoint_begin)
-void ensure_apply_buffers(ftcc_ctx *c, Adjoint *A) {
-  if (A->tau) return;
+// the buffers of one application of J^T to nb grid points
+// (ftcc_adjoint_begin); the intermediates of uncached ones if any
+void alloc_apply_buffers(ftcc_ctx *c, Adjoint *A, int nb, bool uncached) {
   const int64_t O = c->no, V = c->nv, S2 = V * V * O * O;
-  A->tau = aalloc(c, A, S2);
-  A->taut = aalloc(c, A, S2);
-  A->ar = aalloc(c, A, S2);
-  A->vT = aalloc(c, A, S2);
-  A->acc = aalloc(c, A, S2);
-  A->gtau = aalloc(c, A, S2);
-  A->gt = aalloc(c, A, S2);
-  A->gw = aalloc(c, A, O * V * O * V);
-  A->q = aalloc(c, A, V * O * O * V);
-  A->u = aalloc(c, A, O * V * O * O);
-  A->u2 = aalloc(c, A, V * V * V * O);
-  A->small = aalloc(c, A, 5 * small_elems(c));
-  alloc_slice(c, A, A->work);
-}
-
-// Fock-type intermediates inside AdjSlice::f
-struct Fs {
-  double *me, *ae, *mi, *be, *mj;
-};
-Fs fs_of(const ftcc_ctx *c, double *f) {
-  const int64_t O = c->no, V = c->nv;
-  Fs r;
-  r.me = f;
-  r.ae = r.me + O * V;
-  r.mi = r.ae + V * V;
-  r.be = r.mi + O * O;
-  r.mj = r.be + V * V;
-  return r;
+  for (double **p : {&A->tau, &A->taut, &A->ar, &A->vT, &A->acc, &A->gtau,
+                     &A->gt, &A->gw, &A->q})
+    *p = aalloc(c, A, nb * S2);
+  A->u = aalloc(c, A, nb * O * V * O * O);
+  A->u2 = aalloc(c, A, nb * V * V * V * O);
+  A->gFmj = aalloc(c, A, nb * (2 * V * V + 2 * O * O + V * O));
+  A->gFbe = A->gFmj + nb * O * O;
+  A->gFae = A->gFbe + nb * V * V;
+  A->gFmi = A->gFae + nb * V * V;
+  A->gFme = A->gFmi + nb * O * O;
+  alloc_slice(c, A, A->work, uncached ? nb : 0);
+  A->nb = nb;
 }
 
 void copy(ftcc_ctx *c, double *dst, const double *src, int64_t n, double a) {
   axpby(dst, src, n, a, 0.0, c->stream);
 }
 
-// the fixed (amplitude-only) intermediates of one grid point
-void prepare_slice(ftcc_ctx *c, Adjoint *A, const double *t1,
-                   const double *t2, AdjSlice &s) {
+// the fixed (amplitude-only) intermediates of nb grid points
+void prepare_points(ftcc_ctx *c, Adjoint *A, const double *t1,
+                    const double *t2, const AdjSlice &s, int nb) {
   const int O = c->no, V = c->nv;
   const int64_t S2 = (int64_t)V * V * O * O;
   hipStream_t st = c->stream;
-  hipLaunchKernelGGL(tau_kernel, dim3(grid_for(S2)), dim3(AT), 0, st, t1, t2,
-                     V, O, A->tau, A->taut, A->ar);
+  hipLaunchKernelGGL(tau_kernel, dim3(grid_for(S2 * nb)), dim3(AT), 0, st, t1,
+                     t2, V, O, nb, A->tau, A->taut, A->ar);
   FTCC_CHECK_HIP(hipGetLastError());
+  auto cn = [&](double alpha, const Ten &X, const Ten &Y, double beta,
+                const Ten &Z, int line = __builtin_LINE()) {
+    con(c, alpha, X, Y, beta, Z, nb, line);
+  };
   double *const *I = c->I;   // vvvv vvvo vovv vvoo vovo oovv vooo ooov oooo
-  const Fs F = fs_of(c, s.f);
   // Fme = F.ov + t1.oovv
-  copy(c, F.me, c->F[1], (int64_t)O * V, 1.0);
-  con(c, 1.0, ten(c, I[5], "mnef"), ten(c, t1, "fn"), 1.0, ten(c, F.me, "me"));
+  bcast(s.me, c->F[1], (int64_t)O * V, nb, 1.0, 0.0, st);
+  cn(1.0, ten(c, I[5], "mnef"), bten(c, t1, "fn"), 1.0, bten(c, s.me, "me"));
   // Fae = F.vv - 1/2 t1.F.ov - t1.vovv - 1/2 taut.oovv
-  copy(c, F.ae, c->F[3], (int64_t)V * V, 1.0);
-  con(c, -0.5, ten(c, t1, "am"), ten(c, c->F[1], "me"), 1.0,
-      ten(c, F.ae, "ae"));
-  con(c, -1.0, ten(c, I[2], "amfe"), ten(c, t1, "fm"), 1.0,
-      ten(c, F.ae, "ae"));
-  con(c, -0.5, ten(c, A->taut, "afmn"), ten(c, I[5], "mnef"), 1.0,
-      ten(c, F.ae, "ae"));
+  bcast(s.ae, c->F[3], (int64_t)V * V, nb, 1.0, 0.0, st);
+  cn(-0.5, bten(c, t1, "am"), ten(c, c->F[1], "me"), 1.0,
+      bten(c, s.ae, "ae"));
+  cn(-1.0, ten(c, I[2], "amfe"), bten(c, t1, "fm"), 1.0,
+      bten(c, s.ae, "ae"));
+  cn(-0.5, bten(c, A->taut, "afmn"), ten(c, I[5], "mnef"), 1.0,
+      bten(c, s.ae, "ae"));
   // Fmi = F.oo + 1/2 F.ov.t1 + t1.ooov + 1/2 oovv.taut
-  copy(c, F.mi, c->F[0], (int64_t)O * O, 1.0);
-  con(c, 0.5, ten(c, c->F[1], "me"), ten(c, t1, "ei"), 1.0,
-      ten(c, F.mi, "mi"));
-  con(c, 1.0, ten(c, I[7], "mnie"), ten(c, t1, "en"), 1.0,
-      ten(c, F.mi, "mi"));
-  con(c, 0.5, ten(c, I[5], "mnef"), ten(c, A->taut, "efin"), 1.0,
-      ten(c, F.mi, "mi"));
+  bcast(s.mi, c->F[0], (int64_t)O * O, nb, 1.0, 0.0, st);
+  cn(0.5, ten(c, c->F[1], "me"), bten(c, t1, "ei"), 1.0,
+      bten(c, s.mi, "mi"));
+  cn(1.0, ten(c, I[7], "mnie"), bten(c, t1, "en"), 1.0,
+      bten(c, s.mi, "mi"));
+  cn(0.5, ten(c, I[5], "mnef"), bten(c, A->taut, "efin"), 1.0,
+      bten(c, s.mi, "mi"));
   // Fbe = Fae - 1/2 t1.Fme, Fmj = Fmi + 1/2 Fme.t1
-  copy(c, F.be, F.ae, (int64_t)V * V, 1.0);
-  con(c, -0.5, ten(c, t1, "bm"), ten(c, F.me, "me"), 1.0, ten(c, F.be, "be"));
-  copy(c, F.mj, F.mi, (int64_t)O * O, 1.0);
-  con(c, 0.5, ten(c, F.me, "me"), ten(c, t1, "ej"), 1.0, ten(c, F.mj, "mj"));
+  copy(c, s.be, s.ae, nb * (int64_t)V * V, 1.0);
+  cn(-0.5, bten(c, t1, "bm"), bten(c, s.me, "me"), 1.0, bten(c, s.be, "be"));
+  copy(c, s.mj, s.mi, nb * (int64_t)O * O, 1.0);
+  cn(0.5, bten(c, s.me, "me"), bten(c, t1, "ej"), 1.0, bten(c, s.mj, "mj"));
   // Wh_mnij = 1/2 (oooo + P(ij) t1.ooov) + 1/4 oovv.tau
-  copy(c, s.wmnij, I[8], (int64_t)O * O * O * O, 0.5);
-  con(c, 0.5, ten(c, I[7], "mnie"), ten(c, t1, "ej"), 1.0,
-      ten(c, s.wmnij, "mnij"));
-  con(c, -0.5, ten(c, I[7], "mnje"), ten(c, t1, "ei"), 1.0,
-      ten(c, s.wmnij, "mnij"));
-  con(c, 0.25, ten(c, I[5], "mnef"), ten(c, A->tau, "efij"), 1.0,
-      ten(c, s.wmnij, "mnij"));
+  bcast(s.wmnij, I[8], (int64_t)O * O * O * O, nb, 0.5, 0.0, st);
+  cn(0.5, ten(c, I[7], "mnie"), bten(c, t1, "ej"), 1.0,
+      bten(c, s.wmnij, "mnij"));
+  cn(-0.5, ten(c, I[7], "mnje"), bten(c, t1, "ei"), 1.0,
+      bten(c, s.wmnij, "mnij"));
+  cn(0.25, ten(c, I[5], "mnef"), bten(c, A->tau, "efij"), 1.0,
+      bten(c, s.wmnij, "mnij"));
   // Wh_efab = 1/2 (vvvv - P(ab) t1.vovv) + 1/4 tau.oovv, stored [e,f,a,b]
   // vvvv[a,b,e,f] / 2 into [e,f,a,b]
   permute4(I[0], s.wefab, V, V, V, V, (int64_t)V, 1, (int64_t)V * V * V,
-           (int64_t)V * V, 0.5, 0.0, 1, 0, 0, st);
-  con(c, -0.5, ten(c, I[2], "amef"), ten(c, t1, "bm"), 1.0,
-      ten(c, s.wefab, "efab"));
-  con(c, 0.5, ten(c, I[2], "bmef"), ten(c, t1, "am"), 1.0,
-      ten(c, s.wefab, "efab"));
-  con(c, 0.25, ten(c, A->tau, "abmn"), ten(c, I[5], "mnef"), 1.0,
-      ten(c, s.wefab, "efab"));
+           (int64_t)V * V, 0.5, 0.0, nb, 0, (int64_t)V * V * V * V, st);
+  cn(-0.5, ten(c, I[2], "amef"), bten(c, t1, "bm"), 1.0,
+      bten(c, s.wefab, "efab"));
+  cn(0.5, ten(c, I[2], "bmef"), bten(c, t1, "am"), 1.0,
+      bten(c, s.wefab, "efab"));
+  cn(0.25, bten(c, A->tau, "abmn"), ten(c, I[5], "mnef"), 1.0,
+      bten(c, s.wefab, "efab"));
   // Wmbej = <mb||ej> - t1.vovv + t1.ooov - oovv.(t2/2 + t1 t1)
   // <mb||ej> = -vovo[b,m,e,j] into [m,b,e,j]
   permute4(I[4], s.wmbej, V, O, V, O, (int64_t)V * O, (int64_t)V * V * O,
-           (int64_t)O, 1, -1.0, 0.0, 1, 0, 0, st);
-  con(c, -1.0, ten(c, I[2], "bmef"), ten(c, t1, "fj"), 1.0,
-      ten(c, s.wmbej, "mbej"));
-  con(c, 1.0, ten(c, I[7], "mnje"), ten(c, t1, "bn"), 1.0,
-      ten(c, s.wmbej, "mbej"));
-  con(c, -1.0, ten(c, I[5], "mnef"), ten(c, A->ar, "fbjn"), 1.0,
-      ten(c, s.wmbej, "mbej"));
+           (int64_t)O, 1, -1.0, 0.0, nb, 0, S2, st);
+  cn(-1.0, ten(c, I[2], "bmef"), bten(c, t1, "fj"), 1.0,
+      bten(c, s.wmbej, "mbej"));
+  cn(1.0, ten(c, I[7], "mnje"), bten(c, t1, "bn"), 1.0,
+      bten(c, s.wmbej, "mbej"));
+  cn(-1.0, ten(c, I[5], "mnef"), bten(c, A->ar, "fbjn"), 1.0,
+      bten(c, s.wmbej, "mbej"));
   // Zt[e,a,b,i] = tau.ooov, Zv[a,m,i,j] = vovv.tau
-  con(c, 1.0, ten(c, A->tau, "abmn"), ten(c, I[7], "mnie"), 0.0,
-      ten(c, s.zt, "eabi", "ab|ie"));
-  con(c, 1.0, ten(c, I[2], "amef"), ten(c, A->tau, "efij"), 0.0,
-      ten(c, s.zv, "amij"));
+  cn(1.0, bten(c, A->tau, "abmn"), ten(c, I[7], "mnie"), 0.0,
+      bten(c, s.zt, "eabi", "ab|ie"));
+  cn(1.0, ten(c, I[2], "amef"), bten(c, A->tau, "efij"), 0.0,
+      bten(c, s.zv, "amij"));
 }
 
-// (g1, g2) = J^T (v1, v2) at one grid point (v2 antisymmetric); g2 is
+// (g1, g2) = J^T (v1, v2) at nb grid points (v2 antisymmetric); g2 is
 // projected onto antisymmetric tensors
-void apply_slice(ftcc_ctx *c, Adjoint *A, const double *t1, const double *t2,
-                 const AdjSlice &s, const double *v1, const double *v2,
-                 double *g1, double *g2) {
+void apply_points(ftcc_ctx *c, Adjoint *A, const double *t1, const double *t2,
+                  const AdjSlice &s, const double *v1, const double *v2,
+                  double *g1, double *g2, int nb) {
   const int O = c->no, V = c->nv;
   const int64_t S2 = (int64_t)V * V * O * O;
   hipStream_t st = c->stream;
+  auto cn = [&](double alpha, const Ten &X, const Ten &Y, double beta,
+                const Ten &Z, int line = __builtin_LINE()) {
+    con(c, alpha, X, Y, beta, Z, nb, line);
+  };
   double *const *I = c->I;
-  const Fs F = fs_of(c, s.f);
-  const int64_t nsm = small_elems(c);
-  double *gFmj = A->small, *gFbe = gFmj + nsm, *gFae = gFbe + nsm,
-         *gFmi = gFae + nsm, *gFme = gFmi + nsm;
+  double *gFmj = A->gFmj, *gFbe = A->gFbe, *gFae = A->gFae, *gFmi = A->gFmi,
+         *gFme = A->gFme;
   // v2 transposed [i,j,a,b]
   permute4(v2, A->vT, V, V, O, O, (int64_t)V, 1, (int64_t)O * V * V,
-           (int64_t)V * V, 1.0, 0.0, 1, 0, 0, st);
-  fill(g1, (int64_t)V * O, 0.0, st);
-  const Ten V2 = ten(c, v2, "abij"), VT = ten(c, A->vT, "ijab");
+           (int64_t)V * V, 1.0, 0.0, nb, S2, S2, st);
+  fill(g1, nb * (int64_t)V * O, 0.0, st);
+  const Ten V2 = bten(c, v2, "abij"), VT = bten(c, A->vT, "ijab");
   // doubles terms of the residual, transposed (antisymmetrisers give 2, 4)
-  con(c, 2.0, V2, ten(c, I[6], "bmij"), 1.0, ten(c, g1, "am"));      // vooo
-  con(c, 2.0, ten(c, I[1], "abej"), V2, 1.0, ten(c, g1, "ei"));      // vvvo
-  con(c, 4.0, V2, ten(c, s.wmbej, "mbej"), 0.0, ten(c, A->acc, "aeim"));
-  con(c, 4.0, ten(c, t2, "aeim"), V2, 0.0, ten(c, A->gw, "jbme", "mb|ej"));
+  cn(2.0, V2, ten(c, I[6], "bmij"), 1.0, bten(c, g1, "am"));      // vooo
+  cn(2.0, ten(c, I[1], "abej"), V2, 1.0, bten(c, g1, "ei"));      // vvvo
+  cn(4.0, V2, bten(c, s.wmbej, "mbej"), 0.0, bten(c, A->acc, "aeim"));
+  cn(4.0, bten(c, t2, "aeim"), V2, 0.0, bten(c, A->gw, "jbme", "mb|ej"));
   // -t1 t1 <mb||ej> term: <mb||ej> = -vovo[b,m,e,j]
-  con(c, 1.0, ten(c, t1, "am"), V2, 0.0, ten(c, A->u, "mbij"));
-  con(c, 4.0, ten(c, I[4], "bmej"), ten(c, A->u, "mbij"), 1.0,
-      ten(c, g1, "ei"));
-  con(c, 1.0, V2, ten(c, t1, "ei"), 0.0, ten(c, A->u2, "abej"));
-  con(c, 4.0, ten(c, A->u2, "abej"), ten(c, I[4], "bmej"), 1.0,
-      ten(c, g1, "am"));
+  cn(1.0, bten(c, t1, "am"), V2, 0.0, bten(c, A->u, "mbij"));
+  cn(4.0, ten(c, I[4], "bmej"), bten(c, A->u, "mbij"), 1.0,
+      bten(c, g1, "ei"));
+  cn(1.0, V2, bten(c, t1, "ei"), 0.0, bten(c, A->u2, "abej"));
+  cn(4.0, bten(c, A->u2, "abej"), ten(c, I[4], "bmej"), 1.0,
+      bten(c, g1, "am"));
   // ladders (tau adjoint), folded with the W_mnij / W_abef tau terms
-  con(c, 1.0, ten(c, s.wefab, "efab"), VT, 0.0, ten(c, A->gtau, "efij"));
-  con(c, 1.0, V2, ten(c, s.wmnij, "mnij"), 1.0, ten(c, A->gtau, "abmn"));
+  cn(1.0, bten(c, s.wefab, "efab"), VT, 0.0, bten(c, A->gtau, "efij"));
+  cn(1.0, V2, bten(c, s.wmnij, "mnij"), 1.0, bten(c, A->gtau, "abmn"));
   // t1 parts of W_mnij and W_abef through Zt, Zv
-  con(c, 1.0, ten(c, s.zt, "eabi", "ab|ie"), VT, 1.0, ten(c, g1, "ej"));
-  con(c, -1.0, V2, ten(c, s.zv, "amij"), 1.0, ten(c, g1, "bm"));
+  cn(1.0, bten(c, s.zt, "eabi", "ab|ie"), VT, 1.0, bten(c, g1, "ej"));
+  cn(-1.0, V2, bten(c, s.zv, "amij"), 1.0, bten(c, g1, "bm"));
   // Fock-type terms of the doubles
-  con(c, -2.0, V2, ten(c, F.mj, "mj"), 1.0, ten(c, A->acc, "abim"));
-  con(c, -2.0, ten(c, t2, "abim"), V2, 0.0, ten(c, gFmj, "mj"));
-  con(c, 2.0, V2, ten(c, F.be, "be"), 1.0, ten(c, A->acc, "aeij"));
-  con(c, 2.0, ten(c, t2, "aeij"), V2, 0.0, ten(c, gFbe, "be"));
+  cn(-2.0, V2, bten(c, s.mj, "mj"), 1.0, bten(c, A->acc, "abim"));
+  cn(-2.0, bten(c, t2, "abim"), V2, 0.0, bten(c, gFmj, "mj"));
+  cn(2.0, V2, bten(c, s.be, "be"), 1.0, bten(c, A->acc, "aeij"));
+  cn(2.0, bten(c, t2, "aeij"), V2, 0.0, bten(c, gFbe, "be"));
   // Fmj = Fmi + 1/2 t1.Fme ; Fbe = Fae - 1/2 t1.Fme
-  copy(c, gFmi, gFmj, (int64_t)O * O, 1.0);
-  con(c, 0.5, ten(c, gFmj, "mj"), ten(c, F.me, "me"), 1.0, ten(c, g1, "ej"));
-  con(c, 0.5, ten(c, gFmj, "mj"), ten(c, t1, "ej"), 0.0, ten(c, gFme, "me"));
-  copy(c, gFae, gFbe, (int64_t)V * V, 1.0);
-  con(c, -0.5, ten(c, gFbe, "be"), ten(c, F.me, "me"), 1.0,
-      ten(c, g1, "bm"));
-  con(c, -0.5, ten(c, gFbe, "be"), ten(c, t1, "bm"), 1.0,
-      ten(c, gFme, "me"));
+  copy(c, gFmi, gFmj, nb * (int64_t)O * O, 1.0);
+  cn(0.5, bten(c, gFmj, "mj"), bten(c, s.me, "me"), 1.0, bten(c, g1, "ej"));
+  cn(0.5, bten(c, gFmj, "mj"), bten(c, t1, "ej"), 0.0, bten(c, gFme, "me"));
+  copy(c, gFae, gFbe, nb * (int64_t)V * V, 1.0);
+  cn(-0.5, bten(c, gFbe, "be"), bten(c, s.me, "me"), 1.0,
+      bten(c, g1, "bm"));
+  cn(-0.5, bten(c, gFbe, "be"), bten(c, t1, "bm"), 1.0,
+      bten(c, gFme, "me"));
   // singles terms of the residual
-  con(c, 1.0, ten(c, v1, "ai"), ten(c, t1, "ei"), 1.0, ten(c, gFae, "ae"));
-  con(c, 1.0, ten(c, F.ae, "ae"), ten(c, v1, "ai"), 1.0, ten(c, g1, "ei"));
-  con(c, -1.0, ten(c, t1, "am"), ten(c, v1, "ai"), 1.0, ten(c, gFmi, "mi"));
-  con(c, -1.0, ten(c, v1, "ai"), ten(c, F.mi, "mi"), 1.0, ten(c, g1, "am"));
-  con(c, 1.0, ten(c, v1, "ai"), ten(c, F.me, "me"), 1.0,
-      ten(c, A->acc, "aeim"));
-  con(c, 1.0, ten(c, v1, "ai"), ten(c, t2, "aeim"), 1.0,
-      ten(c, gFme, "me"));
-  con(c, -1.0, ten(c, v1, "ai"), ten(c, I[4], "anfi"), 1.0,
-      ten(c, g1, "fn"));
-  con(c, 0.5, ten(c, v1, "ai"), ten(c, I[2], "amef"), 1.0,
-      ten(c, A->acc, "efim"));
-  con(c, 0.5, ten(c, v1, "ai"), ten(c, I[7], "nmie"), 1.0,
-      ten(c, A->acc, "aemn"));
+  cn(1.0, bten(c, v1, "ai"), bten(c, t1, "ei"), 1.0, bten(c, gFae, "ae"));
+  cn(1.0, bten(c, s.ae, "ae"), bten(c, v1, "ai"), 1.0, bten(c, g1, "ei"));
+  cn(-1.0, bten(c, t1, "am"), bten(c, v1, "ai"), 1.0, bten(c, gFmi, "mi"));
+  cn(-1.0, bten(c, v1, "ai"), bten(c, s.mi, "mi"), 1.0, bten(c, g1, "am"));
+  cn(1.0, bten(c, v1, "ai"), bten(c, s.me, "me"), 1.0,
+      bten(c, A->acc, "aeim"));
+  cn(1.0, bten(c, v1, "ai"), bten(c, t2, "aeim"), 1.0,
+      bten(c, gFme, "me"));
+  cn(-1.0, bten(c, v1, "ai"), ten(c, I[4], "anfi"), 1.0,
+      bten(c, g1, "fn"));
+  cn(0.5, bten(c, v1, "ai"), ten(c, I[2], "amef"), 1.0,
+      bten(c, A->acc, "efim"));
+  cn(0.5, bten(c, v1, "ai"), ten(c, I[7], "nmie"), 1.0,
+      bten(c, A->acc, "aemn"));
   // Wmbej: t1.vovv, t1.ooov and the ring amplitude t2/2 + t1 t1
-  con(c, -1.0, ten(c, A->gw, "jbme", "mb|ej"), ten(c, I[2], "bmef"), 1.0,
-      ten(c, g1, "fj"));
-  con(c, 1.0, ten(c, A->gw, "jbme", "mb|ej"), ten(c, I[7], "mnje"), 1.0,
-      ten(c, g1, "bn"));
-  con(c, 1.0, ten(c, A->gw, "jbme", "mb|ej"), ten(c, I[5], "mnef"), 0.0,
-      ten(c, A->q, "bjnf", "bf|jn"));
+  cn(-1.0, bten(c, A->gw, "jbme", "mb|ej"), ten(c, I[2], "bmef"), 1.0,
+      bten(c, g1, "fj"));
+  cn(1.0, bten(c, A->gw, "jbme", "mb|ej"), ten(c, I[7], "mnje"), 1.0,
+      bten(c, g1, "bn"));
+  cn(1.0, bten(c, A->gw, "jbme", "mb|ej"), ten(c, I[5], "mnef"), 0.0,
+      bten(c, A->q, "bjnf", "bf|jn"));
   // acc[f,b,j,n] -= q[b,j,n,f] / 2
   permute4(A->q, A->acc, V, O, O, V, (int64_t)O * O, (int64_t)O, 1,
-           (int64_t)V * O * O, -0.5, 1.0, 1, 0, 0, st);
-  con(c, -1.0, ten(c, A->q, "bjnf", "bf|jn"), ten(c, t1, "bn"), 1.0,
-      ten(c, g1, "fj"));
-  con(c, -1.0, ten(c, A->q, "bjnf", "bf|jn"), ten(c, t1, "fj"), 1.0,
-      ten(c, g1, "bn"));
+           (int64_t)V * O * O, -0.5, 1.0, nb, S2, S2, st);
+  cn(-1.0, bten(c, A->q, "bjnf", "bf|jn"), bten(c, t1, "bn"), 1.0,
+      bten(c, g1, "fj"));
+  cn(-1.0, bten(c, A->q, "bjnf", "bf|jn"), bten(c, t1, "fj"), 1.0,
+      bten(c, g1, "bn"));
   // Fmi, Fae, Fme
-  con(c, 0.5, ten(c, c->F[1], "me"), ten(c, gFmi, "mi"), 1.0,
-      ten(c, g1, "ei"));
-  con(c, 1.0, ten(c, I[7], "mnie"), ten(c, gFmi, "mi"), 1.0,
-      ten(c, g1, "en"));
-  con(c, 0.5, ten(c, gFmi, "mi"), ten(c, I[5], "mnef"), 0.0,
-      ten(c, A->gt, "efin"));
-  con(c, -0.5, ten(c, gFae, "ae"), ten(c, c->F[1], "me"), 1.0,
-      ten(c, g1, "am"));
-  con(c, -1.0, ten(c, gFae, "ae"), ten(c, I[2], "amfe"), 1.0,
-      ten(c, g1, "fm"));
-  con(c, -0.5, ten(c, gFae, "ae"), ten(c, I[5], "mnef"), 1.0,
-      ten(c, A->gt, "afmn"));
-  con(c, 1.0, ten(c, gFme, "me"), ten(c, I[5], "mnef"), 1.0,
-      ten(c, g1, "fn"));
+  cn(0.5, ten(c, c->F[1], "me"), bten(c, gFmi, "mi"), 1.0,
+      bten(c, g1, "ei"));
+  cn(1.0, ten(c, I[7], "mnie"), bten(c, gFmi, "mi"), 1.0,
+      bten(c, g1, "en"));
+  cn(0.5, bten(c, gFmi, "mi"), ten(c, I[5], "mnef"), 0.0,
+      bten(c, A->gt, "efin"));
+  cn(-0.5, bten(c, gFae, "ae"), ten(c, c->F[1], "me"), 1.0,
+      bten(c, g1, "am"));
+  cn(-1.0, bten(c, gFae, "ae"), ten(c, I[2], "amfe"), 1.0,
+      bten(c, g1, "fm"));
+  cn(-0.5, bten(c, gFae, "ae"), ten(c, I[5], "mnef"), 1.0,
+      bten(c, A->gt, "afmn"));
+  cn(1.0, bten(c, gFme, "me"), ten(c, I[5], "mnef"), 1.0,
+      bten(c, g1, "fn"));
   // projection and the tau / taut chain rule into t1
-  hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(S2)), dim3(AT), 0, st,
-                     A->acc, A->gtau, A->gt, V, O, A->tau, g2);
+  hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(S2 * nb)), dim3(AT), 0,
+                     st, A->acc, A->gtau, A->gt, V, O, nb, A->tau, g2);
   FTCC_CHECK_HIP(hipGetLastError());
-  con(c, 4.0, ten(c, A->tau, "abij"), ten(c, t1, "bj"), 1.0,
-      ten(c, g1, "ai"));
+  cn(4.0, bten(c, A->tau, "abij"), bten(c, t1, "bj"), 1.0,
+      bten(c, g1, "ai"));
 }
 
 }  // namespace
@@ -1304,11 +1359,9 @@ void lambda_factors(ftcc_ctx *c, Adjoint *A, const double *T1,
   FTCC_CHECK_HIP(hipMemcpyAsync(A->d_w, A->h_w.data(),
                                 sizeof(double) * 4 * ng,
                                 hipMemcpyHostToDevice, c->stream));
-  for (int y = 0; y < ng; ++y) {
-    copy(c, A->e1 + y * VO, c->fovT, VO, 1.0);
-    con(c, 1.0, ten(c, c->I[5], "ijab"), ten(c, T1 + y * VO, "bj"), 1.0,
-        ten(c, A->e1 + y * VO, "ai"));
-  }
+  bcast(A->e1, c->fovT, VO, ng, 1.0, 0.0, c->stream);
+  con(c, 1.0, ten(c, c->I[5], "ijab"), bten(c, T1, "bj"), 1.0,
+      bten(c, A->e1, "ai"), ng);
 }
 
 void sum4(ftcc_ctx *c, Adjoint *A, int nblocks, double *dst) {
@@ -1379,22 +1432,42 @@ int ftcc_adjoint_begin(ftcc_ctx *c, const double *T1, const double *T2) {
     // the forward residual's operand buffers are rebuilt when next needed
     free_workspace(c);
     adjoint_release(c);
-    Adjoint *A = adjoint_ws(c);
-    ensure_apply_buffers(c, A);
+    double budget_gb = 64.0, work_gb = 120.0;
+    if (const char *env = getenv("FTCC_ADJOINT_CACHE_GB"))
+      budget_gb = atof(env);
+    if (const char *env = getenv("FTCC_WORKSPACE_GB")) work_gb = atof(env);
+    const int keep = (int)std::max<int64_t>(
+        0, std::min<int64_t>(c->ng, (int64_t)(budget_gb * (1LL << 30)) /
+                                        slice_bytes(c)));
+    // grid points per application: as many as a quarter of the budget of
+    // the residual workspace (released above) holds, one at least; they
+    // share their launches (at n = 66 and eight grid points an application
+    // took 3720 launches one point at a time, most of them too small to
+    // fill the device)
+    const int64_t per = buffer_bytes(c) + (keep < c->ng ? slice_bytes(c) : 0);
+    int nb = (int)std::max<int64_t>(
+        1, std::min<int64_t>(c->ng, (int64_t)(work_gb * 0.25 * (1LL << 30)) /
+                                        per));
+    Adjoint *A = nullptr;
+    for (;; nb = (nb + 1) / 2) {
+      A = adjoint_ws(c);
+      try {
+        alloc_apply_buffers(c, A, nb, keep < c->ng);
+        alloc_slice(c, A, A->cache, keep);
+        break;
+      } catch (const Error &e) {
+        if (e.code != FTCC_ENOMEM || nb == 1) throw;
+        adjoint_release(c);   // less memory free than that: fewer at a time
+        (void)hipGetLastError();
+      }
+    }
     A->T1 = T1;
     A->T2 = T2;
     A->ng = c->ng;
-    double budget_gb = 64.0;
-    if (const char *env = getenv("FTCC_ADJOINT_CACHE_GB"))
-      budget_gb = atof(env);
-    const int64_t keep = std::min<int64_t>(
-        c->ng, (int64_t)(budget_gb * (1LL << 30)) / slice_bytes(c));
     const int64_t VO = (int64_t)c->nv * c->no;
-    A->cache.resize((size_t)std::max<int64_t>(0, keep));
-    for (int y = 0; y < (int)A->cache.size(); ++y) {
-      alloc_slice(c, A, A->cache[y]);
-      prepare_slice(c, A, T1 + y * VO, T2 + y * VO * VO, A->cache[y]);
-    }
+    for (int y = 0; y < keep; y += nb)
+      prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
+                     at_point(c, A->cache, y), std::min(nb, keep - y));
     FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
   });
 }
@@ -1402,7 +1475,7 @@ int ftcc_adjoint_begin(ftcc_ctx *c, const double *T1, const double *T2) {
 int ftcc_adjoint_cached(ftcc_ctx *c, int *nslices) {
   return guarded(c, [&] {
     require(nslices != nullptr, "null output pointer");
-    *nslices = c->adj ? (int)c->adj->cache.size() : 0;
+    *nslices = c->adj ? c->adj->cache.n : 0;
   });
 }
 
@@ -1416,15 +1489,15 @@ int ftcc_adjoint_apply(ftcc_ctx *c, const double *Lt1, const double *Lt2,
             FTCC_ESTATE);
     require(Lt1 && Lt2 && G1 && G2, "null pointer");
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
-    for (int y = 0; y < c->ng; ++y) {
+    for (int y = 0; y < c->ng;) {
       const double *t1 = A->T1 + y * VO, *t2 = A->T2 + y * S2;
-      const AdjSlice *s = &A->work;
-      if (y < (int)A->cache.size())
-        s = &A->cache[y];
-      else
-        prepare_slice(c, A, t1, t2, A->work);
-      apply_slice(c, A, t1, t2, *s, Lt1 + y * VO, Lt2 + y * S2, G1 + y * VO,
-                  G2 + y * S2);
+      const bool kept = y < A->cache.n;
+      const int nb = std::min(A->nb, (kept ? A->cache.n : c->ng) - y);
+      const AdjSlice s = kept ? at_point(c, A->cache, y) : A->work;
+      if (!kept) prepare_points(c, A, t1, t2, s, nb);
+      apply_points(c, A, t1, t2, s, Lt1 + y * VO, Lt2 + y * S2, G1 + y * VO,
+                   G2 + y * S2, nb);
+      y += nb;
     }
   });
 }

@@ -694,7 +694,8 @@ int64_t operand_doubles(const ftcc_ctx *c, int prec, int nb) {
       const int64_t elems = rows * split_ld(space_len(c, op_k(c, id))) * slots;
       tot += 2 * carve_len((elems + 3) / 4 + 1);   // four bf16 per double
     } else if (c->spin) {
-      tot += carve_len(rows * space_len(c, op_k(c, id)) * slots);
+      const int64_t elems = rows * space_len(c, op_k(c, id)) * slots;
+      tot += carve_len(prec == FTCC_PREC_FP32 ? (elems + 1) / 2 : elems);
     }
   }
   return tot;
@@ -748,21 +749,26 @@ void ensure_split_buffers(ftcc_ctx *c) {
   c->split_fixed_valid = false;
 }
 
-// FP64 spin-blocked operand buffers (FP64 and FP32 modes), carved from the
-// arena (the split copies there are given up).
+// Spin-blocked operand buffers of the FP64 and FP32 modes (elements of that
+// type), carved from the arena (the other precision's copies there are given
+// up).
 void ensure_b64_buffers(ftcc_ctx *c) {
-  if (c->arena_owner == 2 && c->b64_layout == op_layout(c) &&
+  const bool f32 = c->prec == FTCC_PREC_FP32;
+  const int owner = f32 ? 3 : 2;
+  if (c->arena_owner == owner && c->b64_layout == op_layout(c) &&
       c->b64_nb == c->nb)
     return;
-  double *p = operand_arena(c, operand_doubles(c, FTCC_PREC_FP64, c->nb));
+  double *p = operand_arena(c, operand_doubles(c, c->prec, c->nb));
   for (int id = 0; id < NOPS; ++id) split_of(c, id) = SplitMat();
   c->split_layout = -1;
   for (int id = 0; id < NOPS; ++id) {
     c->b64[id] = p;
-    p += carve_len((int64_t)space_len(c, op_rows(c, id)) *
-                   space_len(c, op_k(c, id)) * (OP_FIXED[id] ? 1 : c->nb));
+    const int64_t elems = (int64_t)space_len(c, op_rows(c, id)) *
+                          space_len(c, op_k(c, id)) *
+                          (OP_FIXED[id] ? 1 : c->nb);
+    p += carve_len(f32 ? (elems + 1) / 2 : elems);
   }
-  c->arena_owner = 2;
+  c->arena_owner = owner;
   c->b64_layout = op_layout(c);
   c->b64_nb = c->nb;
   c->b64_fixed_valid = false;
@@ -806,7 +812,12 @@ void operand_blocks(const ftcc_ctx *c, int id, Range rows[3], Range ks[3]) {
 
 // The spin blocks of operand `id` (operand_blocks) through the pair maps:
 // split(rmap, rows, kmap, K, dst) in bf16x3 mode, f64(rmap, rows, kmap, K,
-// ld, dst, slice stride) otherwise.
+// ld, dst, slice stride) otherwise (dst of FP64 or FP32 elements).
+// (element `off` of operand `id` in the FP64 and FP32 modes)
+void *operand_at(const ftcc_ctx *c, int id, int64_t off) {
+  return c->prec == FTCC_PREC_FP32 ? (void *)((float *)c->b64[id] + off)
+                                   : (void *)(c->b64[id] + off);
+}
 template <typename SplitFn, typename F64Fn>
 void gather_blocks(ftcc_ctx *c, int id, SplitFn split, F64Fn f64,
                    int nb = 1) {
@@ -818,7 +829,7 @@ void gather_blocks(ftcc_ctx *c, int id, SplitFn split, F64Fn f64,
   double elems = 0.0;
   for (int q = 0; q < 3; ++q)
     elems += (double)rows[q].count * ks[q].count * nb;
-  const double per = c->prec == FTCC_PREC_BF16X3 ? 12.0 : 16.0;
+  const double per = c->prec == FTCC_PREC_FP64 ? 16.0 : 12.0;
   timed_class(c, ftcc_ctx::PROF_GATHER, 0.0, per * elems, [&] {
   for (int q = 0; q < 3; ++q) {
     if (rows[q].len == 0 || ks[q].len == 0) continue;
@@ -832,7 +843,7 @@ void gather_blocks(ftcc_ctx *c, int id, SplitFn split, F64Fn f64,
     } else {
       const int64_t ld = K.total;
       f64(rmap, rows[q].len, kmap, ks[q].len, ld,
-          c->b64[id] + (int64_t)rows[q].start * ld + ks[q].start,
+          operand_at(c, id, (int64_t)rows[q].start * ld + ks[q].start),
           (int64_t)R.total * ld);
     }
   }
@@ -850,14 +861,16 @@ void put_operand(ftcc_ctx *c, int id, const double *src, int64_t sr,
                     space_len(c, op_k(c, id)), split_of(c, id), nb, s);
     return;
   }
+  const bool f32 = c->prec == FTCC_PREC_FP32;
   gather_blocks(
       c, id,
       [&](const int *rmap, int R, const int *kmap, int W, const SplitMat &m) {
         split_gather(src, sr, sc, sb, rmap, R, kmap, W, m, nb, s);
       },
       [&](const int *rmap, int R, const int *kmap, int W, int64_t ld,
-          double *dst, int64_t db) {
-        gather64(src, sr, sc, sb, rmap, R, kmap, W, ld, dst, db, nb, s);
+          void *dst, int64_t db) {
+        gather_plain(src, sr, sc, sb, rmap, R, kmap, W, ld, dst, f32, db, nb,
+                     s);
       },
       nb);
 }
@@ -867,16 +880,17 @@ void put_operand(ftcc_ctx *c, int id, const double *src, int64_t sr,
 void put_flip_wr(ftcc_ctx *c, const double *wr, int64_t sb, int nb) {
   const int V = c->nv, O = c->no, hv = c->v_count[0], ho = c->o_count[0];
   hipStream_t s = c->stream;
+  const bool f32 = c->prec == FTCC_PREC_FP32;
   gather_blocks(
       c, OP_WR_B,
       [&](const int *rmap, int R, const int *kmap, int W, const SplitMat &m) {
         flip_ring_gather(wr, V, O, hv, ho, sb, rmap, R, kmap, W, &m, 0,
-                         nullptr, 0, nb, s);
+                         nullptr, false, 0, nb, s);
       },
       [&](const int *rmap, int R, const int *kmap, int W, int64_t ld,
-          double *dst, int64_t db) {
+          void *dst, int64_t db) {
         flip_ring_gather(wr, V, O, hv, ho, sb, rmap, R, kmap, W, nullptr, ld,
-                         dst, db, nb, s);
+                         dst, f32, db, nb, s);
       },
       nb);
 }
@@ -888,15 +902,16 @@ void put_amp_operand(ftcc_ctx *c, int id, int kind, const double *t1,
   require(c->spin, "amplitude gathers need the spin layout");
   hipStream_t s = c->stream;
   const int V = c->nv, O = c->no;
+  const bool f32 = c->prec == FTCC_PREC_FP32;
   gather_blocks(
       c, id,
       [&](const int *rmap, int R, const int *kmap, int W, const SplitMat &m) {
         amp_split_gather(kind, t1, t2, V, O, rmap, R, kmap, W, m, nb, s);
       },
       [&](const int *rmap, int R, const int *kmap, int W, int64_t ld,
-          double *dst, int64_t db) {
-        amp_gather64(kind, t1, t2, V, O, rmap, R, kmap, W, ld, dst, db, nb,
-                     s);
+          void *dst, int64_t db) {
+        amp_gather_plain(kind, t1, t2, V, O, rmap, R, kmap, W, ld, dst, f32,
+                         db, nb, s);
       },
       nb);
 }
@@ -1067,21 +1082,33 @@ void product(ftcc_ctx *c, const Gemm &g, int ia, int ib, int kind) {
       });
     return;
   }
+  PgProblem pb[3];
+  int np = 0;
+  double flops = 0.0;
+  const int64_t ld = K.total;
   for (const Blk &b : blk) {
     if (!b.r.count || !b.c.count || (!b.k.count && g.beta != 0.0)) continue;
-    const double flops = 2.0 * b.r.count * (double)b.c.count * b.k.count * g.nb1;
-    const int64_t ld = K.total;
-    Gemm gb = mk(b.r.len, b.c.len, b.k.len, alpha, g.beta,
-                 c->b64[ia] + (int64_t)b.r.start * ld + b.k.start, ld, 1,
-                 OP_FIXED[ia] ? 0 : (int64_t)R.total * ld,
-                 c->b64[ib] + (int64_t)b.c.start * ld + b.k.start, 1, ld,
-                 OP_FIXED[ib] ? 0 : (int64_t)Cs.total * ld, g.C, g.sCm,
-                 g.sCn, g.sC1, g.nb1);
-    gb.rmap = R.d_map + b.r.start;
-    gb.cmap = Cs.d_map + b.c.start;
-    ensure_partial(c, gb);
-    timed(c, true, flops, [&] { gemm_run(gb, P, c->scr, c->stream); });
+    PgProblem &q = pb[np++];
+    q.M = b.r.len;
+    q.N = b.c.len;
+    q.K = b.k.len;
+    q.A = operand_at(c, ia, (int64_t)b.r.start * ld + b.k.start);
+    q.B = operand_at(c, ib, (int64_t)b.c.start * ld + b.k.start);
+    q.lda = q.ldb = ld;
+    q.sAb = OP_FIXED[ia] ? 0 : (int64_t)R.total * ld;
+    q.sBb = OP_FIXED[ib] ? 0 : (int64_t)Cs.total * ld;
+    q.rmap = R.d_map + b.r.start;
+    q.cmap = Cs.d_map + b.c.start;
+    flops += 2.0 * b.r.count * (double)b.c.count * b.k.count * g.nb1;
   }
+  std::sort(pb, pb + np, [](const PgProblem &x, const PgProblem &y) {
+    return (double)x.M * x.N * x.K > (double)y.M * y.N * y.K;
+  });
+  if (np > 0)
+    timed(c, true, flops, [&] {
+      pgemm_grouped(np, pb, g.nb1, P == FTCC_PREC_FP32, alpha, g.beta, g.C,
+                    g.sCm, g.sCn, g.sC1, c->stream);
+    });
 }
 
 void read_scalars(ftcc_ctx *c, int n);

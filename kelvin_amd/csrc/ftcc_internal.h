@@ -134,19 +134,20 @@ void split_convert(const double *src, int64_t sr, int64_t sc, int64_t sb,
 void split_gather(const double *src, int64_t sr, int64_t sc, int64_t sb,
                   const int *rmap, int R, const int *cmap, int W,
                   const SplitMat &d, int nb, hipStream_t s);
-// the same gather into FP64: dst[b*db + r*os + c], c < W
-void gather64(const double *src, int64_t sr, int64_t sc, int64_t sb,
-              const int *rmap, int R, const int *cmap, int W, int64_t os,
-              double *dst, int64_t db, int nb, hipStream_t s);
+// the same gather unsplit: dst[b*db + r*os + c], c < W, FP64 or rounded to
+// FP32 (f32)
+void gather_plain(const double *src, int64_t sr, int64_t sc, int64_t sb,
+                  const int *rmap, int R, const int *cmap, int W, int64_t os,
+                  void *dst, bool f32, int64_t db, int nb, hipStream_t s);
 // The gather of a ring tensor W[nb][nv][no][nv][no] (slice stride sb) by
 // rows (b,j) and columns (e,m) whose rows of an alpha e only are stored
 // (spin-flip symmetric problem; alpha runs [0, hv) and [0, ho), beta runs
 // after them): a beta e is read from its image.  Into the split pair *d
-// when d is given, else into FP64 dst as gather64.
+// when d is given, else into dst as gather_plain.
 void flip_ring_gather(const double *src, int nv, int no, int hv, int ho,
                       int64_t sb, const int *rmap, int R, const int *cmap,
-                      int W, const SplitMat *d, int64_t os, double *dst,
-                      int64_t db, int nb, hipStream_t s);
+                      int W, const SplitMat *d, int64_t os, void *dst,
+                      bool f32, int64_t db, int nb, hipStream_t s);
 // Amplitude-derived operands gathered straight from t1 [nb][V][O] and
 // t2 [nb][V][V][O][O] (rows / columns are pair indices x * ny + y):
 //   AMP_TAU_AB  rows (a,b), columns (i,j): t2 + t1[a,i]t1[b,j] - t1[b,i]t1[a,j]
@@ -157,9 +158,10 @@ enum AmpKind { AMP_TAU_AB, AMP_TAU_IJ, AMP_T2R, AMP_ARING };
 void amp_split_gather(int kind, const double *t1, const double *t2, int nv,
                       int no, const int *rmap, int R, const int *cmap, int W,
                       const SplitMat &d, int nb, hipStream_t s);
-void amp_gather64(int kind, const double *t1, const double *t2, int nv,
-                  int no, const int *rmap, int R, const int *cmap, int W,
-                  int64_t os, double *dst, int64_t db, int nb, hipStream_t s);
+void amp_gather_plain(int kind, const double *t1, const double *t2, int nv,
+                      int no, const int *rmap, int R, const int *cmap, int W,
+                      int64_t os, void *dst, bool f32, int64_t db, int nb,
+                      hipStream_t s);
 // C[b] = alpha * A[b] . B[b]^T + beta * C[b] with A as [M][K], B as [N][K];
 // output row m goes to row rmap[m] of C and column n to cmap[n] when the
 // maps are given (-1 drops the element)
@@ -177,6 +179,19 @@ struct SbProblem {
 void sbgemm_grouped(int nprob, const SbProblem *prob, int nb, double alpha,
                     double beta, double *C, int64_t sCm, int64_t sCn,
                     int64_t sCb, hipStream_t s);
+
+// The same in FP64, or FP32 (f32), on unsplit K-fast operands: rows of lda
+// (ldb) elements, 16-byte aligned, K padded with zeros to whole slabs of 128
+// bytes (pgemm.hip).
+struct PgProblem {
+  int M, N, K;
+  const void *A, *B;
+  int64_t lda, sAb, ldb, sBb;
+  const int *rmap, *cmap;
+};
+void pgemm_grouped(int nprob, const PgProblem *prob, int nb, bool f32,
+                   double alpha, double beta, double *C, int64_t sCm,
+                   int64_t sCn, int64_t sCb, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // System integrals (ueg.hip)

@@ -259,7 +259,7 @@ __device__ inline void split1(double v, __bf16 &hi, __bf16 &lo) {
 }
 
 // Destination writers of the gather kernels: split into (hi, lo) bf16, or
-// plain FP64 (the spin-blocked operands of the FP64 and FP32 modes).
+// plain FP64 or FP32 (the spin-blocked operands of those modes).
 // store4 writes four consecutive elements (o a multiple of 4).
 struct SplitOut {
   __bf16 *hi, *lo;
@@ -281,6 +281,15 @@ struct SplitOut {
     }
     *(b4_t *)(hi + o) = h;
     *(b4_t *)(lo + o) = l;
+  }
+};
+struct F32Out {
+  float *p;
+  __device__ void operator()(int64_t o, double v) const { p[o] = (float)v; }
+  __device__ void store4(int64_t o, const double v[4]) const {
+    typedef float f4_t __attribute__((ext_vector_type(4)));
+    *(f4_t *)(p + o) =
+        f4_t{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
   }
 };
 struct F64Out {
@@ -546,19 +555,23 @@ void amp_split_gather(int kind, const double *t1, const double *t2, int nv,
              SplitOut{d.hi, d.lo}, nb, s);
 }
 
-void amp_gather64(int kind, const double *t1, const double *t2, int nv,
-                  int no, const int *rmap, int R, const int *cmap, int W,
-                  int64_t os, double *dst, int64_t db, int nb,
-                  hipStream_t s) {
+void amp_gather_plain(int kind, const double *t1, const double *t2, int nv,
+                      int no, const int *rmap, int R, const int *cmap, int W,
+                      int64_t os, void *dst, bool f32, int64_t db, int nb,
+                      hipStream_t s) {
   require(rmap && cmap, "amplitude operands are gathered through pair maps");
-  amp_launch(kind, t1, t2, nv, no, rmap, R, cmap, W, os, db, F64Out{dst}, nb,
-             s);
+  if (f32)
+    amp_launch(kind, t1, t2, nv, no, rmap, R, cmap, W, os, db,
+               F32Out{(float *)dst}, nb, s);
+  else
+    amp_launch(kind, t1, t2, nv, no, rmap, R, cmap, W, os, db,
+               F64Out{(double *)dst}, nb, s);
 }
 
 void flip_ring_gather(const double *src, int nv, int no, int hv, int ho,
                       int64_t sb, const int *rmap, int R, const int *cmap,
-                      int W, const SplitMat *d, int64_t os, double *dst,
-                      int64_t db, int nb, hipStream_t s) {
+                      int W, const SplitMat *d, int64_t os, void *dst,
+                      bool f32, int64_t db, int nb, hipStream_t s) {
   require(2 * hv == nv && 2 * ho == no, "flip gather needs equal spin halves");
   require(rmap && cmap, "flip gather reads through pair maps");
   const FlipRingSrc src_{src, sb, nv, no, hv, ho};
@@ -566,17 +579,26 @@ void flip_ring_gather(const double *src, int nv, int no, int hv, int ho,
     require(d->ld % 32 == 0 && W <= d->ld, "split operand leading dimension");
     gather_launch(src_, true, rmap, R, cmap, W, W, d->ld, d->bstride,
                   SplitOut{d->hi, d->lo}, nb, s);
+  } else if (f32) {
+    gather_launch(src_, true, rmap, R, cmap, W, W, os, db,
+                  F32Out{(float *)dst}, nb, s);
   } else {
-    gather_launch(src_, true, rmap, R, cmap, W, W, os, db, F64Out{dst}, nb, s);
+    gather_launch(src_, true, rmap, R, cmap, W, W, os, db,
+                  F64Out{(double *)dst}, nb, s);
   }
 }
 
-void gather64(const double *src, int64_t sr, int64_t sc, int64_t sb,
-              const int *rmap, int R, const int *cmap, int W, int64_t os,
-              double *dst, int64_t db, int nb, hipStream_t s) {
+void gather_plain(const double *src, int64_t sr, int64_t sc, int64_t sb,
+                  const int *rmap, int R, const int *cmap, int W, int64_t os,
+                  void *dst, bool f32, int64_t db, int nb, hipStream_t s) {
   bool ar;
   const PlainSrc src_ = plain(src, sr, sc, sb, ar);
-  gather_launch(src_, ar, rmap, R, cmap, W, W, os, db, F64Out{dst}, nb, s);
+  if (f32)
+    gather_launch(src_, ar, rmap, R, cmap, W, W, os, db,
+                  F32Out{(float *)dst}, nb, s);
+  else
+    gather_launch(src_, ar, rmap, R, cmap, W, W, os, db,
+                  F64Out{(double *)dst}, nb, s);
 }
 
 void sbgemm_grouped(int nprob, const SbProblem *prob, int nb, double alpha,

@@ -1836,7 +1836,7 @@ void residual_chunk(ftcc_ctx *c, const double *t1, const double *t2,
               [&] {
     r2_final(t2bar, c->wr, c->aring, c->s1, c->s2, c->z, V, O, nb, s,
              c->spin ? c->d_lab_v : nullptr, c->spin ? c->d_lab_o : nullptr,
-             vvoo, c->spin && c->pack, zflip ? hv : 0, zflip ? ho : 0,
+             vvoo, c->spin && c->pack, s5 ? hv : -1, s5 ? ho : -1, zflip,
              !(c->tbar_scratch && c->spin && c->pack), c->d_jl, c->jl_cnt[0],
              c->jl_cnt[1]);
   });

@@ -347,33 +347,33 @@ __global__ __launch_bounds__(256) void r2_final_pair_kernel(
 //   S1          every (a,b), the stored (i,j)   (S1 is antisymmetric in ij)
 //   S2          the stored (a,b), every (i,j)   (S2 is antisymmetric in ab)
 // and add (<ab||ij>) is antisymmetric, so that R2[b,a,i,j] = -R2[a,b,i,j]
-// is written without further reads.  zh > 0 (spin-flip symmetric problem,
-// alpha runs [0, zh) and [0, zo), beta runs after them): Z holds the rows of
-// an alpha first index only, and a row of a beta one is read from its image
-// Z[p - zh][fl(k)][fl(q)][fl(l)].  One workgroup per (a <= b) pair and
-// R2P_ROWS rows i, all j: direct reads and writes run along whole rows of
-// j; the four values read transposed (the stored element of a transposed
-// (i,j), S2[.,.,j,i], the S1 and Z differences at (j,i)) are first staged
-// in LDS as [j][i] strips (row stride R2P_LD doubles: two-way bank
-// conflicts at most on the reads along j).  Four rows per workgroup
-// measured fastest at n = 114 (2, 4, 8, 16 rows: 38.6, 28.5, 33.7, 71.0 ms
-// per iteration).  The row tiles of one (a,b) pair share the cache lines of
-// their staged reads (R2P_ROWS doubles of each line per tile), so the block
-// index is regrouped to run consecutive tiles on one XCD (workgroups are
-// dispatched to the eight XCDs round robin; each XCD has its own L2).
+// is written without further reads.  This form takes any labels: one
+// workgroup per (a <= b) pair and R2P_ROWS rows i, all j; the four values
+// read transposed (the stored element of a transposed (i,j), S2[.,.,j,i],
+// the S1 and Z differences at (j,i)) are first staged in LDS as [j][i]
+// strips.  The block index is regrouped so that the row tiles of one pair,
+// which share the cache lines of their staged reads, run on one XCD.
 constexpr int R2P_ROWS = 4, R2P_LD = 5;
 
-// Logical block of a hardware block id: the ids x, x + 8, x + 16, ... (XCD
-// x) take a contiguous range of logical blocks; a bijection on [0, G).
+// Block index regrouped per XCD: workgroups are dispatched to the eight
+// XCDs round robin and each has its own L2; the hardware ids x, x + 8,
+// x + 16, ... of XCD x take a contiguous range (a bijection on [0, G)).
 __device__ inline int64_t xcd_grouped(int64_t bid, int64_t G) {
   const int64_t q = G / 8, r = G % 8, x = bid % 8, loc = bid / 8;
   return x < r ? x * (q + 1) + loc : r * (q + 1) + (x - r) * q + loc;
 }
+// q -> (a, b), a <= b, q = b (b + 1) / 2 + a
+__device__ inline void triangle(int64_t q, int &a, int &b) {
+  b = (int)((sqrt(8.0 * (double)q + 1.0) - 1.0) * 0.5);
+  while ((int64_t)b * (b + 1) / 2 > q) --b;
+  while ((int64_t)(b + 1) * (b + 2) / 2 <= q) ++b;
+  a = (int)(q - (int64_t)b * (b + 1) / 2);
+}
 __global__ __launch_bounds__(256) void r2_packed_kernel(
     double *t2bar, const double *acc1, const double *acc2, const double *S1,
     const double *S2, const double *Z, const double *add, int nv, int no,
-    const int *lv, const int *lo, int zh, int zo, int zero_forbidden,
-    const int *jl, int jc0, int jc1) {
+    const int *lv, const int *lo, int zero_forbidden, const int *jl, int jc0,
+    int jc1) {
   extern __shared__ double sm[];   // 4 strips of no * R2P_LD
   double *tS2 = sm, *tS1 = sm + no * R2P_LD, *tZ = sm + 2 * no * R2P_LD,
          *tP = sm + 3 * no * R2P_LD;
@@ -382,51 +382,20 @@ __global__ __launch_bounds__(256) void r2_packed_kernel(
   int64_t bid = xcd_grouped(blockIdx.x, gridDim.x);
   const int ti = (int)(bid % tiles);
   bid /= tiles;
-  const int64_t q = bid % npair;
   const int64_t y = bid / npair;
-  int b = (int)((sqrt(8.0 * (double)q + 1.0) - 1.0) * 0.5);
-  while ((int64_t)b * (b + 1) / 2 > q) --b;
-  while ((int64_t)(b + 1) * (b + 2) / 2 <= q) ++b;
-  const int a = (int)(q - (int64_t)b * (b + 1) / 2);
+  int a, b;
+  triangle(bid % npair, a, b);
   const int64_t per = (int64_t)nv * nv * no * no;
   const double *s1 = S1 + y * per, *s2 = S2 + y * per, *z = Z + y * per;
   const double *c1 = acc1 + y * per, *c2 = acc2 + y * per;
   double *out = t2bar + y * per;
   const int i0 = ti * R2P_ROWS;
   const int sab = lv[a] + lv[b];
-  // spin-flip symmetric step (zh > 0, forbidden doubles not written): the
-  // pairs of two beta virtuals are the images of the alpha-alpha pairs,
-  // whose workgroups write them; half of the mixed pairs likewise
-  const bool fimage = zh > 0 && !zero_forbidden;
-  if (fimage && a >= zh) return;   // a <= b: both beta
-  const bool wimage = fimage && b < zh;   // both alpha
-  // a mixed pair (a alpha, b beta) and (b - zh, a + zh) are images of each
-  // other: the one with a < b - zh writes both.  A pair with a == b - zh is
-  // its own image: R2[a,b,i,j] = R2[a,b,fl(j),fl(i)] = -R2[a,b,j,i]
-  // = -R2[a,b,fl(i),fl(j)], so the four elements are written from one of
-  // them, the one with i alpha and the smaller i (computed separately, they
-  // would differ by rounding in the low-precision modes)
-  bool mimage = false, simage = false;
-  if (fimage && b >= zh) {
-    if (a > b - zh) return;
-    mimage = a < b - zh;
-    simage = a == b - zh;
-  }
-  auto flo = [&](int k) { return k < zo ? k + zo : k - zo; };
   auto nat = [&](int p, int r, int k, int l) {
     return (((int64_t)p * nv + r) * no + k) * no + l;
   };
-  auto ring = [&](int p, int k, int r, int l) {
-    return (((int64_t)p * no + k) * nv + r) * no + l;
-  };
   auto zr = [&](int p, int k, int r, int l) {
-    if (zh > 0 && p >= zh) {
-      p -= zh;
-      k = k < zo ? k + zo : k - zo;
-      r = r < zh ? r + zh : r - zh;
-      l = l < zo ? l + zo : l - zo;
-    }
-    return z[ring(p, k, r, l)];
+    return z[(((int64_t)p * no + k) * nv + r) * no + l];
   };
   // the stored (a,b) pair and its sign; a == b is zero throughout
   int pa = a, pb = b;
@@ -486,24 +455,6 @@ __global__ __launch_bounds__(256) void r2_packed_kernel(
     if (add) v += add[nab];
     out[nab] = -v;
     out[nba] = v;
-    if (wimage) {
-      out[nat(a + zh, b + zh, flo(i), flo(j))] = -v;
-      out[nat(b + zh, a + zh, flo(i), flo(j))] = v;
-    }
-    if (mimage) {
-      out[nat(a + zh, b - zh, flo(i), flo(j))] = -v;
-      out[nat(b - zh, a + zh, flo(i), flo(j))] = v;
-    }
-    if (simage) {
-      out[nat(a, b, j, i)] = v;
-      out[nat(b, a, j, i)] = -v;
-      if (i != flo(j)) {
-        out[nat(a, b, flo(j), flo(i))] = -v;
-        out[nat(b, a, flo(j), flo(i))] = v;
-        out[nat(a, b, flo(i), flo(j))] = v;
-        out[nat(b, a, flo(i), flo(j))] = -v;
-      }
-    }
   };
   if (zero_forbidden) {
     const int lanes = blockDim.x / 2;   // two rows at a time
@@ -526,16 +477,181 @@ __global__ __launch_bounds__(256) void r2_packed_kernel(
       const int il = t / cmax, j = allowed_j(il, t % cmax);
       if (j < 0) continue;
       const int i = i0 + il;
-      if (zab) {
-        out[nat(a, b, i, j)] = 0.0;
-        if (wimage) out[nat(a + zh, b + zh, flo(i), flo(j))] = 0.0;
-        continue;
-      }
-      // a self-image pair: written by its element with i alpha and the
-      // smaller i (i beta: from (j, i); fl(j) < i: from (fl(j), fl(i)))
-      if (simage && (lo[i] != 0 || flo(j) < i)) continue;
-      element(il, i, j);
+      if (zab) out[nat(a, b, i, j)] = 0.0;
+      else element(il, i, j);
     }
+  }
+}
+
+// The packed assembly where each label list is one run of alpha then one of
+// beta.  R2 is antisymmetric in (i,j) too, so only the stored (i,j) of the
+// stored (a,b) are computed:
+//   X = acc1 + acc2 + S1[a,b,i,j] - S1[b,a,i,j] + S2[a,b,i,j] - S2[a,b,j,i]
+//       + Z[a,i,b,j] - Z[b,i,a,j] - Z[a,j,b,i] + Z[b,j,a,i] + add,
+// every input read once, and R2 = -X written to the four elements of the
+// couple with their signs.  One workgroup per (a,b) pair and pair of square
+// (i,j) tiles (I, J), I <= J for equal spins: the values at (j,i) are read
+// along i and turned through an LDS tile, the results at (j,i) leave through
+// it, so that every access runs along rows of a tile (the form above reads
+// the transposed values in runs of four).  The run is cut into equal tiles
+// of at most R2T (33 orbitals: two of 17), threads taking the tile's
+// elements in turn whatever its width.
+//   flip (a spin-flip symmetric step; runs of equal length h, Z holds the
+// rows of an alpha first index, the others read from their images): the
+// pairs of two alphas also write their beta images; of the mixed pairs
+// (a, b') (b = b' + h) those with a < b' also write their images (b', a);
+// a == b' is its own image, X[i,j'] = X[j',i] with i and j' counted within
+// their runs, and is computed for i <= j'.
+//   a == b and i == j are zero and written; the spin-forbidden doubles are
+// not touched (r2_zero_kernel).
+// Bound: memory.  24 bytes move per allowed double of a flip step; per
+// eight-point launch at n = 114 5.05 ms with the row strips above.
+constexpr int R2T = 32;
+struct R2Tiles {
+  double *out;
+  const double *acc1, *acc2, *S1, *S2, *Z, *add;
+  int nv, no, hv, ho;          // sizes, alpha runs
+  int flip;
+  // pairs and tile pairs of the three classes (alpha-alpha, mixed,
+  // beta-beta) and the tile edge and count of each occupied run
+  int64_t pairs[3];
+  int tp[3], edge[2], nt[2];
+  int64_t per_y;               // workgroups of one grid point
+};
+__global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
+  __shared__ double tile[R2T][R2T + 1];
+  int64_t bid = xcd_grouped(blockIdx.x, gridDim.x);
+  const int64_t y = bid / p.per_y;
+  bid -= y * p.per_y;
+  int cls = 0;
+  while (bid >= p.pairs[cls] * p.tp[cls]) {
+    bid -= p.pairs[cls] * p.tp[cls];
+    ++cls;
+  }
+  const int64_t q = bid / p.tp[cls];
+  const int t = (int)(bid - q * p.tp[cls]);
+  const int nv = p.nv, no = p.no, hv = p.hv, ho = p.ho;
+  const bool mixed = cls == 1;
+  int a, b, I, J;   // the pair, the tiles
+  if (mixed && !p.flip) {
+    a = (int)(q / (nv - hv));
+    b = hv + (int)(q % (nv - hv));
+  } else {
+    triangle(q, a, b);
+    if (mixed) b += hv;
+    if (cls == 2) a += hv, b += hv;
+  }
+  const int si = cls == 2, sj = cls != 0;   // spins of i and j
+  if (mixed) {
+    I = t / p.nt[1];
+    J = t % p.nt[1];
+  } else {
+    triangle(t, I, J);
+  }
+  const int i0 = (si ? ho : 0) + I * p.edge[si];
+  const int j0 = (sj ? ho : 0) + J * p.edge[sj];
+  const int ni = min(p.edge[si], (si ? no : ho) - i0);
+  const int nj = min(p.edge[sj], (sj ? no : ho) - j0);
+  const int64_t per = (int64_t)nv * nv * no * no, oy = y * per;
+  auto nat = [&](int r, int s, int k, int l) {
+    return oy + (((int64_t)r * nv + s) * no + k) * no + l;
+  };
+  auto fo = [&](int k) { return k < ho ? k + ho : k - ho; };
+  auto fv = [&](int r) { return r < hv ? r + hv : r - hv; };
+  auto zat = [&](int r, int k, int s, int l) {
+    if (p.flip && r >= hv) r = fv(r), k = fo(k), s = fv(s), l = fo(l);
+    return p.Z[oy + (((int64_t)r * no + k) * nv + s) * no + l];
+  };
+  double *out = p.out;
+  // the images of a flip step
+  const bool image = p.flip && (!mixed || a < b - hv);
+  const bool self = p.flip && mixed && a == b - hv;
+  auto put = [&](int k, int l, double v) {   // R2[a,b,k,l] = v
+    out[nat(a, b, k, l)] = v;
+    out[nat(b, a, k, l)] = -v;
+    if (image) {
+      out[nat(fv(a), fv(b), fo(k), fo(l))] = v;
+      out[nat(fv(b), fv(a), fo(k), fo(l))] = -v;
+    }
+  };
+  if (a == b) {
+    for (int e = threadIdx.x; e < ni * nj; e += 256) {
+      const int i = i0 + e / nj, j = j0 + e % nj;
+      out[nat(a, a, i, j)] = 0.0;
+      if (I != J) out[nat(a, a, j, i)] = 0.0;
+      if (image) {
+        out[nat(fv(a), fv(a), fo(i), fo(j))] = 0.0;
+        if (I != J) out[nat(fv(a), fv(a), fo(j), fo(i))] = 0.0;
+      }
+    }
+    return;
+  }
+  // values at (j, i), along i
+  for (int e = threadIdx.x; e < ni * nj; e += 256) {
+    const int r = e / ni, c = e - r * ni;
+    const int j = j0 + r, i = i0 + c;
+    tile[r][c] = zat(b, j, a, i) - zat(a, j, b, i) - p.S2[nat(a, b, j, i)];
+  }
+  __syncthreads();
+  // X at (i, j), along j; the loads of a thread's elements are unconditional
+  // and in flight together (an element that is not used reads valid memory)
+  constexpr int NE = R2T * R2T / 256;
+  double x[NE];
+  bool use[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e0 = threadIdx.x + 256 * k, e = min(e0, ni * nj - 1);
+    const int r = e / nj, c = e - r * nj;
+    const int i = i0 + r, j = j0 + c;
+    // equal spins: i < j; a self-image pair: i <= j within the runs
+    use[k] = e == e0 && (mixed ? !self || i <= j - ho : i < j);
+    const int64_t n = nat(a, b, i, j);
+    const double add = p.add ? p.add[n - oy] : 0.0;
+    x[k] = p.acc1[n] + p.acc2[n] + (p.S1[n] - p.S1[nat(b, a, i, j)]) +
+           p.S2[n] + (zat(a, i, b, j) - zat(b, i, a, j)) + add;
+    x[k] += tile[c][r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = threadIdx.x + 256 * k;
+    if (e >= ni * nj) continue;
+    const int r = e / nj, c = e - r * nj;
+    const int i = i0 + r, j = j0 + c;
+    tile[c][r] = x[k];
+    if (use[k]) {
+      put(i, j, -x[k]);
+      if (self) {   // the image (fl(j), fl(i)) and its transpose
+        put(j - ho, i + ho, -x[k]);
+        put(i + ho, j - ho, x[k]);
+      }
+    } else if (!mixed && i == j) {
+      put(i, i, 0.0);
+    }
+  }
+  __syncthreads();
+  // the elements at (j, i), along i
+  for (int e = threadIdx.x; e < ni * nj; e += 256) {
+    const int r = e / ni, c = e - r * ni;
+    const int j = j0 + r, i = i0 + c;
+    if (mixed ? !self || i <= j - ho : i < j) put(j, i, tile[r][c]);
+  }
+}
+// zeros at the spin-forbidden doubles of nb slices (label runs: alpha below
+// hv, ho): row (a,b,i) allows the j of one spin, or none
+__global__ void r2_zero_kernel(double *out, int nv, int no, int hv, int ho,
+                               int nb) {
+  const int64_t rows = (int64_t)nb * nv * nv * no;
+  const int lane = threadIdx.x & 63;
+  for (int64_t w = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
+       w < rows; w += ((int64_t)gridDim.x * blockDim.x) >> 6) {
+    const int i = (int)(w % no);
+    const int64_t ab = w / no;
+    const int b = (int)(ab % nv), a = (int)(ab / nv % nv);
+    const int sj = (a >= hv) + (b >= hv) - (i >= ho);
+    double *row = out + w * no;
+    for (int j = lane; j < no; j += 64)
+      if ((j >= ho) != sj) row[j] = 0.0;
   }
 }
 
@@ -731,11 +847,11 @@ void ring_assemble(double *Wr, const double *ovvo_ring, const double *Q1,
 void r2_final(double *t2bar, const double *acc1, const double *acc2,
               const double *S1, const double *S2, const double *Z, int nv,
               int no, int nb, hipStream_t s, const int *lab_v,
-              const int *lab_o, const double *add, bool packed, int zh,
-              int zo, bool zero_forbidden, const int *jl, int jc0,
+              const int *lab_o, const double *add, bool packed, int hv,
+              int ho, bool flip, bool zero_forbidden, const int *jl, int jc0,
               int jc1) {
   require(!packed || (lab_v && lab_o), "packed pairs need spin labels");
-  require(zh == 0 || (packed && 2 * zh == nv && 2 * zo == no),
+  require(!flip || (packed && 2 * hv == nv && 2 * ho == no),
           "r2 assembly: flipped Z needs the packed layout and equal halves");
   require(zero_forbidden || packed,
           "r2 assembly: skipping forbidden doubles needs the packed layout");
@@ -745,6 +861,53 @@ void r2_final(double *t2bar, const double *acc1, const double *acc2,
   const int64_t npair = (int64_t)nv * (nv + 1) / 2;
   const int64_t blocks = (int64_t)nb * npair * tiles * tiles;
   require(blocks < (1LL << 31), "r2 assembly grid too large");
+  if (packed && hv >= 0) {
+    // label runs: square tiles of the stored (i,j)
+    R2Tiles t;
+    t.out = t2bar;
+    t.acc1 = acc1;
+    t.acc2 = acc2;
+    t.S1 = S1;
+    t.S2 = S2;
+    t.Z = Z;
+    t.add = add;
+    t.nv = nv;
+    t.no = no;
+    t.hv = hv;
+    t.ho = ho;
+    t.flip = flip ? 1 : 0;
+    const int64_t bv = nv - hv;
+    for (int q = 0; q < 2; ++q) {
+      const int run = q ? no - ho : ho;
+      t.nt[q] = (run + R2T - 1) / R2T;
+      t.edge[q] = t.nt[q] ? (run + t.nt[q] - 1) / t.nt[q] : 0;
+      t.nt[q] = t.edge[q] ? (run + t.edge[q] - 1) / t.edge[q] : 0;
+    }
+    t.pairs[0] = (int64_t)hv * (hv + 1) / 2;
+    t.pairs[1] = flip ? t.pairs[0] : hv * bv;
+    t.pairs[2] = flip ? 0 : bv * (bv + 1) / 2;
+    t.tp[0] = t.nt[0] * (t.nt[0] + 1) / 2;
+    t.tp[1] = t.nt[0] * t.nt[1];
+    t.tp[2] = t.nt[1] * (t.nt[1] + 1) / 2;
+    t.per_y = 0;
+    for (int q = 0; q < 3; ++q) t.per_y += t.pairs[q] * t.tp[q];
+    const int64_t grid = t.per_y * nb;
+    require(grid < (1LL << 31), "r2 assembly grid too large");
+    if (grid > 0) {
+      hipLaunchKernelGGL(r2_tiles_kernel, dim3((unsigned)grid), dim3(256), 0,
+                         s, t);
+      FTCC_CHECK_HIP(hipGetLastError());
+    }
+    if (zero_forbidden) {
+      const int64_t rows = (int64_t)nb * nv * nv * no;
+      hipLaunchKernelGGL(
+          r2_zero_kernel,
+          dim3((unsigned)std::min<int64_t>((rows + 3) / 4, 1 << 16)),
+          dim3(256), 0, s, t2bar, nv, no, hv, ho, nb);
+      FTCC_CHECK_HIP(hipGetLastError());
+    }
+    return;
+  }
   if (packed) {
     const int64_t pblocks =
         (int64_t)nb * npair * ((no + R2P_ROWS - 1) / R2P_ROWS);
@@ -755,8 +918,7 @@ void r2_final(double *t2bar, const double *acc1, const double *acc2,
     set_max_lds_once(attr, (const void *)r2_packed_kernel, 160 * 1024);
     hipLaunchKernelGGL(r2_packed_kernel, dim3((unsigned)pblocks), dim3(256),
                        lds, s, t2bar, acc1, acc2, S1, S2, Z, add, nv, no,
-                       lab_v, lab_o, zh, zo, zero_forbidden ? 1 : 0, jl, jc0,
-                       jc1);
+                       lab_v, lab_o, zero_forbidden ? 1 : 0, jl, jc0, jc1);
   } else
     hipLaunchKernelGGL(r2_final_pair_kernel, dim3((unsigned)blocks),
                        dim3(256), 0, s, t2bar, acc1, acc2, S1, S2, Z, add, nv,

@@ -409,9 +409,9 @@ int ftcc_profile_enable(ftcc_ctx *ctx, int on);
 int ftcc_profile_read(ftcc_ctx *ctx, int64_t *launches, double *ms,
                       double *flops);
 /* Launch plan of the generic GEMMs (the O(n^5) terms, and everything in the
- * FP64/FP32 modes): tile_policy 0 picks the tile (128x128, 128x64, 64x128
- * or 64x64) and the splits of K by their estimated time, 1 keeps 128x128
- * unless a dimension is at most 64, 2 never takes 128x128; K is split at
+ * FP64/FP32 modes): tile_policy 0 takes 64x64 tiles, 1 128x128 unless a
+ * dimension is at most 64, 2 the best of 128x64, 64x128 and 64x64 by their
+ * estimated time; K is split at
  * most until a launch has split_target workgroups (default 1024).
  * Results are the same up to the summation order of split K.  No
  * counterpart in the reference (the tile autotuner of the batch sets it). */

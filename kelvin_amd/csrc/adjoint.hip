@@ -921,16 +921,10 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
   // per-call-site timing: the GEMMs below belong to the caller's line
   struct Site {
     ftcc_ctx *c;
-    int saved, policy;
-    ~Site() {
-      c->site_override = saved;
-      c->tile_policy = policy;
-    }
-  } site{c, c->site_override, c->tile_policy};
+    int saved;
+    ~Site() { c->site_override = saved; }
+  } site{c, c->site_override};
   if (!c->site_override) c->site_override = line;
-  // the adjoint's blocks run on narrow tiles: 41 against 24 TFLOP/s on its
-  // 3249^3 blocks at n = 114 (three workgroups per CU instead of two)
-  c->tile_policy = 2;
   const Groups G = groups_of(A0, B0, C);
   Extents full;
   std::vector<char> letters;
@@ -1002,6 +996,7 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
           }
         group.clear();
       };
+      std::vector<const Block *> rest;
       for (const Block &blk : blocks) {
         if (lowp_ok(c, blk.g)) {
           bool clash = group.size() == 3;
@@ -1011,10 +1006,28 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
           continue;
         }
         Gemm g = blk.g;
-        pack_block(c, g);
-        run(c, g, FTCC_PREC_FP64, false);
+        if (pack_block(c, g)) run(c, g, FTCC_PREC_FP64, false);
+        else rest.push_back(&blk);
       }
       flush();
+      // the others share launches: blocks that add into one output follow
+      // one another, or go out together as partial sums where it is small
+      while (!rest.empty()) {
+        std::vector<Gemm> now;
+        std::vector<int> key;
+        std::vector<const Block *> later;
+        for (const Block *b : rest) {
+          const bool small = (int64_t)b->g.M * b->g.N * nb <= 64 * 1024;
+          if (!small && std::find(key.begin(), key.end(), b->ckey) != key.end())
+            later.push_back(b);
+          else {
+            now.push_back(b->g);
+            key.push_back(b->ckey);
+          }
+        }
+        run_group(c, now.data(), key.data(), (int)now.size(), FTCC_PREC_FP64);
+        rest.swap(later);
+      }
       return;
     }
   }

@@ -26,8 +26,6 @@
 
 #include <algorithm>
 #include <cstring>
-#include <map>
-#include <set>
 #include <vector>
 
 using namespace ftcc;
@@ -143,8 +141,7 @@ Gemm mk(int M, int N, int K, double alpha, double beta, const double *A,
   return g;
 }
 
-void ensure_partial(ftcc_ctx *c, const Gemm &g) {
-  const size_t need = gemm_partial_elems(g);
+void ensure_partial(ftcc_ctx *c, size_t need) {
   if (need > c->scr.partial_elems) {
     // grow: allocation happens outside the kernel stream order, so drain it
     FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
@@ -263,7 +260,7 @@ double gemm_bytes(const Gemm &g) {
   const double sl = (double)g.nb1 * g.nb2;
   const double a = (double)g.M * g.K * ((g.sA1 || g.sA2) ? sl : 1.0);
   const double b = (double)g.K * g.N * ((g.sB1 || g.sB2) ? sl : 1.0);
-  const double cm = (double)g.M * g.N * (g.reduce_b2 ? g.nb1 : sl);
+  const double cm = (double)g.M * g.N * sl;
   return 8.0 * (a + b + cm * (g.beta != 0.0 ? 2.0 : 1.0));
 }
 
@@ -291,26 +288,66 @@ Gemm fold_n(Gemm g) {
   return g;
 }
 
-void run(ftcc_ctx *c, const Gemm &g0, int prec, bool big, int line) {
-  Gemm g = g0;
-  g.tile_policy = c->tile_policy;
-  g.split_target = c->split_target;
-  ensure_partial(c, g);
-  c->cur_line = c->site_override ? c->site_override : line;
-  c->cur_M = g.M;
-  c->cur_N = g.N;
-  c->cur_K = g.K;
-  c->cur_nb = g.nb1 * g.nb2;
-  timed_class(c, big ? ftcc_ctx::PROF_PRODUCTS : ftcc_ctx::PROF_N5,
-              gemm_flops(g), big ? 0.0 : gemm_bytes(g),
-              [&] { gemm_run(g, prec, c->scr, c->stream); });
+void run(ftcc_ctx *c, const Gemm &g, int prec, bool big, int line) {
+  const int blk = 0;
+  run_group(c, &g, &blk, 1, prec, big, line);
+}
+
+// Products of one contraction (gemm_run_group's conventions), any number:
+// launched GEMM_GROUP at a time, products of one output always together.
+void run_group(ftcc_ctx *c, const Gemm *g0, const int *cblk0, int n, int prec,
+               bool big, int line) {
+  std::vector<int> order(n);
+  for (int k = 0; k < n; ++k) order[k] = k;
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int x, int y) { return cblk0[x] < cblk0[y]; });
+  Gemm g[GEMM_GROUP];
+  int cblk[GEMM_GROUP];
+  for (int at = 0; at < n;) {
+    int m = 0;
+    while (at < n) {
+      int e = at + 1;   // the products of the next output
+      while (e < n && cblk0[order[e]] == cblk0[order[at]]) ++e;
+      require(e - at <= GEMM_GROUP, "too many products of one output");
+      if (m + e - at > GEMM_GROUP ||
+          (m > 0 && !gemm_groupable(g[0], g0[order[at]])))
+        break;
+      for (; at < e; ++at, ++m) {
+        g[m] = g0[order[at]];
+        g[m].tile_policy = c->tile_policy;
+        g[m].split_target = c->split_target;
+        cblk[m] = cblk0[order[at]];
+      }
+    }
+    ensure_partial(c, gemm_group_scratch(g, cblk, m));
+    c->cur_line = c->site_override ? c->site_override : line;
+    c->cur_M = g[0].M;
+    c->cur_N = g[0].N;
+    c->cur_K = g[0].K;
+    c->cur_nb = g[0].nb1 * g[0].nb2;
+    double flops = 0.0, bytes = 0.0;
+    for (int k = 0; k < m; ++k) {
+      flops += gemm_flops(g[k]);
+      bytes += big ? 0.0 : gemm_bytes(g[k]);
+    }
+    timed_class(c, big ? ftcc_ctx::PROF_PRODUCTS : ftcc_ctx::PROF_N5, flops,
+                bytes,
+                [&] { gemm_run_group(g, cblk, m, prec, c->scr, c->stream); });
+  }
   c->cur_line = 0;
 }
 
+// the spins of a contraction's letters (-1: not one of them)
+struct Spins {
+  int v[128];
+  Spins() { std::fill(v, v + 128, -1); }
+  int &operator[](char x) { return v[(unsigned char)x]; }
+  int at(char x) const { return v[(unsigned char)x]; }
+};
 
 // Spin conservation rule of an operand, "mn|ie": the spins of the letters
 // left of '|' sum to those right of it ("e|j": a spin-diagonal matrix).
-bool rule_holds(const char *rule, const std::map<char, int> &sp) {
+bool rule_holds(const char *rule, const Spins &sp) {
   int left = 0, right = 0;
   bool r = false;
   for (const char *q = rule; *q; ++q) {
@@ -405,14 +442,10 @@ void run_spin(ftcc_ctx *c, const Gemm &base, int prec,
           "spin-restricted GEMM: skipped pair is not in C");
   require(!qx || (in_c(qx, true) && in_c(qy, true)),
           "spin-restricted GEMM: skipped pair is not in C");
-  auto spin_of = [](const std::map<char, int> &sp, char l) {
-    const auto it = sp.find(l);
-    return it == sp.end() ? -1 : it->second;
-  };
-  auto lead_beta = [&](const std::map<char, int> &sp) {
-    if (lead && spin_of(sp, lead) == 1) return true;
-    if (bx && spin_of(sp, bx) == 1 && spin_of(sp, by) == 0) return true;
-    return qx && spin_of(sp, qx) == 1 && spin_of(sp, qy) == 1;
+  auto lead_beta = [&](const Spins &sp) {
+    if (lead && sp.at(lead) == 1) return true;
+    if (bx && sp.at(bx) == 1 && sp.at(by) == 0) return true;
+    return qx && sp.at(qx) == 1 && sp.at(qy) == 1;
   };
   // a pair index runs over the packed pairs of its spin class (x < y for
   // equal spins, every mixed pair once, none for the beta-alpha class);
@@ -420,14 +453,14 @@ void run_spin(ftcc_ctx *c, const Gemm &base, int prec,
   auto pair_space = [&](const SIdx &x) -> const PairSpace & {
     return x.role == 'P' ? c->ps_oop : c->ps_vvp;
   };
-  auto cls = [&](const SIdx &x, std::map<char, int> &sp) {
+  auto cls = [&](const SIdx &x, Spins &sp) {
     return 2 * sp[x.l] + sp[x.l2];
   };
-  auto start = [&](const SIdx &x, std::map<char, int> &sp) -> int64_t {
+  auto start = [&](const SIdx &x, Spins &sp) -> int64_t {
     if (x.role == 'y' || x.role == '1' || is_pair(x)) return 0;
     return x.role == 'o' ? c->o_start[sp[x.l]] : c->v_start[sp[x.l]];
   };
-  auto count = [&](const SIdx &x, std::map<char, int> &sp) -> int64_t {
+  auto count = [&](const SIdx &x, Spins &sp) -> int64_t {
     if (x.role == 'y') return base.nb1;
     if (x.role == '1') return 1;
     if (is_pair(x)) return pair_space(x).count[cls(x, sp)];
@@ -436,11 +469,14 @@ void run_spin(ftcc_ctx *c, const Gemm &base, int prec,
   // D's stride along an index: none along the slices
   auto sd = [](const SIdx &x) { return x.role == 'y' ? 0 : x.sc; };
   const bool writes_all = base.beta == 0.0 || base.D != nullptr;
-  std::set<std::vector<int>> c_blocks;   // C spin blocks that were written
+  // C spin blocks that were written, by the spins of C's letters
+  std::vector<int> c_blocks(1 << 8, -1);
+  std::vector<Gemm> items;
+  std::vector<int> item_blk;
   const int L = (int)letters.size();
   const SIdx z{0, 'o', 0, 0, 0};
   for (int mask = 0; mask < (1 << L); ++mask) {
-    std::map<char, int> sp;
+    Spins sp;
     for (int k = 0; k < L; ++k) sp[letters[k]] = (mask >> k) & 1;
     if (!rule_holds(ruleA, sp) || !rule_holds(ruleB, sp) ||
         !rule_holds(ruleC, sp) || lead_beta(sp))
@@ -467,22 +503,18 @@ void run_spin(ftcc_ctx *c, const Gemm &base, int prec,
       ck.push_back((int)count(x, sp));
       K *= count(x, sp);
     }
-    std::vector<int> cb;
-    for (const SIdx &x : Mi) {
-      cb.push_back(sp[x.l]);
-      if (is_pair(x)) cb.push_back(sp[x.l2]);
-    }
-    for (const SIdx &x : Ni) {
-      cb.push_back(sp[x.l]);
-      if (is_pair(x)) cb.push_back(sp[x.l2]);
-    }
-    // several K spin blocks onto one C block: the first applies beta and
-    // D, the others accumulate
-    const bool first = c_blocks.insert(cb).second;
-    if (!first) {
-      g.beta = 1.0;
-      g.D = nullptr;
-    }
+    int cb = 1;   // C's spins as bits below a leading one
+    auto bit = [&](const SIdx &x) {
+      cb = 2 * cb + (x.role == 'y' || x.role == '1' ? 0 : sp[x.l]);
+      if (is_pair(x)) cb = 2 * cb + sp[x.l2];
+    };
+    for (const SIdx &x : Mi) bit(x);
+    for (const SIdx &x : Ni) bit(x);
+    require(cb < (1 << 8), "spin-restricted GEMM: too many output indices");
+    // several K spin blocks onto one C block are added up, with the beta and
+    // D of the first
+    const bool first = c_blocks[cb] < 0;
+    c_blocks[cb] = cb;
     if (M == 0 || N == 0) continue;
     require(M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31),
             "spin block too large");
@@ -550,29 +582,32 @@ void run_spin(ftcc_ctx *c, const Gemm &base, int prec,
       g.K1 = 1;
       g.K2 = 0;
     }
-    run(c, g, prec);
+    items.push_back(g);
+    item_blk.push_back(cb);
   }
+  if (!items.empty())
+    run_group(c, items.data(), item_blk.data(), (int)items.size(), prec,
+              false, line);
   if (writes_all) {
     // every spin-allowed, nonempty block of C must have been written
     const int nc = (int)(Mi.size() + Ni.size()) - batch - unit + pm + pn;
     for (int mask = 0; mask < (1 << nc); ++mask) {
-      std::map<char, int> sp;
-      std::vector<int> cb;
-      int k = 0;
+      Spins sp;
+      int k = 0, cb = 1;
       int64_t cells = 1;
       auto take = [&](const SIdx &x) {
         sp[x.l] = (x.role == 'y' || x.role == '1') ? 0 : (mask >> k++) & 1;
-        cb.push_back(sp[x.l]);
+        cb = 2 * cb + sp[x.l];
         if (is_pair(x)) {
           sp[x.l2] = (mask >> k++) & 1;
-          cb.push_back(sp[x.l2]);
+          cb = 2 * cb + sp[x.l2];
         }
         cells *= count(x, sp);
       };
       for (const SIdx &x : Mi) take(x);
       for (const SIdx &x : Ni) take(x);
       if (rule_holds(ruleC, sp) && cells > 0 && !lead_beta(sp))
-        require(c_blocks.count(cb) == 1,
+        require(c_blocks[cb] >= 0,
                 "spin-restricted GEMM leaves an allowed output block unset");
     }
   }

@@ -221,6 +221,10 @@ int guarded(ftcc_ctx *c, Fn fn) {
 // one GEMM of the engine (split-K scratch grown as needed)
 void run(ftcc_ctx *c, const Gemm &g, int prec, bool big = false,
          int line = __builtin_LINE());
+// products of one contraction in as few launches as they fit, with the
+// outputs named by cblk (gemm_run_group)
+void run_group(ftcc_ctx *c, const Gemm *g, const int *cblk, int n, int prec,
+               bool big = false, int line = __builtin_LINE());
 // One index of a spin-restricted contraction: its letter, its orbital role
 // ('o' or 'v'; 'y' the slices of the base, '1' extent one) and its stride
 // in A, B and C (C's strides also address D).

@@ -44,14 +44,10 @@ inline void set_max_lds_once(std::once_flag &flag, const void *kernel,
 //   A(m,k) at A + b1*sA1 + b2*sA2 + m*sAm + k*sAk   (b1 < nb1, b2 < nb2)
 //   B(k,n) at B + b1*sB1 + b2*sB2 + k*sBk + n*sBn
 //   C(m,n) at C + b1*sC1 + b2*sC2 + m*sCm + n*sCn
-// If reduce_b2 is set, the nb2 products are summed into one C per b1
-// (sC2 is ignored): used for contractions whose K index is split over a
-// stride break.
 // ---------------------------------------------------------------------------
 struct Gemm {
   int M = 0, N = 0, K = 0;
   int nb1 = 1, nb2 = 1;
-  bool reduce_b2 = false;
   double alpha = 1.0, beta = 0.0;
   const double *A = nullptr;
   int64_t sAm = 0, sAk = 0, sA1 = 0, sA2 = 0;
@@ -84,8 +80,8 @@ struct Gemm {
   const int *mmap = nullptr, *nmap = nullptr;
   int mlvl = -1, nlvl = -1;
   int64_t sAk0 = 0, sAk1 = 0, sBk0 = 0, sBk1 = 0;
-  // launch plan: tile shape policy (0 by the estimated time; 1 wide: 128x128
-  // unless one dimension is at most 64; 2 narrow: never 128x128) and the
+  // launch plan: tile shape policy (0: 64x64; 1 wide: 128x128 unless one
+  // dimension is at most 64; 2: 128x64 or 64x128, or 64x64) and the
   // workgroup count up to which K may be split
   int tile_policy = 0;
   int split_target = 1024;
@@ -101,8 +97,16 @@ struct Scratch {
   size_t lowp_bytes = 0;
 };
 
-void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s);
-size_t gemm_partial_elems(const Gemm &g);
+// Up to GEMM_GROUP products in one launch, n >= 1, of equal operand layouts
+// (gemm_groupable) and batch.  cblk names each product's output: products of
+// equal cblk are added up in the order given (equal M, N and C; alpha, beta
+// and D of the first apply), the outputs of different cblk are disjoint.
+constexpr int GEMM_GROUP = 8;
+bool gemm_groupable(const Gemm &x, const Gemm &y);
+// doubles of Scratch::partial that gemm_run_group needs
+size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n);
+void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
+                    Scratch &scr, hipStream_t s);
 
 // Split-BF16 operand: x = hi + lo, two bf16 arrays [rows][ld] (K contiguous,
 // zero-padded to ld), batch stride in elements.

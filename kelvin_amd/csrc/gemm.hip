@@ -4,10 +4,9 @@
 // wave owns a quadrant as 16x16 MFMA blocks.  K advances in slabs of 16 staged
 // through LDS (the largest tile double buffered, one barrier per slab) with
 // the next slab prefetched into registers while the current one feeds the
-// MFMAs.  The tile and the splits of K are the pair of least estimated time
-// (plan_of).  Measured, FP64, K contiguous in both operands: 4096^3 52 to 55
-// TFLOP/s with every tile; 15 of 722^3 42 with 64x64, 30 with 128x128; one
-// 361x722x722 in 59 us with 64x64, 30 us with its K split as well.
+// MFMAs.  Tile and splits of K: plan_of.  A launch takes up to GEMM_GROUP
+// products (the spin blocks of a contraction), and products that add into
+// one output leave partial sums for one reduction.
 //
 // LDS holds both operands "K-inner": As[m][k], Bs[n][k], rows padded so the
 // 16 lanes that share a k-group hit distinct banks.  Inside a slab the
@@ -31,6 +30,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 namespace ftcc {
 namespace {
@@ -49,7 +49,6 @@ struct Tile {
 struct GemmDev {
   int M, N, K, nb1, nb2, splits, kchunk, tilesM, tilesN;
   int m_inner;               // tile rows vary fastest (fewer of them)
-  int reduce_b2;
   double alpha, beta;
   const double *A;
   int64_t sAm, sAk, sA1, sA2;
@@ -57,8 +56,10 @@ struct GemmDev {
   int64_t sBk, sBn, sB1, sB2;
   double *C;
   int64_t sCm, sCn, sC1, sC2;
-  double *partial;   // [R][nbC][M][N] when splits*R > 1
-  int nbC;           // number of distinct C batches (nb1 or nb1*nb2)
+  // [R][nb1 * nb2][M][N] when R partial sums make up C, this product's
+  // splits being rbase, rbase + 1, ... (nullptr: C is written directly)
+  double *partial;
+  int rbase, R;
   const int *rmap, *cmap;   // output scatter (nullptr: identity)
   const double *D;          // addend gamma*D laid out like C (or nullptr)
   double gamma;
@@ -74,6 +75,15 @@ struct GemmDev {
   // -1: none): that level's index x becomes map[x] before the strides
   const int *mmap, *nmap;
   int mlvl, nlvl;
+};
+
+// Up to GEMM_GROUP products in one launch: the spin blocks of a contraction,
+// each a product of a few tiles.  Launched one by one, the sixty of a step
+// at n = 38 took 10 to 25 us each whatever their size.
+struct GemmGroup {
+  int n;
+  int tile0[GEMM_GROUP];     // first workgroup of each product
+  GemmDev pr[GEMM_GROUP];
 };
 
 struct Lvl {
@@ -118,38 +128,40 @@ template <> struct Mma<float> {
   }
 };
 
-// Decode the flat block index into (tile n, tile m, split, b2, b1), the
-// tiles along the dimension with fewer of them innermost: those tiles share
-// one panel of the operand with more panels, which is then read from HBM
-// once instead of once per tile row (an O(n^5) term of 456 x 185193 x 57
-// read 1.72 GB with columns innermost against 0.84 GB of distinct data).
-// The index is first regrouped per XCD: workgroups are dispatched to the
+// The flat block index regrouped per XCD: workgroups are dispatched to the
 // eight XCDs round robin and each XCD has its own L2; the hardware ids x,
 // x + 8, x + 16, ... of XCD x take a contiguous range of tiles (a bijection
 // on [0, gridDim.x)).
+__device__ inline int64_t xcd_block() {
+  const int64_t G = gridDim.x, hw = blockIdx.x;
+  const int64_t q8 = G / 8, r8 = G % 8, x = hw % 8, loc = hw / 8;
+  return x < r8 ? x * (q8 + 1) + loc : r8 * (q8 + 1) + (x - r8) * q8 + loc;
+}
+// Decode a product's block into (tile n, tile m, split, b2, b1), the tiles
+// along the dimension with fewer of them innermost: those tiles share one
+// panel of the operand with more panels, which is then read from HBM once
+// instead of once per tile row (an O(n^5) term of 456 x 185193 x 57 read
+// 1.72 GB with columns innermost against 0.84 GB of distinct data).
 struct BlockPos {
   int tn, tm, ks, b1, b2;
 };
-__device__ inline BlockPos decode(const GemmDev &p) {
-  const int64_t G = gridDim.x, hw = blockIdx.x;
-  const int64_t q8 = G / 8, r8 = G % 8, x = hw % 8, loc = hw / 8;
-  int64_t bid = x < r8 ? x * (q8 + 1) + loc : r8 * (q8 + 1) + (x - r8) * q8 + loc;
+__device__ inline BlockPos decode(const GemmDev &p, int bid) {
   BlockPos q;
   if (p.m_inner) {
-    q.tm = (int)(bid % p.tilesM);
+    q.tm = bid % p.tilesM;
     bid /= p.tilesM;
-    q.tn = (int)(bid % p.tilesN);
+    q.tn = bid % p.tilesN;
     bid /= p.tilesN;
   } else {
-    q.tn = (int)(bid % p.tilesN);
+    q.tn = bid % p.tilesN;
     bid /= p.tilesN;
-    q.tm = (int)(bid % p.tilesM);
+    q.tm = bid % p.tilesM;
     bid /= p.tilesM;
   }
-  q.ks = (int)(bid % p.splits);
+  q.ks = bid % p.splits;
   bid /= p.splits;
-  q.b2 = (int)(bid % p.nb2);
-  q.b1 = (int)(bid / p.nb2);
+  q.b2 = bid % p.nb2;
+  q.b1 = bid / p.nb2;
   return q;
 }
 
@@ -254,7 +266,7 @@ __device__ inline void load4(const T *src, T out[4]) {
 // TM x TN output tile per workgroup (128x128 down to 64x64): the four
 // waves form a 2x2 grid, each owning (TM/2) x (TN/2) as RT x CT MFMA blocks.
 template <typename T, bool A_MFAST, bool B_NFAST, int TM, int TN, bool KL>
-__global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmDev p) {
+__global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmGroup grp) {
   using acc_t = typename Mma<T>::acc_t;
   constexpr int LDK = Mma<T>::LDK;
   constexpr int RT = TM / 32, CT = TN / 32;
@@ -268,7 +280,12 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmDev p) {
   __shared__ T Bs[NBUF][TN * LDK];
   __shared__ int64_t aoff[TM], boff[TN], drow[TM], dcol[TN];
 
-  const BlockPos q = decode(p);
+  const int64_t bid = xcd_block();
+  int item = 0;
+  for (int k = 1; k < grp.n; ++k)
+    if (bid >= grp.tile0[k]) item = k;
+  const GemmDev &p = grp.pr[item];
+  const BlockPos q = decode(p, (int)(bid - grp.tile0[item]));
   const double *A = p.A + q.b1 * p.sA1 + q.b2 * p.sA2;
   const double *B = p.B + q.b1 * p.sB1 + q.b2 * p.sB2;
   const int m0 = q.tm * TM, n0 = q.tn * TN;
@@ -354,10 +371,9 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmDev p) {
     }
     __syncthreads();
   }
-  const int cb = p.reduce_b2 ? q.b1 : q.b1 * p.nb2 + q.b2;
-  const int rsel = p.reduce_b2 ? q.b2 * p.splits + q.ks : q.ks;
   double *P = direct ? nullptr
-                     : p.partial + ((int64_t)rsel * p.nbC + cb) *
+                     : p.partial + ((int64_t)(p.rbase + q.ks) * p.nb1 * p.nb2 +
+                                    q.b1 * p.nb2 + q.b2) *
                                        (int64_t)p.M * p.N;
   // Direct stores go one 16-row block at a time: all its reads of D and C
   // are issued before any store (a store may alias them as far as the
@@ -432,8 +448,7 @@ __device__ inline void put_sum(const GemmDev &p, int64_t cb, int64_t mn,
   const int m0 = (int)(mn / p.N), n0 = (int)(mn % p.N);
   const int m = p.rmap ? p.rmap[m0] : m0, n = p.cmap ? p.cmap[n0] : n0;
   if (m < 0 || n < 0) return;
-  const int64_t b1 = p.reduce_b2 ? cb : cb / p.nb2;
-  const int64_t b2 = p.reduce_b2 ? 0 : cb % p.nb2;
+  const int64_t b1 = cb / p.nb2, b2 = cb % p.nb2;
   const Lvl lr = map_level(levels(m, p.M1, p.M2), p.mmap, p.mlvl),
             lc = map_level(levels(n, p.N1, p.N2), p.nmap, p.nlvl);
   double *c = p.C + b1 * p.sC1 + b2 * p.sC2 +
@@ -447,45 +462,44 @@ __device__ inline void put_sum(const GemmDev &p, int64_t cb, int64_t mn,
   *c = y;
 }
 
-// C[b][m,n] = alpha * sum_r partial[r][b][m][n] + beta*C  (fixed order).
+// C[b][m,n] = alpha * sum_r partial[r][b][m][n] + beta*C  (fixed order), for
+// the outputs of a group (tile0: the first workgroup of each).
 // A block of RG x 64 threads takes 64 consecutive elements (coalesced rows
 // of the partial buffer); its RG groups sum interleaved partials (several
 // loads in flight per thread) and combine in LDS, so that even a small
 // output (a few thousand elements) spreads its R-deep sums over the chip.
 constexpr int RG = 16;
-__global__ __launch_bounds__(64 * RG) void reduce_partial_kernel(GemmDev p,
-                                                                 int R) {
+__global__ __launch_bounds__(64 * RG) void reduce_partial_kernel(
+    GemmGroup grp) {
   __shared__ double part[RG][64];
+  int item = 0;
+  for (int k = 1; k < grp.n; ++k)
+    if ((int)blockIdx.x >= grp.tile0[k]) item = k;
+  const GemmDev &p = grp.pr[item];
   const int64_t MN = (int64_t)p.M * p.N;
-  const int64_t total = MN * p.nbC;
-  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
-  for (int64_t base = (int64_t)blockIdx.x * 64; base < total;
-       base += (int64_t)gridDim.x * 64) {
-    const int64_t idx = base + lane;
-    const int64_t cb = idx / MN;
-    const int64_t mn = idx % MN;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    if (idx < total) {
-      const double *src = p.partial + cb * MN + mn;
-      const int64_t step = (int64_t)p.nbC * MN;
-      int r = g;
-      for (; r + 3 * RG < R; r += 4 * RG) {
-        s0 += src[(int64_t)r * step];
-        s1 += src[(int64_t)(r + RG) * step];
-        s2 += src[(int64_t)(r + 2 * RG) * step];
-        s3 += src[(int64_t)(r + 3 * RG) * step];
-      }
-      for (; r < R; r += RG) s0 += src[(int64_t)r * step];
+  const int64_t total = MN * p.nb1 * p.nb2;
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, R = p.R;
+  const int64_t idx =
+      (int64_t)((int)blockIdx.x - grp.tile0[item]) * 64 + lane;
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  if (idx < total) {
+    const double *src = p.partial + idx;
+    int r = g;
+    for (; r + 3 * RG < R; r += 4 * RG) {
+      s0 += src[(int64_t)r * total];
+      s1 += src[(int64_t)(r + RG) * total];
+      s2 += src[(int64_t)(r + 2 * RG) * total];
+      s3 += src[(int64_t)(r + 3 * RG) * total];
     }
-    part[g][lane] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    if (g == 0 && idx < total) {
-      double s = 0.0;
+    for (; r < R; r += RG) s0 += src[(int64_t)r * total];
+  }
+  part[g][lane] = (s0 + s1) + (s2 + s3);
+  __syncthreads();
+  if (g == 0 && idx < total) {
+    double s = 0.0;
 #pragma unroll
-      for (int q = 0; q < RG; ++q) s += part[q][lane];
-      put_sum(p, cb, mn, s);
-    }
-    __syncthreads();
+    for (int q = 0; q < RG; ++q) s += part[q][lane];
+    put_sum(p, idx / MN, idx % MN, s);
   }
 }
 
@@ -493,78 +507,105 @@ __global__ __launch_bounds__(64 * RG) void reduce_partial_kernel(GemmDev p,
 // order with all its loads in flight (the form above leaves RG - R of its
 // RG groups idle).
 constexpr int FEW = 12;
-__global__ __launch_bounds__(256) void reduce_few_kernel(GemmDev p, int R) {
+__global__ __launch_bounds__(256) void reduce_few_kernel(GemmGroup grp) {
+  int item = 0;
+  for (int k = 1; k < grp.n; ++k)
+    if ((int)blockIdx.x >= grp.tile0[k]) item = k;
+  const GemmDev &p = grp.pr[item];
   const int64_t MN = (int64_t)p.M * p.N;
-  const int64_t total = MN * p.nbC;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * 256) {
-    double v[FEW];
+  const int64_t total = MN * p.nb1 * p.nb2;
+  const int R = p.R;
+  const int64_t idx =
+      (int64_t)((int)blockIdx.x - grp.tile0[item]) * 256 + threadIdx.x;
+  if (idx >= total) return;
+  double v[FEW];
 #pragma unroll
-    for (int r = 0; r < FEW; ++r)
-      v[r] = p.partial[(int64_t)(r < R ? r : 0) * total + idx];
-    double s = v[0];
+  for (int r = 0; r < FEW; ++r)
+    v[r] = p.partial[(int64_t)(r < R ? r : 0) * total + idx];
+  double s = v[0];
 #pragma unroll
-    for (int r = 1; r < FEW; ++r) s += r < R ? v[r] : 0.0;
-    put_sum(p, idx / MN, idx % MN, s);
-  }
+  for (int r = 1; r < FEW; ++r) s += r < R ? v[r] : 0.0;
+  put_sum(p, idx / MN, idx % MN, s);
 }
 
-// Tile shape and K splits of a product: the pair with the least estimated
-// time.  Per CU a workgroup's slab takes the time of its MFMAs, and a CU
-// works through its workgroups of a launch at that rate or at that of the
-// load latency of its resident ones, whichever is longer; splitting K adds
-// the partial sums' write and read.  (Splitting every launch of fewer than
-// 1024 workgroups, as this rule did before, spent half of an FP64 step at
-// n = 54 in the sums of partials: 7.4 of 14.4 ms.)
+// Tile shape and K splits of a group: 64x64 tiles (policy 0), and the K per
+// split with the least estimated time.  64x64 was the fastest tile at every
+// size measured but one 4096^3 (TFLOP/s FP64, 64x64 | 128x64 | 128x128: 11
+// of 1458^3 51 | 48 | 42; 3249^3 48 | 44 | 43; 15 of 722^3 42 | 36 | 30;
+// 4096^3 54 | 53 | 55), and for the short-K terms, whose groups it shortens
+// by 4% of a step at n = 66; the wider ones are left to the autotuner.  Per CU a workgroup's slab takes the time of its
+// MFMAs, and a CU works through its workgroups of a launch at that rate or
+// at that of the load latency of its resident ones, whichever is longer;
+// partial sums (splits of K, and products of one output) add their write
+// and read.  (Splitting every launch of fewer than 1024 workgroups, as this
+// rule did before, spent half of an FP64 step at n = 54 in the sums of
+// partials: 7.4 of 14.4 ms.)
 struct Plan {
   Tile t;
-  int splits;
+  int kc;   // K of a split, whole slabs
 };
-double estimate_us(const Gemm &g, Tile t, int splits) {
-  const double tiles = (double)((g.M + t.m - 1) / t.m) *
-                       ((g.N + t.n - 1) / t.n) * g.nb1 * g.nb2;
+int64_t tiles_of(const Gemm &g, Tile t) {
+  return (int64_t)((g.M + t.m - 1) / t.m) * ((g.N + t.n - 1) / t.n) * g.nb1 *
+         g.nb2;
+}
+int splits_of(const Gemm &g, int kc) {
+  return g.K <= kc ? 1 : (g.K + kc - 1) / kc;
+}
+double estimate_us(const Gemm *g, const int *cblk, int n, Tile t, int kc) {
   const int occ = t.m * t.n >= 128 * 128 ? 2 : (t.m * t.n >= 8192 ? 3 : 4);
-  const double slabs = std::ceil(std::ceil(g.K / (double)BK) / splits);
   // one slab of the tile on a CU's four matrix cores, us, and the time
   // from a slab's loads to its use
   const double ts = 1.9 * t.m * t.n / (128.0 * 128.0), lat = 1.2;
-  const double b = tiles * splits;
+  double b = 0.0, sum = 0.0;
+  for (int k = 0; k < n; ++k) {
+    const int sp = splits_of(g[k], kc);
+    // the last split of a product is shorter than the others
+    b += tiles_of(g[k], t) * (double)std::min(kc, std::max(g[k].K, BK)) / kc *
+         sp;
+    bool shared = false;
+    for (int q = 0; q < n; ++q) shared |= q != k && cblk[q] == cblk[k];
+    if (sp > 1 || shared)
+      sum += (double)g[k].M * g[k].N * g[k].nb1 * g[k].nb2 * 8e-6 *   // MB
+             (sp * 2.0 + 1.0) / 3.0;
+  }
   const double us =
-      (slabs + 2.0) * std::max(std::ceil(b / 256.0) * ts,
-                               std::ceil(b / (256.0 * occ)) * lat);
-  const double R = splits * (g.reduce_b2 ? (double)g.nb2 : 1.0);
-  const double out = (double)g.M * g.N * g.nb1 * g.nb2 * 8e-6;   // MB
-  const double sum = R > 1.0 ? 4.0 + out * (splits * 2.0 + 1.0) / 3.0 : 0.0;
-  return us + sum;
+      (kc / BK + 2.0) * std::max(std::ceil(b / 256.0) * ts,
+                                 std::ceil(b / (256.0 * occ)) * lat);
+  return us + (sum > 0.0 ? 4.0 + sum : 0.0);
 }
-Plan plan_of(const Gemm &g) {
-  const int pol = g.tile_policy;
+Plan plan_of(const Gemm *g, const int *cblk, int n) {
+  const int pol = g[0].tile_policy;
   const Tile cand[4] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
-  Plan best{{128, 128}, 1};
+  int M = 0, N = 0, K = 0;
+  for (int k = 0; k < n; ++k) {
+    M = std::max(M, g[k].M);
+    N = std::max(N, g[k].N);
+    K = std::max(K, g[k].K);
+  }
+  const int whole = std::max(1, (K + BK - 1) / BK) * BK;
+  Plan best{{64, 64}, whole};
   double us = 1e300;
-  for (int q = 0; q < 4; ++q) {
-    const Tile t = cand[q];
-    // a side of at most 64 takes no 128-wide tile
-    if ((g.M <= 64 && t.m > 64) || (g.N <= 64 && t.n > 64)) continue;
-    if (pol == 1 && ((g.M > 64 && t.m < 128) || (g.N > 64 && t.n < 128)))
-      continue;
+  for (const Tile &t : cand) {
+    // the wide policies take no 128-wide tile for a side of at most 64
+    if ((M <= 64 && t.m > 64) || (N <= 64 && t.n > 64)) continue;
+    const bool full = t.m >= std::min(128, (M + 63) / 64 * 64) &&
+                      t.n >= std::min(128, (N + 63) / 64 * 64);
+    if (pol == 0 && t.m * t.n > 64 * 64) continue;
+    if (pol == 1 && !full) continue;
     if (pol == 2 && t.m * t.n == 128 * 128) continue;
-    // short K (the O(n^5) contractions over one index): the single-buffered
-    // tiles (three or more workgroups per CU) stream the output faster than
-    // 128x128 (3.5% on those launches at n = 114)
-    if (pol == 0 && g.K <= 64 && t.m * t.n == 128 * 128) continue;
-    const int64_t blocks = (int64_t)((g.M + t.m - 1) / t.m) *
-                           ((g.N + t.n - 1) / t.n) * g.nb1 * g.nb2;
+    int64_t blocks = 0;
+    for (int k = 0; k < n; ++k) blocks += tiles_of(g[k], t);
     const int64_t want =
-        (std::max(1, g.split_target) + blocks - 1) / blocks;
+        (std::max(1, g[0].split_target) + blocks - 1) / blocks;
     const int maxs = (int)std::max<int64_t>(
-        1, std::min<int64_t>(std::min<int64_t>(want, 2048),
-                             g.K / (4 * BK)));
+        1, std::min<int64_t>(std::min<int64_t>(want, 2048), K / (4 * BK)));
     for (int sp = 1; sp <= maxs; sp += 1 + sp / 8) {
-      const double e = estimate_us(g, t, sp);
+      const int kc = ((K + sp - 1) / sp + BK - 1) / BK * BK;
+      const double e =
+          estimate_us(g, cblk, n, t, std::max(BK, std::min(kc, whole)));
       if (e < us * 0.98) {
         us = e;
-        best = Plan{t, sp};
+        best = Plan{t, std::max(BK, std::min(kc, whole))};
       }
     }
   }
@@ -572,54 +613,45 @@ Plan plan_of(const Gemm &g) {
 }
 
 template <typename K3>
-void launch(K3 kernel, const GemmDev &d, hipStream_t s) {
-  const int64_t nblocks =
-      (int64_t)d.tilesM * d.tilesN * d.splits * d.nb1 * d.nb2;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)nblocks), dim3(NT), 0, s, d);
+void launch(K3 kernel, const GemmGroup &d, int64_t blocks, hipStream_t s) {
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(NT), 0, s, d);
   FTCC_CHECK_HIP(hipGetLastError());
 }
 
 template <typename T, int TM, int TN>
-void launch_tile(bool amf, bool bnf, bool kl, const GemmDev &d,
+void launch_tile(bool amf, bool bnf, bool kl, const GemmGroup &d, int64_t nb,
                  hipStream_t s) {
-  if (kl) launch(gemm_mfma_kernel<T, false, false, TM, TN, true>, d, s);
+  if (kl) launch(gemm_mfma_kernel<T, false, false, TM, TN, true>, d, nb, s);
   else if (amf && bnf)
-    launch(gemm_mfma_kernel<T, true, true, TM, TN, false>, d, s);
-  else if (amf) launch(gemm_mfma_kernel<T, true, false, TM, TN, false>, d, s);
-  else if (bnf) launch(gemm_mfma_kernel<T, false, true, TM, TN, false>, d, s);
-  else launch(gemm_mfma_kernel<T, false, false, TM, TN, false>, d, s);
+    launch(gemm_mfma_kernel<T, true, true, TM, TN, false>, d, nb, s);
+  else if (amf)
+    launch(gemm_mfma_kernel<T, true, false, TM, TN, false>, d, nb, s);
+  else if (bnf)
+    launch(gemm_mfma_kernel<T, false, true, TM, TN, false>, d, nb, s);
+  else launch(gemm_mfma_kernel<T, false, false, TM, TN, false>, d, nb, s);
 }
 
 template <typename T>
-void launch_layout(Tile tl, bool amf, bool bnf, bool kl, const GemmDev &d,
-                   hipStream_t s) {
-  if (tl.m == 64 && tl.n == 64) launch_tile<T, 64, 64>(amf, bnf, kl, d, s);
-  else if (tl.m == 64) launch_tile<T, 64, 128>(amf, bnf, kl, d, s);
-  else if (tl.n == 64) launch_tile<T, 128, 64>(amf, bnf, kl, d, s);
-  else launch_tile<T, 128, 128>(amf, bnf, kl, d, s);
+void launch_layout(Tile tl, bool amf, bool bnf, bool kl, const GemmGroup &d,
+                   int64_t nb, hipStream_t s) {
+  if (tl.m == 64 && tl.n == 64)
+    launch_tile<T, 64, 64>(amf, bnf, kl, d, nb, s);
+  else if (tl.m == 64) launch_tile<T, 64, 128>(amf, bnf, kl, d, nb, s);
+  else if (tl.n == 64) launch_tile<T, 128, 64>(amf, bnf, kl, d, nb, s);
+  else launch_tile<T, 128, 128>(amf, bnf, kl, d, nb, s);
 }
 
-}  // namespace
+// operand layouts of the kernel instantiations
+bool a_mfast(const Gemm &g) { return g.sAm == 1 && g.sAk != 1; }
+bool b_nfast(const Gemm &g) { return g.sBn == 1 && g.sBk != 1; }
 
-size_t gemm_partial_elems(const Gemm &g) {
-  const int R = (g.K > 0 ? plan_of(g).splits : 1) * (g.reduce_b2 ? g.nb2 : 1);
-  if (R <= 1) return 0;
-  const int nbC = g.reduce_b2 ? g.nb1 : g.nb1 * g.nb2;
-  return (size_t)R * nbC * g.M * g.N;
-}
-
-void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
-  if (g.M <= 0 || g.N <= 0 || g.nb1 <= 0 || g.nb2 <= 0) return;
-  require(precision == FTCC_PREC_FP64 || precision == FTCC_PREC_FP32,
-          "the generic GEMM runs FP64 or FP32 (bf16x3 uses sbgemm)");
-  const int bk = BK;
+GemmDev device_form(const Gemm &g) {
   GemmDev d;
   d.M = g.M;
   d.N = g.N;
   d.K = g.K;
   d.nb1 = g.nb1;
   d.nb2 = g.nb2;
-  d.reduce_b2 = g.reduce_b2 ? 1 : 0;
   d.alpha = g.alpha;
   d.beta = g.beta;
   d.A = g.A;
@@ -637,26 +669,6 @@ void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
   d.sCn = g.sCn;
   d.sC1 = g.sC1;
   d.sC2 = g.sC2;
-  const Plan pl = plan_of(g);
-  const Tile tl = pl.t;
-  d.tilesM = (g.M + tl.m - 1) / tl.m;
-  d.tilesN = (g.N + tl.n - 1) / tl.n;
-  d.m_inner = d.tilesM < d.tilesN ? 1 : 0;
-  if (g.K <= 0) {
-    // C = beta*C only
-    d.splits = 1;
-    d.kchunk = 0;
-  } else {
-    d.splits = pl.splits;
-    // round the chunk to whole slabs of the active precision
-    int kc = (g.K + d.splits - 1) / d.splits;
-    kc = ((kc + bk - 1) / bk) * bk;
-    d.kchunk = kc;
-    d.splits = (g.K + kc - 1) / kc;
-  }
-  const int R = d.splits * (g.reduce_b2 ? g.nb2 : 1);
-  d.nbC = g.reduce_b2 ? g.nb1 : g.nb1 * g.nb2;
-  d.partial = nullptr;
   d.rmap = g.rmap;
   d.cmap = g.cmap;
   d.D = g.D;
@@ -698,6 +710,8 @@ void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
   d.K2 = g.K2 > 0 ? g.K2 : (1 << 30);
   d.sAk0 = g.sAk0;
   d.sAk1 = g.sAk1;
+  d.sBk0 = g.sBk0;
+  d.sBk1 = g.sBk1;
   require((g.mlvl < 0 || (g.mmap && g.mlvl <= 2)) &&
               (g.nlvl < 0 || (g.nmap && g.nlvl <= 2)),
           "GEMM level map without a map or level");
@@ -705,37 +719,119 @@ void gemm_run(const Gemm &g, int precision, Scratch &scr, hipStream_t s) {
   d.nmap = g.nmap;
   d.mlvl = g.mmap ? g.mlvl : -1;
   d.nlvl = g.nmap ? g.nlvl : -1;
-  d.sBk0 = g.sBk0;
-  d.sBk1 = g.sBk1;
-  if (R > 1) {
-    const size_t need = (size_t)R * d.nbC * g.M * g.N;
-    require(need <= scr.partial_elems, "GEMM split-K scratch too small",
-            FTCC_ENOMEM);
-    d.partial = scr.partial;
-  }
-  const bool amf = (g.sAm == 1 && g.sAk != 1);
-  const bool bnf = (g.sBn == 1 && g.sBk != 1);
-  const bool kl = g.K2 > 0;
-  require(!kl || (!amf && !bnf),
+  require(g.K2 == 0 || (!a_mfast(g) && !b_nfast(g)),
           "K over several indices needs both operands K-fastest");
-  if (precision == FTCC_PREC_FP64)
-    launch_layout<double>(tl, amf, bnf, kl, d, s);
-  else
-    launch_layout<float>(tl, amf, bnf, kl, d, s);
-  if (R > 1) {
-    const int64_t total = (int64_t)d.nbC * g.M * g.N;
-    // few partials of a large output: a thread for each element
-    if (R <= FEW && total >= 32 * 1024) {
-      const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65536);
-      hipLaunchKernelGGL(reduce_few_kernel, dim3(blocks), dim3(256), 0, s, d,
-                         R);
-    } else {
-      const int blocks = (int)std::min<int64_t>((total + 63) / 64, 65536);
-      hipLaunchKernelGGL(reduce_partial_kernel, dim3(blocks), dim3(64 * RG),
-                         0, s, d, R);
-    }
-    FTCC_CHECK_HIP(hipGetLastError());
+  d.partial = nullptr;
+  d.rbase = 0;
+  d.R = 1;
+  return d;
+}
+
+}  // namespace
+
+bool gemm_groupable(const Gemm &x, const Gemm &y) {
+  return a_mfast(x) == a_mfast(y) && b_nfast(x) == b_nfast(y) &&
+         (x.K2 > 0) == (y.K2 > 0) && x.nb1 == y.nb1 && x.nb2 == y.nb2;
+}
+
+size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n) {
+  const Plan pl = plan_of(g, cblk, n);
+  size_t need = 0;
+  for (int k = 0; k < n; ++k) {
+    const int sp = splits_of(g[k], pl.kc);
+    bool shared = false;
+    for (int q = 0; q < n; ++q) shared |= q != k && cblk[q] == cblk[k];
+    if (sp > 1 || shared)
+      need += (size_t)sp * g[k].M * g[k].N * g[k].nb1 * g[k].nb2;
   }
+  return need;
+}
+
+void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
+                    Scratch &scr, hipStream_t s) {
+  require(precision == FTCC_PREC_FP64 || precision == FTCC_PREC_FP32,
+          "the generic GEMM runs FP64 or FP32 (bf16x3 uses sbgemm)");
+  require(n >= 1 && n <= GEMM_GROUP, "GEMM group size");
+  const Plan pl = plan_of(g, cblk, n);
+  const Tile tl = pl.t;
+  GemmGroup grp, red;
+  grp.n = red.n = 0;
+  int64_t blocks = 0, rblocks = 0, elems = 0;
+  size_t used = 0;
+  int maxR = 1;
+  for (int k = 0; k < n; ++k) {
+    if (g[k].M <= 0 || g[k].N <= 0 || g[k].nb1 <= 0 || g[k].nb2 <= 0) continue;
+    require(gemm_groupable(g[0], g[k]), "GEMM group of different layouts");
+    GemmDev &d = grp.pr[grp.n];
+    d = device_form(g[k]);
+    d.tilesM = (g[k].M + tl.m - 1) / tl.m;
+    d.tilesN = (g[k].N + tl.n - 1) / tl.n;
+    d.m_inner = d.tilesM < d.tilesN ? 1 : 0;
+    d.splits = splits_of(g[k], pl.kc);
+    d.kchunk = pl.kc;
+    grp.tile0[grp.n++] = (int)blocks;
+    blocks += (int64_t)d.tilesM * d.tilesN * d.splits * d.nb1 * d.nb2;
+  }
+  if (grp.n == 0) return;
+  require(blocks < (1LL << 31), "GEMM grid too large");
+  // partial sums: each output of several products, or of a split K, in the
+  // order the products are given
+  int q = 0;
+  std::vector<int> blk(grp.n);
+  for (int k = 0; k < n; ++k)
+    if (!(g[k].M <= 0 || g[k].N <= 0 || g[k].nb1 <= 0 || g[k].nb2 <= 0))
+      blk[q++] = cblk[k];
+  for (int k = 0; k < grp.n; ++k) {
+    int R = 0;
+    bool first = true;
+    for (int j = 0; j < grp.n; ++j)
+      if (blk[j] == blk[k]) {
+        if (j < k) first = false;
+        R += grp.pr[j].splits;
+      }
+    if (R == 1 || !first) continue;
+    GemmDev &d = grp.pr[k];
+    const int64_t per = (int64_t)d.M * d.N * d.nb1 * d.nb2;
+    double *part = scr.partial + used;
+    used += (size_t)R * per;
+    require(used <= scr.partial_elems, "GEMM split-K scratch too small",
+            FTCC_ENOMEM);
+    int rb = 0;
+    for (int j = k; j < grp.n; ++j)
+      if (blk[j] == blk[k]) {
+        GemmDev &e = grp.pr[j];
+        require(e.M == d.M && e.N == d.N, "GEMM group: outputs differ");
+        e.partial = part;
+        e.rbase = rb;
+        rb += e.splits;
+      }
+    d.R = R;
+    red.pr[red.n++] = d;
+    maxR = std::max(maxR, R);
+    elems += per;
+  }
+  const bool amf = a_mfast(g[0]), bnf = b_nfast(g[0]), kl = g[0].K2 > 0;
+  if (precision == FTCC_PREC_FP64)
+    launch_layout<double>(tl, amf, bnf, kl, grp, blocks, s);
+  else
+    launch_layout<float>(tl, amf, bnf, kl, grp, blocks, s);
+  if (red.n == 0) return;
+  // few partials of a large output: a thread for each element
+  const bool few = maxR <= FEW && elems >= 32 * 1024;
+  const int unit = few ? 256 : 64;
+  for (int k = 0; k < red.n; ++k) {
+    const GemmDev &d = red.pr[k];
+    red.tile0[k] = (int)rblocks;
+    rblocks += ((int64_t)d.M * d.N * d.nb1 * d.nb2 + unit - 1) / unit;
+  }
+  require(rblocks < (1LL << 31), "GEMM grid too large");
+  if (few)
+    hipLaunchKernelGGL(reduce_few_kernel, dim3((unsigned)rblocks), dim3(256),
+                       0, s, red);
+  else
+    hipLaunchKernelGGL(reduce_partial_kernel, dim3((unsigned)rblocks),
+                       dim3(64 * RG), 0, s, red);
+  FTCC_CHECK_HIP(hipGetLastError());
 }
 
 }  // namespace ftcc

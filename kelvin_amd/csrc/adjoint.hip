@@ -137,12 +137,13 @@ __device__ inline double proj(const double *x, int a, int b, int i, int j,
                  at(b, a, j, i));
 }
 
-// S = P(gtau + gt/2) and out2 = P(acc + gt/2) + S: the doubles of J^T
-// (the transposed residual is projected onto antisymmetric tensors) and
-// the adjoint of tau/taut for the t1 chain rule
-__global__ void assemble_kernel(const double *acc, const double *gtau,
-                                const double *gt, int V, int O, int nb,
-                                double *S, double *out2) {
+// S = P(gtau + gt/2) and out2 = P(v + gt/2) + S, v[a,b,i,j] =
+// acc[a,i,b,j] - q[b,i,a,j] / 2: the doubles of J^T (the transposed residual
+// is projected onto antisymmetric tensors) and the adjoint of tau/taut for
+// the t1 chain rule, for dense gtau (project_doubles: packed)
+__global__ void assemble_kernel(const double *acc, const double *q,
+                                const double *gtau, const double *gt, int V,
+                                int O, int nb, double *S, double *out2) {
   const int64_t n = (int64_t)V * V * O * O;
   ADJ_LOOP(e, n * nb) {
     const int64_t y = e / n * n;
@@ -153,10 +154,16 @@ __global__ void assemble_kernel(const double *acc, const double *gtau,
     r /= O;
     const int b = (int)(r % V);
     const int a = (int)(r / V);
+    auto v = [&](int p, int s, int k, int l) {
+      return acc[y + (((int64_t)p * O + k) * V + s) * O + l] -
+             0.5 * q[y + (((int64_t)s * O + k) * V + p) * O + l];
+    };
     const double pt = proj(gt + y, a, b, i, j, V, O);
     const double s = proj(gtau + y, a, b, i, j, V, O) + 0.5 * pt;
     S[e] = s;
-    out2[e] = proj(acc + y, a, b, i, j, V, O) + 0.5 * pt + s;
+    out2[e] = 0.25 * (v(a, b, i, j) - v(b, a, i, j) - v(a, b, j, i) +
+                      v(b, a, j, i)) +
+              0.5 * pt + s;
   }
 }
 
@@ -1048,8 +1055,10 @@ void con(ftcc_ctx *c, double alpha, const Ten &A0, const Ten &B0, double beta,
 // (each array holds `n` grid points, one after another)
 struct AdjSlice {
   int n = 0;
-  double *wmnij = nullptr, *wefab = nullptr, *wmbej = nullptr, *zt = nullptr,
-         *zv = nullptr;
+  // intermediates of the O(n^6) products: operand copies in the packed spin
+  // layout, whole tensors otherwise (wmbej as [e,m,b,j], t2r not formed)
+  double *wmnij = nullptr, *wefab = nullptr, *wmbej = nullptr, *t2r = nullptr;
+  double *zt = nullptr, *zv = nullptr;
   double *me = nullptr, *ae = nullptr, *mi = nullptr, *be = nullptr,
          *mj = nullptr;   // the Fock-type intermediates
 };
@@ -1058,14 +1067,24 @@ struct Adjoint {
   const double *T1 = nullptr, *T2 = nullptr;   // the checkpoint
   int ng = 0;
   int nb = 1;                    // grid points of one application's launches
+  // the O(n^6) products run on spin-blocked, packed operand copies
+  bool blocked = false;
   AdjSlice cache;                // grid points [0, cache.n) are kept
   AdjSlice work;                 // intermediates of uncached grid points
-  // application buffers of nb grid points
-  double *tau = nullptr, *taut = nullptr, *ar = nullptr, *vT = nullptr,
-         *acc = nullptr, *gtau = nullptr, *gt = nullptr, *gw = nullptr,
-         *q = nullptr, *u = nullptr, *u2 = nullptr;
+  // buffers of nb grid points (prepare_points and apply_points each say
+  // what they hold when)
+  double *acc = nullptr, *gtau = nullptr, *gt = nullptr, *gw = nullptr,
+         *q = nullptr;
   double *gFmj = nullptr, *gFbe = nullptr, *gFae = nullptr, *gFmi = nullptr,
          *gFme = nullptr;
+  // operand copies (blocked): of the adjoint amplitudes (tau-like with rows
+  // (i,j) and with rows (a,b), ring) and of gw, nb grid points, and of the
+  // ring integrals
+  double *vB = nullptr, *vA = nullptr, *vR = nullptr, *gwA = nullptr,
+         *ring = nullptr;
+  // split-bf16 copies for the low-precision form (lowp_arena): made at each
+  // application
+  double *lowp = nullptr;
   double *partials = nullptr;
   // lambda update: per-slice scales and weights (4 * ng on the device, the
   // host copy alive until the stream passes the upload), singles energy
@@ -1085,13 +1104,73 @@ double *aalloc(ftcc_ctx *c, Adjoint *A, int64_t n) {
   return p;
 }
 
+// The operand copies of the five products of J^T at one grid point: rows
+// and K are pair spaces (ab and ij packed, ring), stored with row stride
+// K.total.  The three blocks of each are (row, K) class pairs: equal total
+// spin (LADDER), opposite spin flip (CROSS) or the same one (SAME).
+enum AdjKind { LADDER_OP, CROSS_OP, SAME_OP };
+struct AdjOp {
+  const PairSpace *R, *K;
+  int kind;
+  int64_t size() const { return (int64_t)R->total * K->total; }
+};
+AdjOp op_wefab(const ftcc_ctx *c) {
+  return AdjOp{&c->ps_vvp, &c->ps_vvp, LADDER_OP};
+}
+AdjOp op_wmnij(const ftcc_ctx *c) {
+  return AdjOp{&c->ps_oop, &c->ps_oop, LADDER_OP};
+}
+AdjOp op_vB(const ftcc_ctx *c) {
+  return AdjOp{&c->ps_oop, &c->ps_vvp, LADDER_OP};
+}
+AdjOp op_vA(const ftcc_ctx *c) {
+  return AdjOp{&c->ps_vvp, &c->ps_oop, LADDER_OP};
+}
+AdjOp op_cross(const ftcc_ctx *c) {
+  return AdjOp{&c->ps_vo, &c->ps_vo, CROSS_OP};
+}
+AdjOp op_same(const ftcc_ctx *c) {
+  return AdjOp{&c->ps_vo, &c->ps_vo, SAME_OP};
+}
+struct Span {
+  int start = 0, len = 0, count = 0;
+};
+Span span(const PairSpace &p, int c1, int c2 = -1) {
+  Span g{p.start[c1], p.len[c1], p.count[c1]};
+  if (c2 >= 0) {
+    g.len += p.len[c2];
+    g.count += p.count[c2];
+  }
+  return g;
+}
+// the class ranges of block q (0..2) of a pair space; `other`: crossed
+Span block_span(const PairSpace &p, bool ladder, int q, bool other) {
+  if (ladder) return q == 0 ? span(p, 0) : q == 1 ? span(p, 1, 2) : span(p, 3);
+  if (q == 0) return span(p, 0, 3);
+  return span(p, (q == 1) != other ? 1 : 2);
+}
+
+// per-grid-point doubles of the kept intermediates of the products
+struct SliceSize {
+  int64_t wmnij, wefab, wmbej, t2r;
+};
+SliceSize slice_size(const ftcc_ctx *c, bool blocked) {
+  const int64_t O = c->no, V = c->nv;
+  if (blocked)
+    return SliceSize{op_wmnij(c).size(), op_wefab(c).size(),
+                     op_same(c).size(), op_cross(c).size()};
+  return SliceSize{O * O * O * O, V * V * V * V, O * V * V * O, 0};
+}
+
 void alloc_slice(ftcc_ctx *c, Adjoint *A, AdjSlice &s, int n) {
   const int64_t O = c->no, V = c->nv;
   s = AdjSlice();
   if (n <= 0) return;
-  s.wmnij = aalloc(c, A, n * O * O * O * O);
-  s.wefab = aalloc(c, A, n * V * V * V * V);
-  s.wmbej = aalloc(c, A, n * O * V * V * O);
+  const SliceSize z = slice_size(c, A->blocked);
+  s.wmnij = aalloc(c, A, n * z.wmnij);
+  s.wefab = aalloc(c, A, n * z.wefab);
+  s.wmbej = aalloc(c, A, n * z.wmbej);
+  if (A->blocked) s.t2r = aalloc(c, A, n * z.t2r);
   s.zt = aalloc(c, A, n * V * V * V * O);
   s.zv = aalloc(c, A, n * V * O * O * O);
   s.me = aalloc(c, A, n * (O * V + 2 * V * V + 2 * O * O));
@@ -1102,13 +1181,16 @@ void alloc_slice(ftcc_ctx *c, Adjoint *A, AdjSlice &s, int n) {
   s.n = n;
 }
 // the intermediates from grid point y of the block on
-AdjSlice at_point(const ftcc_ctx *c, const AdjSlice &b, int64_t y) {
+AdjSlice at_point(const ftcc_ctx *c, const Adjoint *A, const AdjSlice &b,
+                  int64_t y) {
   const int64_t O = c->no, V = c->nv;
+  const SliceSize z = slice_size(c, A->blocked);
   AdjSlice s = b;
   s.n = b.n - (int)y;
-  s.wmnij += y * O * O * O * O;
-  s.wefab += y * V * V * V * V;
-  s.wmbej += y * O * V * V * O;
+  s.wmnij += y * z.wmnij;
+  s.wefab += y * z.wefab;
+  s.wmbej += y * z.wmbej;
+  if (s.t2r) s.t2r += y * z.t2r;
   s.zt += y * V * V * V * O;
   s.zv += y * V * O * O * O;
   s.me += y * O * V;
@@ -1119,15 +1201,33 @@ AdjSlice at_point(const ftcc_ctx *c, const AdjSlice &b, int64_t y) {
   return s;
 }
 
-int64_t slice_bytes(const ftcc_ctx *c) {
+int64_t slice_bytes(const ftcc_ctx *c, bool blocked) {
   const int64_t O = c->no, V = c->nv;
-  return 8 * (O * O * O * O + V * V * V * V + O * V * V * O + V * V * V * O +
+  const SliceSize z = slice_size(c, blocked);
+  return 8 * (z.wmnij + z.wefab + z.wmbej + z.t2r + V * V * V * O +
               V * O * O * O + O * V + 2 * V * V + 2 * O * O);
 }
-// application buffers of one grid point
-int64_t buffer_bytes(const ftcc_ctx *c) {
-  const int64_t O = c->no, V = c->nv;
-  return 8 * (9 * V * V * O * O + V * O * O * O + V * V * V * O);
+// doubles of the application buffers of one grid point: the five shared by
+// prepare_points and apply_points, and the operand copies
+int64_t max3(int64_t x, int64_t y, int64_t z) {
+  return std::max(x, std::max(y, z));
+}
+struct BufferSize {
+  int64_t acc, gt, q, s2;
+};
+BufferSize buffer_size(const ftcc_ctx *c) {
+  const int64_t O = c->no, V = c->nv, S2 = V * V * O * O;
+  return BufferSize{max3(S2, V * V * V * V, O * O * O * O),
+                    std::max(S2, O * O * O * V), std::max(S2, V * V * V * O),
+                    S2};
+}
+int64_t buffer_bytes(const ftcc_ctx *c, bool blocked) {
+  const BufferSize z = buffer_size(c);
+  int64_t n = z.acc + 2 * z.s2 + z.gt + z.q;
+  if (blocked)
+    n += op_vB(c).size() + op_vA(c).size() + op_cross(c).size() +
+         op_same(c).size();
+  return 8 * n;
 }
 
 // the adjoint's reduction buffers (allocated on first use)
@@ -1142,33 +1242,168 @@ Adjoint *adjoint_ws(ftcc_ctx *c) {
 // the buffers of one application of J^T to nb grid points
 // (ftcc_adjoint_begin); the intermediates of uncached ones if any
 void alloc_apply_buffers(ftcc_ctx *c, Adjoint *A, int nb, bool uncached) {
-  const int64_t O = c->no, V = c->nv, S2 = V * V * O * O;
-  for (double **p : {&A->tau, &A->taut, &A->ar, &A->vT, &A->acc, &A->gtau,
-                     &A->gt, &A->gw, &A->q})
-    *p = aalloc(c, A, nb * S2);
-  A->u = aalloc(c, A, nb * O * V * O * O);
-  A->u2 = aalloc(c, A, nb * V * V * V * O);
+  const int64_t O = c->no, V = c->nv;
+  const BufferSize z = buffer_size(c);
+  A->acc = aalloc(c, A, nb * z.acc);
+  A->gtau = aalloc(c, A, nb * z.s2);
+  A->gt = aalloc(c, A, nb * z.gt);
+  A->gw = aalloc(c, A, nb * z.s2);
+  A->q = aalloc(c, A, nb * z.q);
   A->gFmj = aalloc(c, A, nb * (2 * V * V + 2 * O * O + V * O));
   A->gFbe = A->gFmj + nb * O * O;
   A->gFae = A->gFbe + nb * V * V;
   A->gFmi = A->gFae + nb * V * V;
   A->gFme = A->gFmi + nb * O * O;
+  if (A->blocked) {
+    A->vB = aalloc(c, A, nb * op_vB(c).size());
+    A->vA = aalloc(c, A, nb * op_vA(c).size());
+    A->vR = aalloc(c, A, nb * op_cross(c).size());
+    A->gwA = aalloc(c, A, nb * op_same(c).size());
+    A->ring = aalloc(c, A, op_cross(c).size());
+  }
   alloc_slice(c, A, A->work, uncached ? nb : 0);
   A->nb = nb;
+}
+
+// Write the spin blocks of operand copy `dst` (nb grid points) from
+// src[b*sb + row*sr + k*sc], row and k dense pair indices.
+void put_op(ftcc_ctx *c, const AdjOp &o, const double *src, int64_t sr,
+            int64_t sc, int64_t sb, double *dst, int nb) {
+  for (int q = 0; q < 3; ++q) {
+    const bool lad = o.kind == LADDER_OP;
+    const Span r = block_span(*o.R, lad, q, false),
+               k = block_span(*o.K, lad, q, o.kind == CROSS_OP);
+    if (r.len == 0 || k.len == 0) continue;
+    gather_plain(src, sr, sc, sb, o.R->d_map + r.start, r.len,
+                 o.K->d_map + k.start, k.len, o.K->total,
+                 dst + (int64_t)r.start * o.K->total + k.start, false,
+                 o.size(), nb, c->stream);
+  }
+}
+// ... the ring copy X[a,b,i,j] -> [(a,i)][(b,j)] of doubles
+void put_ring_op(ftcc_ctx *c, const double *x2, double *dst, int nb) {
+  const AdjOp o = op_cross(c);
+  for (int q = 0; q < 3; ++q) {
+    const Span r = block_span(*o.R, false, q, false),
+               k = block_span(*o.K, false, q, true);
+    if (r.len == 0 || k.len == 0) continue;
+    amp_gather_plain(AMP_T2R, x2, x2, c->nv, c->no, o.R->d_map + r.start,
+                     r.len, o.K->d_map + k.start, k.len, o.K->total,
+                     dst + (int64_t)r.start * o.K->total + k.start, false,
+                     o.size(), nb, c->stream);
+  }
+}
+
+// One product C[R, C] = alpha A[R, K] B[C, K]^T + beta C of operand copies
+// at nb grid points (sa, sb = 0: shared by them), its blocks in one launch,
+// written through the pair maps with row and column strides sr, sc.  As
+// split-bf16 products when `low` (the copies are split here).
+void op_product(ftcc_ctx *c, Adjoint *A, double alpha, const AdjOp &oa,
+                const double *a, int64_t sa, const AdjOp &ob, const double *b,
+                int64_t sb, double beta, double *C, int64_t sr, int64_t sc,
+                int nb, bool low, int line = __builtin_LINE()) {
+  const bool lad = oa.kind == LADDER_OP;
+  const int64_t S2 = (int64_t)c->nv * c->nv * c->no * c->no;
+  const int64_t la = oa.K->total, lb = ob.K->total;
+  PgProblem pg[3];
+  SbProblem sp[3];
+  SplitMat xa, xb;
+  const int na = sa ? nb : 1, nbb = sb ? nb : 1;
+  if (low) {
+    xa.ld = split_ld((int)la);
+    xb.ld = split_ld((int)lb);
+    const int64_t ea = (int64_t)oa.R->total * xa.ld,
+                  eb = (int64_t)ob.R->total * xb.ld;
+    xa.bstride = sa ? ea : 0;
+    xb.bstride = sb ? eb : 0;
+    xa.hi = (__bf16 *)A->lowp;
+    xa.lo = xa.hi + na * ea;
+    xb.hi = xa.lo + na * ea;
+    xb.lo = xb.hi + nbb * eb;
+  }
+  int np = 0;
+  double flops = 0.0;
+  for (int q = 0; q < 3; ++q) {
+    const Span r = block_span(*oa.R, lad, q, false),
+               k = block_span(*oa.K, lad, q, oa.kind == CROSS_OP),
+               n = block_span(*ob.R, lad, q,
+                              (oa.kind == CROSS_OP) != (ob.kind == CROSS_OP));
+    if (!r.count || !n.count || (!k.count && beta != 0.0)) continue;
+    const int64_t ao = (int64_t)r.start * la + k.start,
+                  bo = (int64_t)n.start * lb + k.start;
+    flops += 2.0 * r.count * (double)n.count * k.count * nb;
+    if (low) {
+      SplitMat ua = xa, ub = xb;
+      const int64_t ua0 = (int64_t)r.start * xa.ld + k.start,
+                    ub0 = (int64_t)n.start * xb.ld + k.start;
+      ua.hi += ua0;
+      ua.lo += ua0;
+      ub.hi += ub0;
+      ub.lo += ub0;
+      split_rows(a + ao, la, sa, r.len, k.len, ua, na, c->stream);
+      split_rows(b + bo, lb, sb, n.len, k.len, ub, nbb, c->stream);
+      sp[np++] = SbProblem{r.len, n.len, k.len, ua, ub,
+                           oa.R->d_map + r.start, ob.R->d_map + n.start};
+    } else {
+      pg[np++] = PgProblem{r.len, n.len, k.len, a + ao, b + bo, la, sa, lb,
+                           sb, oa.R->d_map + r.start, ob.R->d_map + n.start};
+    }
+  }
+  if (np == 0) return;
+  c->cur_line = c->site_override ? c->site_override : line;
+  const int tok = prof_begin(c, ftcc_ctx::PROF_PRODUCTS, flops, 0.0);
+  if (low)
+    sbgemm_grouped(np, sp, nb, alpha, beta, C, sr, sc, S2, c->stream);
+  else
+    pgemm_grouped(np, pg, nb, false, alpha, beta, C, sr, sc, S2, c->stream);
+  prof_end(c, tok);
+  c->cur_line = 0;
+}
+
+// In the low-precision mode of the lambda iteration a product of which each
+// spin block (of single spins in every index) has at least
+// adj_lowp_min_flops runs split-bf16, the others FP64: v and o the numbers
+// of virtual and occupied indices of the product.
+bool low_product(const ftcc_ctx *c, int v, int o) {
+  if (c->adj_prec != FTCC_PREC_BF16X3) return false;
+  auto least = [](const int *n) {
+    return !n[0] ? n[1] : !n[1] ? n[0] : std::min(n[0], n[1]);
+  };
+  return 2.0 * std::pow((double)least(c->v_count), v) *
+             std::pow((double)least(c->o_count), o) >=
+         c->adj_lowp_min_flops;
+}
+// room for the split copies of the largest product's operands
+void ensure_lowp(ftcc_ctx *c, Adjoint *A) {
+  if (A->lowp) return;
+  const int64_t ring = (int64_t)c->ps_vo.total * split_ld(c->ps_vo.total);
+  const int64_t l1 = (int64_t)c->ps_vvp.total * split_ld(c->ps_vvp.total) +
+                     (int64_t)c->ps_oop.total * split_ld(c->ps_vvp.total);
+  const int64_t l2 = (int64_t)c->ps_vvp.total * split_ld(c->ps_oop.total) +
+                     (int64_t)c->ps_oop.total * split_ld(c->ps_oop.total);
+  // two bf16 arrays of each element: half a double
+  A->lowp = aalloc(c, A, A->nb * max3(2 * ring, l1, l2) / 2 + 8);
 }
 
 void copy(ftcc_ctx *c, double *dst, const double *src, int64_t n, double a) {
   axpby(dst, src, n, a, 0.0, c->stream);
 }
 
-// the fixed (amplitude-only) intermediates of nb grid points
+// the fixed (amplitude-only) intermediates of nb grid points (tau, taut and
+// the ring amplitude in gtau, gt and gw; in the blocked form each tensor of
+// the products is formed in acc and its operand copy kept)
 void prepare_points(ftcc_ctx *c, Adjoint *A, const double *t1,
                     const double *t2, const AdjSlice &s, int nb) {
   const int O = c->no, V = c->nv;
   const int64_t S2 = (int64_t)V * V * O * O;
+  const int64_t VO = (int64_t)V * O, VV = (int64_t)V * V, OO = (int64_t)O * O;
+  double *tau = A->gtau, *taut = A->gt, *ar = A->gw;
+  double *wmnij = A->blocked ? A->acc : s.wmnij,
+         *wefab = A->blocked ? A->acc : s.wefab,
+         *wmbej = A->blocked ? A->acc : s.wmbej;
   hipStream_t st = c->stream;
   hipLaunchKernelGGL(tau_kernel, dim3(grid_for(S2 * nb)), dim3(AT), 0, st, t1,
-                     t2, V, O, nb, A->tau, A->taut, A->ar);
+                     t2, V, O, nb, tau, taut, ar);
   FTCC_CHECK_HIP(hipGetLastError());
   auto cn = [&](double alpha, const Ten &X, const Ten &Y, double beta,
                 const Ten &Z, int line = __builtin_LINE()) {
@@ -1184,7 +1419,7 @@ void prepare_points(ftcc_ctx *c, Adjoint *A, const double *t1,
       bten(c, s.ae, "ae"));
   cn(-1.0, ten(c, I[2], "amfe"), bten(c, t1, "fm"), 1.0,
       bten(c, s.ae, "ae"));
-  cn(-0.5, bten(c, A->taut, "afmn"), ten(c, I[5], "mnef"), 1.0,
+  cn(-0.5, bten(c, taut, "afmn"), ten(c, I[5], "mnef"), 1.0,
       bten(c, s.ae, "ae"));
   // Fmi = F.oo + 1/2 F.ov.t1 + t1.ooov + 1/2 oovv.taut
   bcast(s.mi, c->F[0], (int64_t)O * O, nb, 1.0, 0.0, st);
@@ -1192,7 +1427,7 @@ void prepare_points(ftcc_ctx *c, Adjoint *A, const double *t1,
       bten(c, s.mi, "mi"));
   cn(1.0, ten(c, I[7], "mnie"), bten(c, t1, "en"), 1.0,
       bten(c, s.mi, "mi"));
-  cn(0.5, ten(c, I[5], "mnef"), bten(c, A->taut, "efin"), 1.0,
+  cn(0.5, ten(c, I[5], "mnef"), bten(c, taut, "efin"), 1.0,
       bten(c, s.mi, "mi"));
   // Fbe = Fae - 1/2 t1.Fme, Fmj = Fmi + 1/2 Fme.t1
   copy(c, s.be, s.ae, nb * (int64_t)V * V, 1.0);
@@ -1200,42 +1435,51 @@ void prepare_points(ftcc_ctx *c, Adjoint *A, const double *t1,
   copy(c, s.mj, s.mi, nb * (int64_t)O * O, 1.0);
   cn(0.5, bten(c, s.me, "me"), bten(c, t1, "ej"), 1.0, bten(c, s.mj, "mj"));
   // Wh_mnij = 1/2 (oooo + P(ij) t1.ooov) + 1/4 oovv.tau
-  bcast(s.wmnij, I[8], (int64_t)O * O * O * O, nb, 0.5, 0.0, st);
+  bcast(wmnij, I[8], (int64_t)O * O * O * O, nb, 0.5, 0.0, st);
   cn(0.5, ten(c, I[7], "mnie"), bten(c, t1, "ej"), 1.0,
-      bten(c, s.wmnij, "mnij"));
+      bten(c, wmnij, "mnij"));
   cn(-0.5, ten(c, I[7], "mnje"), bten(c, t1, "ei"), 1.0,
-      bten(c, s.wmnij, "mnij"));
-  cn(0.25, ten(c, I[5], "mnef"), bten(c, A->tau, "efij"), 1.0,
-      bten(c, s.wmnij, "mnij"));
+      bten(c, wmnij, "mnij"));
+  cn(0.25, ten(c, I[5], "mnef"), bten(c, tau, "efij"), 1.0,
+      bten(c, wmnij, "mnij"));
+  if (A->blocked)
+    put_op(c, op_wmnij(c), wmnij, OO, 1, OO * OO, s.wmnij, nb);
   // Wh_efab = 1/2 (vvvv - P(ab) t1.vovv) + 1/4 tau.oovv, stored [e,f,a,b]
   // vvvv[a,b,e,f] / 2 into [e,f,a,b]
-  permute4(I[0], s.wefab, V, V, V, V, (int64_t)V, 1, (int64_t)V * V * V,
+  permute4(I[0], wefab, V, V, V, V, (int64_t)V, 1, (int64_t)V * V * V,
            (int64_t)V * V, 0.5, 0.0, nb, 0, (int64_t)V * V * V * V, st);
   cn(-0.5, ten(c, I[2], "amef"), bten(c, t1, "bm"), 1.0,
-      bten(c, s.wefab, "efab"));
+      bten(c, wefab, "efab"));
   cn(0.5, ten(c, I[2], "bmef"), bten(c, t1, "am"), 1.0,
-      bten(c, s.wefab, "efab"));
-  cn(0.25, bten(c, A->tau, "abmn"), ten(c, I[5], "mnef"), 1.0,
-      bten(c, s.wefab, "efab"));
-  // Wmbej = <mb||ej> - t1.vovv + t1.ooov - oovv.(t2/2 + t1 t1)
-  // <mb||ej> = -vovo[b,m,e,j] into [m,b,e,j]
-  permute4(I[4], s.wmbej, V, O, V, O, (int64_t)V * O, (int64_t)V * V * O,
-           (int64_t)O, 1, -1.0, 0.0, nb, 0, S2, st);
+      bten(c, wefab, "efab"));
+  cn(0.25, bten(c, tau, "abmn"), ten(c, I[5], "mnef"), 1.0,
+      bten(c, wefab, "efab"));
+  if (A->blocked) put_op(c, op_wefab(c), wefab, VV, 1, VV * VV, s.wefab, nb);
+  // Wmbej = <mb||ej> - t1.vovv + t1.ooov - oovv.(t2/2 + t1 t1), stored
+  // [e,m,b,j]
+  bcast(wmbej, c->ovvo_ring, S2, nb, 1.0, 0.0, st);
   cn(-1.0, ten(c, I[2], "bmef"), bten(c, t1, "fj"), 1.0,
-      bten(c, s.wmbej, "mbej"));
+     bten(c, wmbej, "embj", "mb|ej"));
   cn(1.0, ten(c, I[7], "mnje"), bten(c, t1, "bn"), 1.0,
-      bten(c, s.wmbej, "mbej"));
-  cn(-1.0, ten(c, I[5], "mnef"), bten(c, A->ar, "fbjn"), 1.0,
-      bten(c, s.wmbej, "mbej"));
+     bten(c, wmbej, "embj", "mb|ej"));
+  cn(-1.0, ten(c, I[5], "mnef"), bten(c, ar, "fbjn"), 1.0,
+     bten(c, wmbej, "embj", "mb|ej"));
+  if (A->blocked) {
+    put_op(c, op_same(c), wmbej, VO, 1, S2, s.wmbej, nb);
+    put_ring_op(c, t2, s.t2r, nb);
+  }
   // Zt[e,a,b,i] = tau.ooov, Zv[a,m,i,j] = vovv.tau
-  cn(1.0, bten(c, A->tau, "abmn"), ten(c, I[7], "mnie"), 0.0,
+  cn(1.0, bten(c, tau, "abmn"), ten(c, I[7], "mnie"), 0.0,
       bten(c, s.zt, "eabi", "ab|ie"));
-  cn(1.0, ten(c, I[2], "amef"), bten(c, A->tau, "efij"), 0.0,
+  cn(1.0, ten(c, I[2], "amef"), bten(c, tau, "efij"), 0.0,
       bten(c, s.zv, "amij"));
 }
 
 // (g1, g2) = J^T (v1, v2) at nb grid points (v2 antisymmetric); g2 is
-// projected onto antisymmetric tensors
+// projected onto antisymmetric tensors.  acc, gw and q are ring tensors
+// ([a,i,e,m], [b,j,e,m], [b,j,f,n]); before their own contents, gt holds
+// the t1.v2 of the t1 t1 <mb||ej> term and q its v2.t1; S takes gw's place
+// once gw has been read.
 void apply_points(ftcc_ctx *c, Adjoint *A, const double *t1, const double *t2,
                   const AdjSlice &s, const double *v1, const double *v2,
                   double *g1, double *g2, int nb) {
@@ -1249,33 +1493,62 @@ void apply_points(ftcc_ctx *c, Adjoint *A, const double *t1, const double *t2,
   double *const *I = c->I;
   double *gFmj = A->gFmj, *gFbe = A->gFbe, *gFae = A->gFae, *gFmi = A->gFmi,
          *gFme = A->gFme;
-  // v2 transposed [i,j,a,b]
-  permute4(v2, A->vT, V, V, O, O, (int64_t)V, 1, (int64_t)O * V * V,
-           (int64_t)V * V, 1.0, 0.0, nb, S2, S2, st);
+  const int64_t VO = (int64_t)V * O, OO = (int64_t)O * O;
+  double *u = A->gt, *u2 = A->q, *S = A->gw;
   fill(g1, nb * (int64_t)V * O, 0.0, st);
-  const Ten V2 = bten(c, v2, "abij"), VT = bten(c, A->vT, "ijab");
+  const Ten V2 = bten(c, v2, "abij");
+  const Ten GW = bten(c, A->gw, "bjem", "mb|ej");
+  if (A->blocked) {
+    put_op(c, op_vB(c), v2, 1, OO, S2, A->vB, nb);
+    put_op(c, op_vA(c), v2, OO, 1, S2, A->vA, nb);
+    put_ring_op(c, v2, A->vR, nb);
+  }
+  const int64_t sR = op_cross(c).size();
   // doubles terms of the residual, transposed (antisymmetrisers give 2, 4)
   cn(2.0, V2, ten(c, I[6], "bmij"), 1.0, bten(c, g1, "am"));      // vooo
   cn(2.0, ten(c, I[1], "abej"), V2, 1.0, bten(c, g1, "ei"));      // vvvo
-  cn(4.0, V2, bten(c, s.wmbej, "mbej"), 0.0, bten(c, A->acc, "aeim"));
-  cn(4.0, bten(c, t2, "aeim"), V2, 0.0, bten(c, A->gw, "jbme", "mb|ej"));
+  if (A->blocked) {
+    const bool low = low_product(c, 3, 3);
+    op_product(c, A, 4.0, op_cross(c), A->vR, sR, op_same(c), s.wmbej, sR,
+               0.0, A->acc, VO, 1, nb, low);
+    op_product(c, A, 4.0, op_cross(c), A->vR, sR, op_cross(c), s.t2r, sR, 0.0,
+               A->gw, VO, 1, nb, low);
+  } else {
+    cn(4.0, V2, bten(c, s.wmbej, "embj", "mb|ej"), 0.0,
+       bten(c, A->acc, "aiem", "ae|im"));
+    cn(4.0, bten(c, t2, "aeim"), V2, 0.0, GW);
+  }
   // -t1 t1 <mb||ej> term: <mb||ej> = -vovo[b,m,e,j]
-  cn(1.0, bten(c, t1, "am"), V2, 0.0, bten(c, A->u, "mbij"));
-  cn(4.0, ten(c, I[4], "bmej"), bten(c, A->u, "mbij"), 1.0,
+  cn(1.0, bten(c, t1, "am"), V2, 0.0, bten(c, u, "mbij"));
+  cn(4.0, ten(c, I[4], "bmej"), bten(c, u, "mbij"), 1.0,
       bten(c, g1, "ei"));
-  cn(1.0, V2, bten(c, t1, "ei"), 0.0, bten(c, A->u2, "abej"));
-  cn(4.0, bten(c, A->u2, "abej"), ten(c, I[4], "bmej"), 1.0,
+  cn(1.0, V2, bten(c, t1, "ei"), 0.0, bten(c, u2, "abej"));
+  cn(4.0, bten(c, u2, "abej"), ten(c, I[4], "bmej"), 1.0,
       bten(c, g1, "am"));
   // ladders (tau adjoint), folded with the W_mnij / W_abef tau terms
-  cn(1.0, bten(c, s.wefab, "efab"), VT, 0.0, bten(c, A->gtau, "efij"));
-  cn(1.0, V2, bten(c, s.wmnij, "mnij"), 1.0, bten(c, A->gtau, "abmn"));
+  // (blocked: one pair of each antisymmetric couple, K twice)
+  if (A->blocked) {
+    op_product(c, A, 2.0, op_wefab(c), s.wefab, op_wefab(c).size(), op_vB(c),
+               A->vB, op_vB(c).size(), 0.0, A->gtau, OO, 1, nb,
+               low_product(c, 4, 2));
+    op_product(c, A, 2.0, op_vA(c), A->vA, op_vA(c).size(), op_wmnij(c),
+               s.wmnij, op_wmnij(c).size(), 1.0, A->gtau, OO, 1, nb,
+               low_product(c, 2, 4));
+  } else {
+    cn(1.0, bten(c, s.wefab, "efab"), V2, 0.0, bten(c, A->gtau, "efij"));
+    cn(1.0, V2, bten(c, s.wmnij, "mnij"), 1.0, bten(c, A->gtau, "abmn"));
+  }
   // t1 parts of W_mnij and W_abef through Zt, Zv
-  cn(1.0, bten(c, s.zt, "eabi", "ab|ie"), VT, 1.0, bten(c, g1, "ej"));
+  // (v2[a,b,i,j] = -v2[a,b,j,i]: i fastest in both)
+  cn(-1.0, bten(c, s.zt, "eabi", "ab|ie"), bten(c, v2, "abji"), 1.0,
+     bten(c, g1, "ej"));
   cn(-1.0, V2, bten(c, s.zv, "amij"), 1.0, bten(c, g1, "bm"));
   // Fock-type terms of the doubles
-  cn(-2.0, V2, bten(c, s.mj, "mj"), 1.0, bten(c, A->acc, "abim"));
-  cn(-2.0, bten(c, t2, "abim"), V2, 0.0, bten(c, gFmj, "mj"));
-  cn(2.0, V2, bten(c, s.be, "be"), 1.0, bten(c, A->acc, "aeij"));
+  cn(-2.0, V2, bten(c, s.mj, "mj"), 1.0, bten(c, A->acc, "aibm", "ab|im"));
+  // (t2[a,b,i,m] v2[a,b,i,j] with both last pairs turned: i fastest)
+  cn(-2.0, bten(c, t2, "abmi"), bten(c, v2, "abji"), 0.0,
+     bten(c, gFmj, "mj"));
+  cn(2.0, V2, bten(c, s.be, "be"), 1.0, bten(c, A->acc, "aiej", "ae|ij"));
   cn(2.0, bten(c, t2, "aeij"), V2, 0.0, bten(c, gFbe, "be"));
   // Fmj = Fmi + 1/2 t1.Fme ; Fbe = Fae - 1/2 t1.Fme
   copy(c, gFmi, gFmj, nb * (int64_t)O * O, 1.0);
@@ -1292,29 +1565,31 @@ void apply_points(ftcc_ctx *c, Adjoint *A, const double *t1, const double *t2,
   cn(-1.0, bten(c, t1, "am"), bten(c, v1, "ai"), 1.0, bten(c, gFmi, "mi"));
   cn(-1.0, bten(c, v1, "ai"), bten(c, s.mi, "mi"), 1.0, bten(c, g1, "am"));
   cn(1.0, bten(c, v1, "ai"), bten(c, s.me, "me"), 1.0,
-      bten(c, A->acc, "aeim"));
+      bten(c, A->acc, "aiem", "ae|im"));
   cn(1.0, bten(c, v1, "ai"), bten(c, t2, "aeim"), 1.0,
       bten(c, gFme, "me"));
   cn(-1.0, bten(c, v1, "ai"), ten(c, I[4], "anfi"), 1.0,
       bten(c, g1, "fn"));
   cn(0.5, bten(c, v1, "ai"), ten(c, I[2], "amef"), 1.0,
-      bten(c, A->acc, "efim"));
+      bten(c, A->acc, "eifm", "ef|im"));
   cn(0.5, bten(c, v1, "ai"), ten(c, I[7], "nmie"), 1.0,
-      bten(c, A->acc, "aemn"));
+      bten(c, A->acc, "amen", "ae|mn"));
   // Wmbej: t1.vovv, t1.ooov and the ring amplitude t2/2 + t1 t1
-  cn(-1.0, bten(c, A->gw, "jbme", "mb|ej"), ten(c, I[2], "bmef"), 1.0,
-      bten(c, g1, "fj"));
-  cn(1.0, bten(c, A->gw, "jbme", "mb|ej"), ten(c, I[7], "mnje"), 1.0,
-      bten(c, g1, "bn"));
-  cn(1.0, bten(c, A->gw, "jbme", "mb|ej"), ten(c, I[5], "mnef"), 0.0,
-      bten(c, A->q, "bjnf", "bf|jn"));
-  // acc[f,b,j,n] -= q[b,j,n,f] / 2
-  permute4(A->q, A->acc, V, O, O, V, (int64_t)O * O, (int64_t)O, 1,
-           (int64_t)V * O * O, -0.5, 1.0, nb, S2, S2, st);
-  cn(-1.0, bten(c, A->q, "bjnf", "bf|jn"), bten(c, t1, "bn"), 1.0,
-      bten(c, g1, "fj"));
-  cn(-1.0, bten(c, A->q, "bjnf", "bf|jn"), bten(c, t1, "fj"), 1.0,
-      bten(c, g1, "bn"));
+  // (vovv[b,m,e,f] and ooov[m,n,j,e] in the layouts with m fastest)
+  cn(-1.0, GW, ten(c, c->vovv_aefm, "befm", "bm|ef"), 1.0,
+     bten(c, g1, "fj"));
+  cn(1.0, GW, ten(c, c->ooov_iemn, "jenm", "mn|je"), 1.0, bten(c, g1, "bn"));
+  const Ten Q = bten(c, A->q, "bjfn", "bf|jn");
+  if (A->blocked) {
+    put_op(c, op_same(c), A->gw, VO, 1, S2, A->gwA, nb);
+    op_product(c, A, 1.0, op_same(c), A->gwA, sR, op_cross(c), A->ring, 0, 0.0,
+               A->q, VO, 1, nb, low_product(c, 3, 3));
+  } else {
+    cn(1.0, GW, ten(c, c->oovv_ring, "fnem", "mn|ef"), 0.0, Q);
+  }
+  // (acc[f,j,b,n] -= q[b,j,f,n] / 2 with the projection below)
+  cn(-1.0, Q, bten(c, t1, "bn"), 1.0, bten(c, g1, "fj"));
+  cn(-1.0, Q, bten(c, t1, "fj"), 1.0, bten(c, g1, "bn"));
   // Fmi, Fae, Fme
   cn(0.5, ten(c, c->F[1], "me"), bten(c, gFmi, "mi"), 1.0,
       bten(c, g1, "ei"));
@@ -1331,10 +1606,15 @@ void apply_points(ftcc_ctx *c, Adjoint *A, const double *t1, const double *t2,
   cn(1.0, bten(c, gFme, "me"), ten(c, I[5], "mnef"), 1.0,
       bten(c, g1, "fn"));
   // projection and the tau / taut chain rule into t1
-  hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(S2 * nb)), dim3(AT), 0,
-                     st, A->acc, A->gtau, A->gt, V, O, nb, A->tau, g2);
-  FTCC_CHECK_HIP(hipGetLastError());
-  cn(4.0, bten(c, A->tau, "abij"), bten(c, t1, "bj"), 1.0,
+  if (A->blocked) {
+    project_doubles(S, g2, A->acc, A->q, A->gtau, A->gt, V, O, c->v_count[0],
+                    c->o_count[0], nb, st);
+  } else {
+    hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(S2 * nb)), dim3(AT), 0,
+                       st, A->acc, A->q, A->gtau, A->gt, V, O, nb, S, g2);
+    FTCC_CHECK_HIP(hipGetLastError());
+  }
+  cn(4.0, bten(c, S, "abij"), bten(c, t1, "bj"), 1.0,
       bten(c, g1, "ai"));
 }
 
@@ -1449,21 +1729,24 @@ int ftcc_adjoint_begin(ftcc_ctx *c, const double *T1, const double *T2) {
     if (const char *env = getenv("FTCC_ADJOINT_CACHE_GB"))
       budget_gb = atof(env);
     if (const char *env = getenv("FTCC_WORKSPACE_GB")) work_gb = atof(env);
+    const bool blocked = c->spin && c->spin5 && c->pack;
     const int keep = (int)std::max<int64_t>(
         0, std::min<int64_t>(c->ng, (int64_t)(budget_gb * (1LL << 30)) /
-                                        slice_bytes(c)));
+                                        slice_bytes(c, blocked)));
     // grid points per application: as many as a quarter of the budget of
     // the residual workspace (released above) holds, one at least; they
     // share their launches (at n = 66 and eight grid points an application
     // took 3720 launches one point at a time, most of them too small to
     // fill the device)
-    const int64_t per = buffer_bytes(c) + (keep < c->ng ? slice_bytes(c) : 0);
+    const int64_t per = buffer_bytes(c, blocked) +
+                        (keep < c->ng ? slice_bytes(c, blocked) : 0);
     int nb = (int)std::max<int64_t>(
         1, std::min<int64_t>(c->ng, (int64_t)(work_gb * 0.25 * (1LL << 30)) /
                                         per));
     Adjoint *A = nullptr;
     for (;; nb = (nb + 1) / 2) {
       A = adjoint_ws(c);
+      A->blocked = blocked;
       try {
         alloc_apply_buffers(c, A, nb, keep < c->ng);
         alloc_slice(c, A, A->cache, keep);
@@ -1478,9 +1761,10 @@ int ftcc_adjoint_begin(ftcc_ctx *c, const double *T1, const double *T2) {
     A->T2 = T2;
     A->ng = c->ng;
     const int64_t VO = (int64_t)c->nv * c->no;
+    if (blocked) put_op(c, op_cross(c), c->oovv_ring, VO, 1, 0, A->ring, 1);
     for (int y = 0; y < keep; y += nb)
       prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
-                     at_point(c, A->cache, y), std::min(nb, keep - y));
+                     at_point(c, A, A->cache, y), std::min(nb, keep - y));
     FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
   });
 }
@@ -1502,11 +1786,16 @@ int ftcc_adjoint_apply(ftcc_ctx *c, const double *Lt1, const double *Lt2,
             FTCC_ESTATE);
     require(Lt1 && Lt2 && G1 && G2, "null pointer");
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
+    require(!A->blocked || (c->spin && c->spin5 && c->pack),
+            "the spin labels changed since ftcc_adjoint_begin", FTCC_ESTATE);
+    if (A->blocked && (low_product(c, 3, 3) || low_product(c, 4, 2) ||
+                       low_product(c, 2, 4)))
+      ensure_lowp(c, A);
     for (int y = 0; y < c->ng;) {
       const double *t1 = A->T1 + y * VO, *t2 = A->T2 + y * S2;
       const bool kept = y < A->cache.n;
       const int nb = std::min(A->nb, (kept ? A->cache.n : c->ng) - y);
-      const AdjSlice s = kept ? at_point(c, A->cache, y) : A->work;
+      const AdjSlice s = kept ? at_point(c, A, A->cache, y) : A->work;
       if (!kept) prepare_points(c, A, t1, t2, s, nb);
       apply_points(c, A, t1, t2, s, Lt1 + y * VO, Lt2 + y * S2, G1 + y * VO,
                    G2 + y * S2, nb);

@@ -138,6 +138,9 @@ void split_convert(const double *src, int64_t sr, int64_t sc, int64_t sb,
 void split_gather(const double *src, int64_t sr, int64_t sc, int64_t sb,
                   const int *rmap, int R, const int *cmap, int W,
                   const SplitMat &d, int nb, hipStream_t s);
+// the same of a plain R x W matrix (rows of stride sr, unit column stride)
+void split_rows(const double *src, int64_t sr, int64_t sb, int R, int W,
+                const SplitMat &d, int nb, hipStream_t s);
 // the same gather unsplit: dst[b*db + r*os + c], c < W, FP64 or rounded to
 // FP32 (f32)
 void gather_plain(const double *src, int64_t sr, int64_t sc, int64_t sb,
@@ -294,6 +297,14 @@ void r2_final(double *t2bar, const double *acc1, const double *acc2,
               const int *lab_o, const double *add, bool packed, int hv = -1,
               int ho = -1, bool flip = false, bool zero_forbidden = true,
               const int *jl = nullptr, int jc0 = 0, int jc1 = 0);
+// The doubles of the transposed residual (label runs: alpha below hv, ho;
+// adjoint.hip): S = gtau + P(gt) / 2 on the allowed doubles and
+// out = P(acc[a,i,b,j] - q[b,i,a,j] / 2) + P(gt) / 2 + S, zero elsewhere,
+// with P the projection onto antisymmetric tensors; gtau holds one pair of
+// each antisymmetric couple.
+void project_doubles(double *S, double *out, const double *acc,
+                     const double *q, const double *gtau, const double *gt,
+                     int nv, int no, int hv, int ho, int nb, hipStream_t s);
 // Spin-flip images of a ring tensor X[nb][nv][no][nv][no] (slice stride
 // sb) whose rows with a virtual alpha index are computed: every allowed
 // element with that index beta is copied from its flipped partner (alpha

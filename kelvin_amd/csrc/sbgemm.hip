@@ -546,6 +546,13 @@ void split_gather(const double *src, int64_t sr, int64_t sc, int64_t sb,
                 SplitOut{d.hi, d.lo}, nb, s);
 }
 
+void split_rows(const double *src, int64_t sr, int64_t sb, int R, int W,
+                const SplitMat &d, int nb, hipStream_t s) {
+  require(d.ld % 32 == 0 && W <= d.ld, "split operand leading dimension");
+  gather_launch(PlainSrc{src, sr, 1, sb}, false, nullptr, R, nullptr, W, W,
+                d.ld, d.bstride, SplitOut{d.hi, d.lo}, nb, s);
+}
+
 void amp_split_gather(int kind, const double *t1, const double *t2, int nv,
                       int no, const int *rmap, int R, const int *cmap, int W,
                       const SplitMat &d, int nb, hipStream_t s) {

@@ -507,22 +507,25 @@ __global__ __launch_bounds__(256) void r2_packed_kernel(
 // Bound: memory.  24 bytes move per allowed double of a flip step; per
 // eight-point launch at n = 114 5.05 ms with the row strips above.
 constexpr int R2T = 32;
-struct R2Tiles {
-  double *out;
-  const double *acc1, *acc2, *S1, *S2, *Z, *add;
+// The work of such a launch: (a,b) pairs and pairs of (i,j) tiles of the
+// three spin classes (alpha-alpha, mixed, beta-beta)
+struct PairTiles {
   int nv, no, hv, ho;          // sizes, alpha runs
   int flip;
-  // pairs and tile pairs of the three classes (alpha-alpha, mixed,
-  // beta-beta) and the tile edge and count of each occupied run
   int64_t pairs[3];
-  int tp[3], edge[2], nt[2];
+  int tp[3], edge[2], nt[2];   // tile pairs; edge and count of each run
   int64_t per_y;               // workgroups of one grid point
 };
-__global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
-  __shared__ double tile[R2T][R2T + 1];
+struct PairTile {
+  int64_t y;
+  int a, b, i0, j0, ni, nj;
+  bool mixed, off;             // mixed spins; i and j in different tiles
+};
+__device__ inline PairTile pair_tile(const PairTiles &p) {
+  PairTile w;
   int64_t bid = xcd_grouped(blockIdx.x, gridDim.x);
-  const int64_t y = bid / p.per_y;
-  bid -= y * p.per_y;
+  w.y = bid / p.per_y;
+  bid -= w.y * p.per_y;
   int cls = 0;
   while (bid >= p.pairs[cls] * p.tp[cls]) {
     bid -= p.pairs[cls] * p.tp[cls];
@@ -530,28 +533,42 @@ __global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
   }
   const int64_t q = bid / p.tp[cls];
   const int t = (int)(bid - q * p.tp[cls]);
-  const int nv = p.nv, no = p.no, hv = p.hv, ho = p.ho;
-  const bool mixed = cls == 1;
-  int a, b, I, J;   // the pair, the tiles
-  if (mixed && !p.flip) {
-    a = (int)(q / (nv - hv));
-    b = hv + (int)(q % (nv - hv));
+  w.mixed = cls == 1;
+  int I, J;
+  if (w.mixed && !p.flip) {
+    w.a = (int)(q / (p.nv - p.hv));
+    w.b = p.hv + (int)(q % (p.nv - p.hv));
   } else {
-    triangle(q, a, b);
-    if (mixed) b += hv;
-    if (cls == 2) a += hv, b += hv;
+    triangle(q, w.a, w.b);
+    if (w.mixed) w.b += p.hv;
+    if (cls == 2) w.a += p.hv, w.b += p.hv;
   }
   const int si = cls == 2, sj = cls != 0;   // spins of i and j
-  if (mixed) {
+  if (w.mixed) {
     I = t / p.nt[1];
     J = t % p.nt[1];
   } else {
     triangle(t, I, J);
   }
-  const int i0 = (si ? ho : 0) + I * p.edge[si];
-  const int j0 = (sj ? ho : 0) + J * p.edge[sj];
-  const int ni = min(p.edge[si], (si ? no : ho) - i0);
-  const int nj = min(p.edge[sj], (sj ? no : ho) - j0);
+  w.off = I != J;
+  w.i0 = (si ? p.ho : 0) + I * p.edge[si];
+  w.j0 = (sj ? p.ho : 0) + J * p.edge[sj];
+  w.ni = min(p.edge[si], (si ? p.no : p.ho) - w.i0);
+  w.nj = min(p.edge[sj], (sj ? p.no : p.ho) - w.j0);
+  return w;
+}
+struct R2Tiles {
+  double *out;
+  const double *acc1, *acc2, *S1, *S2, *Z, *add;
+  PairTiles g;
+};
+__global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
+  __shared__ double tile[R2T][R2T + 1];
+  const PairTile w = pair_tile(p.g);
+  const int nv = p.g.nv, no = p.g.no, hv = p.g.hv, ho = p.g.ho;
+  const int a = w.a, b = w.b, i0 = w.i0, j0 = w.j0, ni = w.ni, nj = w.nj;
+  const bool mixed = w.mixed, flip = p.g.flip;
+  const int64_t y = w.y;
   const int64_t per = (int64_t)nv * nv * no * no, oy = y * per;
   auto nat = [&](int r, int s, int k, int l) {
     return oy + (((int64_t)r * nv + s) * no + k) * no + l;
@@ -559,13 +576,13 @@ __global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
   auto fo = [&](int k) { return k < ho ? k + ho : k - ho; };
   auto fv = [&](int r) { return r < hv ? r + hv : r - hv; };
   auto zat = [&](int r, int k, int s, int l) {
-    if (p.flip && r >= hv) r = fv(r), k = fo(k), s = fv(s), l = fo(l);
+    if (flip && r >= hv) r = fv(r), k = fo(k), s = fv(s), l = fo(l);
     return p.Z[oy + (((int64_t)r * no + k) * nv + s) * no + l];
   };
   double *out = p.out;
   // the images of a flip step
-  const bool image = p.flip && (!mixed || a < b - hv);
-  const bool self = p.flip && mixed && a == b - hv;
+  const bool image = flip && (!mixed || a < b - hv);
+  const bool self = flip && mixed && a == b - hv;
   auto put = [&](int k, int l, double v) {   // R2[a,b,k,l] = v
     out[nat(a, b, k, l)] = v;
     out[nat(b, a, k, l)] = -v;
@@ -578,10 +595,10 @@ __global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
     for (int e = threadIdx.x; e < ni * nj; e += 256) {
       const int i = i0 + e / nj, j = j0 + e % nj;
       out[nat(a, a, i, j)] = 0.0;
-      if (I != J) out[nat(a, a, j, i)] = 0.0;
+      if (w.off) out[nat(a, a, j, i)] = 0.0;
       if (image) {
         out[nat(fv(a), fv(a), fo(i), fo(j))] = 0.0;
-        if (I != J) out[nat(fv(a), fv(a), fo(j), fo(i))] = 0.0;
+        if (w.off) out[nat(fv(a), fv(a), fo(j), fo(i))] = 0.0;
       }
     }
     return;
@@ -637,6 +654,91 @@ __global__ __launch_bounds__(256) void r2_tiles_kernel(R2Tiles p) {
     if (mixed ? !self || i <= j - ho : i < j) put(j, i, tile[r][c]);
   }
 }
+// Doubles of the transposed residual over the same tiles (label runs, no
+// flip): with P the projection onto antisymmetric tensors and
+// v[a,b,i,j] = acc[a,i,b,j] - q[b,i,a,j] / 2 (ring layouts),
+//   S = gtau + P(gt) / 2,   out = P(v) + P(gt) / 2 + S.
+// gtau holds the stored couples, gt every element; S and out are written
+// on the allowed doubles.  (Reading all four terms of each projection for
+// each element took 7.1 of 64 ms of a lambda iteration at n = 66.)
+struct ProjTiles {
+  double *S, *out;
+  const double *acc, *q, *gtau, *gt;
+  PairTiles g;
+};
+__global__ __launch_bounds__(256) void proj_tiles_kernel(ProjTiles p) {
+  __shared__ double tv[R2T][R2T + 1], tt[R2T][R2T + 1];
+  const PairTile w = pair_tile(p.g);
+  const int nv = p.g.nv, no = p.g.no;
+  const int a = w.a, b = w.b, i0 = w.i0, j0 = w.j0, ni = w.ni, nj = w.nj;
+  const int64_t oy = w.y * ((int64_t)nv * nv * no * no);
+  auto nat = [&](int r, int s, int k, int l) {
+    return oy + (((int64_t)r * nv + s) * no + k) * no + l;
+  };
+  auto put = [&](int k, int l, double s, double o) {
+    const int64_t n = nat(a, b, k, l), m = nat(b, a, k, l);
+    p.S[n] = s;
+    p.out[n] = o;
+    if (a != b) {
+      p.S[m] = -s;
+      p.out[m] = -o;
+    }
+  };
+  if (a == b) {
+    for (int e = threadIdx.x; e < ni * nj; e += 256) {
+      const int i = i0 + e / nj, j = j0 + e % nj;
+      put(i, j, 0.0, 0.0);
+      if (w.off) put(j, i, 0.0, 0.0);
+    }
+    return;
+  }
+  // v and gt at (k, l), antisymmetrised in (a,b)
+  auto vab = [&](int k, int l) {
+    const int64_t r = oy + (((int64_t)a * no + k) * nv + b) * no + l;
+    const int64_t s = oy + (((int64_t)b * no + k) * nv + a) * no + l;
+    return (p.acc[r] - 0.5 * p.q[s]) - (p.acc[s] - 0.5 * p.q[r]);
+  };
+  auto tab = [&](int k, int l) {
+    return p.gt[nat(a, b, k, l)] - p.gt[nat(b, a, k, l)];
+  };
+  for (int e = threadIdx.x; e < ni * nj; e += 256) {
+    const int r = e / ni, c = e - r * ni;
+    tv[r][c] = vab(j0 + r, i0 + c);
+    tt[r][c] = tab(j0 + r, i0 + c);
+  }
+  __syncthreads();
+  constexpr int NE = R2T * R2T / 256;
+  double xs[NE], xo[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = min((int)threadIdx.x + 256 * k, ni * nj - 1);
+    const int r = e / nj, c = e - r * nj;
+    const int i = i0 + r, j = j0 + c;
+    const double pv = 0.25 * (vab(i, j) - tv[c][r]);
+    const double pt = 0.25 * (tab(i, j) - tt[c][r]);
+    xs[k] = p.gtau[nat(a, b, i, j)] + 0.5 * pt;
+    xo[k] = pv + 0.5 * pt + xs[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = threadIdx.x + 256 * k;
+    if (e >= ni * nj) continue;
+    const int r = e / nj, c = e - r * nj;
+    const int i = i0 + r, j = j0 + c;
+    tv[c][r] = xs[k];
+    tt[c][r] = xo[k];
+    if (w.mixed || i < j) put(i, j, xs[k], xo[k]);
+    else if (i == j) put(i, i, 0.0, 0.0);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < ni * nj; e += 256) {
+    const int r = e / ni, c = e - r * ni;
+    const int j = j0 + r, i = i0 + c;
+    if (w.mixed || i < j) put(j, i, -tv[r][c], -tt[r][c]);
+  }
+}
+
 // zeros at the spin-forbidden doubles of nb slices (label runs: alpha below
 // hv, ho): row (a,b,i) allows the j of one spin, or none
 __global__ void r2_zero_kernel(double *out, int nv, int no, int hv, int ho,
@@ -844,6 +946,62 @@ void ring_assemble(double *Wr, const double *ovvo_ring, const double *Q1,
          ovvo_ring, Q1, Q2, nv, no, nb);
 }
 
+static PairTiles pair_tiles(int nv, int no, int hv, int ho, bool flip) {
+  PairTiles t;
+  t.nv = nv;
+  t.no = no;
+  t.hv = hv;
+  t.ho = ho;
+  t.flip = flip ? 1 : 0;
+  const int64_t bv = nv - hv;
+  for (int q = 0; q < 2; ++q) {
+    const int run = q ? no - ho : ho;
+    t.nt[q] = (run + R2T - 1) / R2T;
+    t.edge[q] = t.nt[q] ? (run + t.nt[q] - 1) / t.nt[q] : 0;
+    t.nt[q] = t.edge[q] ? (run + t.edge[q] - 1) / t.edge[q] : 0;
+  }
+  t.pairs[0] = (int64_t)hv * (hv + 1) / 2;
+  t.pairs[1] = flip ? t.pairs[0] : hv * bv;
+  t.pairs[2] = flip ? 0 : bv * (bv + 1) / 2;
+  t.tp[0] = t.nt[0] * (t.nt[0] + 1) / 2;
+  t.tp[1] = t.nt[0] * t.nt[1];
+  t.tp[2] = t.nt[1] * (t.nt[1] + 1) / 2;
+  t.per_y = 0;
+  for (int q = 0; q < 3; ++q) t.per_y += t.pairs[q] * t.tp[q];
+  return t;
+}
+
+static void zero_forbidden_doubles(double *x, int nv, int no, int hv, int ho,
+                                   int nb, hipStream_t s) {
+  const int64_t rows = (int64_t)nb * nv * nv * no;
+  if (rows == 0) return;
+  hipLaunchKernelGGL(r2_zero_kernel,
+                     dim3((unsigned)std::min<int64_t>((rows + 3) / 4, 1 << 16)),
+                     dim3(256), 0, s, x, nv, no, hv, ho, nb);
+  FTCC_CHECK_HIP(hipGetLastError());
+}
+
+void project_doubles(double *S, double *out, const double *acc,
+                     const double *q, const double *gtau, const double *gt,
+                     int nv, int no, int hv, int ho, int nb, hipStream_t s) {
+  ProjTiles t;
+  t.S = S;
+  t.out = out;
+  t.acc = acc;
+  t.q = q;
+  t.gtau = gtau;
+  t.gt = gt;
+  t.g = pair_tiles(nv, no, hv, ho, false);
+  const int64_t grid = t.g.per_y * nb;
+  require(grid < (1LL << 31), "projection grid too large");
+  if (grid > 0) {
+    hipLaunchKernelGGL(proj_tiles_kernel, dim3((unsigned)grid), dim3(256), 0,
+                       s, t);
+    FTCC_CHECK_HIP(hipGetLastError());
+  }
+  zero_forbidden_doubles(out, nv, no, hv, ho, nb, s);
+}
+
 void r2_final(double *t2bar, const double *acc1, const double *acc2,
               const double *S1, const double *S2, const double *Z, int nv,
               int no, int nb, hipStream_t s, const int *lab_v,
@@ -871,41 +1029,15 @@ void r2_final(double *t2bar, const double *acc1, const double *acc2,
     t.S2 = S2;
     t.Z = Z;
     t.add = add;
-    t.nv = nv;
-    t.no = no;
-    t.hv = hv;
-    t.ho = ho;
-    t.flip = flip ? 1 : 0;
-    const int64_t bv = nv - hv;
-    for (int q = 0; q < 2; ++q) {
-      const int run = q ? no - ho : ho;
-      t.nt[q] = (run + R2T - 1) / R2T;
-      t.edge[q] = t.nt[q] ? (run + t.nt[q] - 1) / t.nt[q] : 0;
-      t.nt[q] = t.edge[q] ? (run + t.edge[q] - 1) / t.edge[q] : 0;
-    }
-    t.pairs[0] = (int64_t)hv * (hv + 1) / 2;
-    t.pairs[1] = flip ? t.pairs[0] : hv * bv;
-    t.pairs[2] = flip ? 0 : bv * (bv + 1) / 2;
-    t.tp[0] = t.nt[0] * (t.nt[0] + 1) / 2;
-    t.tp[1] = t.nt[0] * t.nt[1];
-    t.tp[2] = t.nt[1] * (t.nt[1] + 1) / 2;
-    t.per_y = 0;
-    for (int q = 0; q < 3; ++q) t.per_y += t.pairs[q] * t.tp[q];
-    const int64_t grid = t.per_y * nb;
+    t.g = pair_tiles(nv, no, hv, ho, flip);
+    const int64_t grid = t.g.per_y * nb;
     require(grid < (1LL << 31), "r2 assembly grid too large");
     if (grid > 0) {
       hipLaunchKernelGGL(r2_tiles_kernel, dim3((unsigned)grid), dim3(256), 0,
                          s, t);
       FTCC_CHECK_HIP(hipGetLastError());
     }
-    if (zero_forbidden) {
-      const int64_t rows = (int64_t)nb * nv * nv * no;
-      hipLaunchKernelGGL(
-          r2_zero_kernel,
-          dim3((unsigned)std::min<int64_t>((rows + 3) / 4, 1 << 16)),
-          dim3(256), 0, s, t2bar, nv, no, hv, ho, nb);
-      FTCC_CHECK_HIP(hipGetLastError());
-    }
+    if (zero_forbidden) zero_forbidden_doubles(t2bar, nv, no, hv, ho, nb, s);
     return;
   }
   if (packed) {

@@ -441,6 +441,164 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmGroup grp) {
   }
 }
 
+// The same product for K of one index and at most KP (16 to 64): the O(n^5)
+// terms over one spin run of an orbital index, whose time is the passes over
+// their outputs.  In the kernel above a workgroup takes its slabs and then
+// its C one after another, each at the latency of memory: 20 us in all for
+// the Z -= t1.u term at n = 66, of which 1.3 us is the matrix cores'.  Here
+// everything a workgroup reads (both whole panels, C and the addend) is in
+// flight together before the first use.  RT x CT MFMA blocks per wave, WM x
+// WN waves: 16 RT rows where the rows are one orbital run (33 take 48, not
+// 64), likewise for columns, 64x64 otherwise.  MFMA step s takes the k from
+// 4s to 4s + 3, steps past K are left out; row stride KP + 2 doubles, so
+// that the 32 lanes of a read (16 rows, two k) hit distinct banks.
+template <int RT, int CT, int WM, int WN, int KP>
+__global__ __launch_bounds__(NT, KP > 48 ? 2 : 3) void gemm_short_kernel(
+    GemmGroup grp, int amf, int bnf) {
+  constexpr int TM = 16 * RT * WM, TN = 16 * CT * WN, LDK = KP + 2;
+  constexpr int EA = TM * KP / NT, EB = TN * KP / NT;
+  static_assert(WM * WN == 4 && TM + TN <= NT / 2, "four waves, 128 offsets");
+  extern __shared__ double sm[];   // A [TM][LDK], B [TN][LDK]
+  double *As = sm, *Bs = sm + TM * LDK;
+  __shared__ int64_t aoff[TM], boff[TN], crow[TM], ccol[TN], drow[TM],
+      dcol[TN];
+  const int64_t bid = xcd_block();
+  int item = 0;
+  for (int k = 1; k < grp.n; ++k)
+    if (bid >= grp.tile0[k]) item = k;
+  const GemmDev &p = grp.pr[item];
+  const BlockPos q = decode(p, (int)(bid - grp.tile0[item]));
+  const int t = threadIdx.x, m0 = q.tm * TM, n0 = q.tn * TN, K = p.K;
+  // offsets: of A and B by the first half of the threads, of C and D (after
+  // the scatter maps; -1: dropped or past the end) by the second
+  if (t < NT / 2) {
+    tile_offsets<TM, TN>(p, m0, n0, aoff, boff);
+  } else {
+    const int u = t - NT / 2;
+    if (u < TM) {
+      const int row = m0 + u;
+      const int rr = row < p.M ? (p.rmap ? p.rmap[row] : row) : -1;
+      const Lvl l =
+          map_level(levels(rr < 0 ? 0 : rr, p.M1, p.M2), p.mmap, p.mlvl);
+      crow[u] = rr < 0 ? -1 : at(l, p.sCm0, p.sCm1, p.sCm);
+      drow[u] = rr < 0 ? -1 : at(l, p.sDm0, p.sDm1, p.sDm);
+    } else if (u < TM + TN) {
+      const int col = n0 + u - TM;
+      const int cc = col < p.N ? (p.cmap ? p.cmap[col] : col) : -1;
+      const Lvl l =
+          map_level(levels(cc < 0 ? 0 : cc, p.N1, p.N2), p.nmap, p.nlvl);
+      ccol[u - TM] = cc < 0 ? -1 : at(l, p.sCn0, p.sCn1, p.sCn);
+      dcol[u - TM] = cc < 0 ? -1 : at(l, p.sDn0, p.sDn1, p.sDn);
+    }
+  }
+  __syncthreads();
+  // both panels: threads along the index that is contiguous in memory;
+  // loads past an edge read element 0 and count as zero
+  const double *A = p.A + q.b1 * p.sA1 + q.b2 * p.sA2;
+  const double *B = p.B + q.b1 * p.sB1 + q.b2 * p.sB2;
+  double ra[EA], rb[EB];
+#pragma unroll
+  for (int r = 0; r < EA; ++r) {
+    const int e = t + NT * r;
+    const int m = amf ? e % TM : e / KP, k = amf ? e / TM : e % KP;
+    const int64_t off = aoff[m];
+    const bool ok = off >= 0 && k < K;
+    const double v = A[ok ? off + (int64_t)k * p.sAk : (int64_t)0];
+    ra[r] = ok ? v : 0.0;
+  }
+#pragma unroll
+  for (int r = 0; r < EB; ++r) {
+    const int e = t + NT * r;
+    const int n = bnf ? e % TN : e / KP, k = bnf ? e / TN : e % KP;
+    const int64_t off = boff[n];
+    const bool ok = off >= 0 && k < K;
+    const double v = B[ok ? off + (int64_t)k * p.sBk : (int64_t)0];
+    rb[r] = ok ? v : 0.0;
+  }
+  // the old C and the addend of this lane's elements
+  const int lane = t & 63, wave = t >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+  const int li = lane & 15, lg = lane >> 4;
+  double *C = p.C + q.b1 * p.sC1 + q.b2 * p.sC2;
+  const double *D = p.D ? p.D + q.b1 * p.sD1 + q.b2 * p.sD2 : nullptr;
+  double cv[RT][CT][4];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) cv[rt][ct][v] = 0.0;
+  if (p.beta != 0.0) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int64_t r = crow[(wm * RT + rt) * 16 + lg + 4 * v];
+          const int64_t c = ccol[(wn * CT + ct) * 16 + li];
+          cv[rt][ct][v] = p.beta * C[r >= 0 && c >= 0 ? r + c : (int64_t)0];
+        }
+  }
+  if (D) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int x = (wm * RT + rt) * 16 + lg + 4 * v;
+          const int z = (wn * CT + ct) * 16 + li;
+          cv[rt][ct][v] +=
+              p.gamma *
+              D[crow[x] >= 0 && ccol[z] >= 0 ? drow[x] + dcol[z] : (int64_t)0];
+        }
+  }
+#pragma unroll
+  for (int r = 0; r < EA; ++r) {
+    const int e = t + NT * r;
+    As[(amf ? e % TM : e / KP) * LDK + (amf ? e / TM : e % KP)] = ra[r];
+  }
+#pragma unroll
+  for (int r = 0; r < EB; ++r) {
+    const int e = t + NT * r;
+    Bs[(bnf ? e % TN : e / KP) * LDK + (bnf ? e / TN : e % KP)] = rb[r];
+  }
+  __syncthreads();
+  d4_t acc[RT][CT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = d4_t{0, 0, 0, 0};
+#pragma unroll
+  for (int st = 0; st < KP / 4; ++st) {
+    if (4 * st >= K) break;
+    double a[RT], b[CT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      a[rt] = As[((wm * RT + rt) * 16 + li) * LDK + 4 * st + lg];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+      b[ct] = Bs[((wn * CT + ct) * 16 + li) * LDK + 4 * st + lg];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        acc[rt][ct] = Mma<double>::op(a[rt], b[ct], acc[rt][ct]);
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t r = crow[(wm * RT + rt) * 16 + lg + 4 * v];
+        const int64_t c = ccol[(wn * CT + ct) * 16 + li];
+        if (r >= 0 && c >= 0)
+          C[r + c] = p.alpha * acc[rt][ct][v] + cv[rt][ct][v];
+      }
+}
+
 // Epilogue of one element of a split product: C[b][m,n] = alpha * s + gamma
 // * D + beta * C through the scatter maps.
 __device__ inline void put_sum(const GemmDev &p, int64_t cb, int64_t mn,
@@ -641,6 +799,50 @@ void launch_layout(Tile tl, bool amf, bool bnf, bool kl, const GemmGroup &d,
   else launch_tile<T, 128, 128>(amf, bnf, kl, d, nb, s);
 }
 
+template <int RT, int CT, int WM, int WN, int KP>
+void launch_short(const GemmGroup &d, int64_t nb, bool amf, bool bnf,
+                  hipStream_t s) {
+  constexpr int LDS =
+      (16 * RT * WM + 16 * CT * WN) * (KP + 2) * (int)sizeof(double);
+  static std::once_flag attr;
+  set_max_lds_once(attr, (const void *)gemm_short_kernel<RT, CT, WM, WN, KP>,
+                   LDS);
+  hipLaunchKernelGGL((gemm_short_kernel<RT, CT, WM, WN, KP>),
+                     dim3((unsigned)nb), dim3(NT), LDS, s, d, amf ? 1 : 0,
+                     bnf ? 1 : 0);
+  FTCC_CHECK_HIP(hipGetLastError());
+}
+template <int RT, int CT, int WM, int WN>
+void launch_short_k(int K, const GemmGroup &d, int64_t nb, bool amf, bool bnf,
+                    hipStream_t s) {
+  if (K <= 32) launch_short<RT, CT, WM, WN, 32>(d, nb, amf, bnf, s);
+  else if (K <= 48) launch_short<RT, CT, WM, WN, 48>(d, nb, amf, bnf, s);
+  else launch_short<RT, CT, WM, WN, 64>(d, nb, amf, bnf, s);
+}
+// Most 64x64 tiles of a launch of the short-K kernel, some five for each of
+// its places on the chip.  Below it the latencies count, above it the passes
+// over memory, which its three workgroups a CU hide less well than the four
+// of the kernel above (n = 66: 162 -> 185 us at 28 000 tiles; the narrow
+// forms are faster at any count, their tiles hold no empty rows: 492 -> 468
+// us for the Z -= t1.u term).  n = 38, bf16x3 step: 1572 -> 1505 us.
+constexpr int64_t SHORT_TILES = 4096;
+// tile of the short-K kernel: as few 16-wide blocks as hold a side of at
+// most 64 (the other side 64), else 64x64
+Tile short_tile(int M, int N) {
+  if (M <= 64) return Tile{std::max(2, (M + 15) / 16) * 16, 64};
+  if (N <= 64) return Tile{64, std::max(2, (N + 15) / 16) * 16};
+  return Tile{64, 64};
+}
+void launch_short_tile(Tile t, bool rows, int K, const GemmGroup &d,
+                       int64_t nb, bool amf, bool bnf, hipStream_t s) {
+  if (rows && t.m == 32) launch_short_k<2, 1, 1, 4>(K, d, nb, amf, bnf, s);
+  else if (rows && t.m == 48)
+    launch_short_k<3, 1, 1, 4>(K, d, nb, amf, bnf, s);
+  else if (t.n == 32) launch_short_k<1, 2, 4, 1>(K, d, nb, amf, bnf, s);
+  else if (t.n == 48) launch_short_k<1, 3, 4, 1>(K, d, nb, amf, bnf, s);
+  else launch_short_k<2, 2, 2, 2>(K, d, nb, amf, bnf, s);
+}
+
 // operand layouts of the kernel instantiations
 bool a_mfast(const Gemm &g) { return g.sAm == 1 && g.sAk != 1; }
 bool b_nfast(const Gemm &g) { return g.sBn == 1 && g.sBk != 1; }
@@ -753,7 +955,25 @@ void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
           "the generic GEMM runs FP64 or FP32 (bf16x3 uses sbgemm)");
   require(n >= 1 && n <= GEMM_GROUP, "GEMM group size");
   const Plan pl = plan_of(g, cblk, n);
-  const Tile tl = pl.t;
+  // K of one index and at most 64, each output of one product: the short-K
+  // kernel (in FP64, the precision of those terms, and under the default
+  // launch plan)
+  int Mx = 0, Nx = 0, Kx = 0;
+  bool brief = precision == FTCC_PREC_FP64 && g[0].tile_policy == 0;
+  for (int k = 0; k < n; ++k) {
+    Mx = std::max(Mx, g[k].M);
+    Nx = std::max(Nx, g[k].N);
+    Kx = std::max(Kx, g[k].K);
+    brief = brief && g[k].K >= 1 && g[k].K <= 64 && g[k].K2 == 0;
+    for (int q = 0; q < k; ++q) brief = brief && cblk[q] != cblk[k];
+  }
+  const Tile st = short_tile(Mx, Nx);
+  if (brief && st.m * st.n == 64 * 64) {
+    int64_t tiles = 0;
+    for (int k = 0; k < n; ++k) tiles += tiles_of(g[k], st);
+    brief = tiles <= SHORT_TILES;
+  }
+  const Tile tl = brief ? st : pl.t;
   GemmGroup grp, red;
   grp.n = red.n = 0;
   int64_t blocks = 0, rblocks = 0, elems = 0;
@@ -811,6 +1031,10 @@ void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
     elems += per;
   }
   const bool amf = a_mfast(g[0]), bnf = b_nfast(g[0]), kl = g[0].K2 > 0;
+  if (brief) {
+    launch_short_tile(tl, Mx <= 64, Kx, grp, blocks, amf, bnf, s);
+    return;
+  }
   if (precision == FTCC_PREC_FP64)
     launch_layout<double>(tl, amf, bnf, kl, grp, blocks, s);
   else

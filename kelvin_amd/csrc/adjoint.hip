@@ -746,23 +746,23 @@ bool pack_block(ftcc_ctx *c, Gemm &g) {
   return true;
 }
 
-// dst_hi/dst_lo[r][k] (row length ld) = the split of src(r, k) for k < K,
-// zero for K <= k < ld (the split-bf16 GEMM reads whole 32-deep slabs)
-// (slice blockIdx.z: src + z * sb, R * ld further on in hi and lo)
+// dst[r][k] (row length ld) = the split of src(r, k) for k < K, zero for K
+// <= k < ld (the split-bf16 GEMM reads whole 32-deep slabs)
+// (slice blockIdx.z: src + z * sb, R * ld elements further on in dst)
 __global__ __launch_bounds__(256) void split_pack_kernel(
     const double *src, PackIdx rl, PackIdx kl, int R, int K, int ld,
-    __bf16 *hi, __bf16 *lo, int along_r, int64_t sb) {
+    __bf16 *dst, int along_r, int64_t sb) {
   __shared__ double tile[32][33];
   src += blockIdx.z * sb;
-  hi += (int64_t)blockIdx.z * R * ld;
-  lo += (int64_t)blockIdx.z * R * ld;
+  dst += 2 * (int64_t)blockIdx.z * R * ld;
   const int r0 = blockIdx.y * 32, k0 = blockIdx.x * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   auto put = [&](int r, int k, double v) {
     const float f = (float)v;
     const __bf16 h = (__bf16)f;
-    hi[(int64_t)r * ld + k] = h;
-    lo[(int64_t)r * ld + k] = (__bf16)(f - (float)h);
+    const int64_t o = SplitMat::place((int64_t)r * ld + k);
+    dst[o] = h;
+    dst[o + 16] = (__bf16)(f - (float)h);
   };
   if (along_r) {
     for (int i = ty; i < 32; i += 8) {
@@ -867,10 +867,8 @@ bool lowp_group(ftcc_ctx *c, const Gemm *const *gs, int n) {
     A.ld = B.ld = ld;
     A.bstride = na > 1 ? (int64_t)g.M * ld : 0;
     B.bstride = nbb > 1 ? (int64_t)g.N * ld : 0;
-    A.hi = (__bf16 *)p;
-    A.lo = A.hi + (int64_t)g.M * na * ld;
-    B.hi = A.lo + (int64_t)g.M * na * ld;
-    B.lo = B.hi + (int64_t)g.N * nbb * ld;
+    A.p = (__bf16 *)p;
+    B.p = A.p + 2 * (int64_t)g.M * na * ld;
     p += lowp_split_doubles(g);
     int *rmap = (int *)p, *cmap = rmap + g.M;
     p += lowp_table_doubles(g);
@@ -883,10 +881,10 @@ bool lowp_group(ftcc_ctx *c, const Gemm *const *gs, int n) {
     require(ga.y < 65536 && gb.y < 65536 && g.nb1 < 65536,
             "split pack: grid too large");
     hipLaunchKernelGGL(split_pack_kernel, ga, dim3(256), 0, c->stream, g.A,
-                       rA, kA, g.M, g.K, (int)ld, A.hi, A.lo,
+                       rA, kA, g.M, g.K, (int)ld, A.p,
                        g.sAm == 1 ? 1 : 0, g.sA1);
     hipLaunchKernelGGL(split_pack_kernel, gb, dim3(256), 0, c->stream, g.B,
-                       rB, kB, g.N, g.K, (int)ld, B.hi, B.lo,
+                       rB, kB, g.N, g.K, (int)ld, B.p,
                        g.sBn == 1 ? 1 : 0, g.sB1);
     hipLaunchKernelGGL(level_offsets_kernel, dim3((g.M + 255) / 256),
                        dim3(256), 0, c->stream, c_rows(g), g.M,
@@ -1316,10 +1314,8 @@ void op_product(ftcc_ctx *c, Adjoint *A, double alpha, const AdjOp &oa,
                   eb = (int64_t)ob.R->total * xb.ld;
     xa.bstride = sa ? ea : 0;
     xb.bstride = sb ? eb : 0;
-    xa.hi = (__bf16 *)A->lowp;
-    xa.lo = xa.hi + na * ea;
-    xb.hi = xa.lo + na * ea;
-    xb.lo = xb.hi + nbb * eb;
+    xa.p = (__bf16 *)A->lowp;
+    xb.p = xa.p + 2 * na * ea;
   }
   int np = 0;
   double flops = 0.0;
@@ -1333,13 +1329,8 @@ void op_product(ftcc_ctx *c, Adjoint *A, double alpha, const AdjOp &oa,
                   bo = (int64_t)n.start * lb + k.start;
     flops += 2.0 * r.count * (double)n.count * k.count * nb;
     if (low) {
-      SplitMat ua = xa, ub = xb;
-      const int64_t ua0 = (int64_t)r.start * xa.ld + k.start,
-                    ub0 = (int64_t)n.start * xb.ld + k.start;
-      ua.hi += ua0;
-      ua.lo += ua0;
-      ub.hi += ub0;
-      ub.lo += ub0;
+      const SplitMat ua = xa.from((int64_t)r.start * xa.ld + k.start),
+                     ub = xb.from((int64_t)n.start * xb.ld + k.start);
       split_rows(a + ao, la, sa, r.len, k.len, ua, na, c->stream);
       split_rows(b + bo, lb, sb, n.len, k.len, ub, nbb, c->stream);
       sp[np++] = SbProblem{r.len, n.len, k.len, ua, ub,

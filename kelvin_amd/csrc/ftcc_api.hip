@@ -773,10 +773,8 @@ void ensure_split_buffers(ftcc_ctx *c) {
     const int64_t rows = space_len(c, op_rows(c, id));
     m.bstride = OP_FIXED[id] ? 0 : rows * m.ld;
     const int64_t len = carve_len((split_elems(c, id) + 3) / 4 + 1);
-    m.hi = (__bf16 *)p;
-    p += len;
-    m.lo = (__bf16 *)p;
-    p += len;
+    m.p = (__bf16 *)p;
+    p += 2 * len;
   }
   c->arena_owner = 1;
   c->split_layout = op_layout(c);
@@ -870,11 +868,9 @@ void gather_blocks(ftcc_ctx *c, int id, SplitFn split, F64Fn f64,
     if (rows[q].len == 0 || ks[q].len == 0) continue;
     const int *rmap = R.d_map + rows[q].start, *kmap = K.d_map + ks[q].start;
     if (c->prec == FTCC_PREC_BF16X3) {
-      SplitMat m = split_of(c, id);
-      const int64_t off = (int64_t)rows[q].start * m.ld + ks[q].start;
-      m.hi += off;
-      m.lo += off;
-      split(rmap, rows[q].len, kmap, ks[q].len, m);
+      const SplitMat &m = split_of(c, id);
+      split(rmap, rows[q].len, kmap, ks[q].len,
+            m.from((int64_t)rows[q].start * m.ld + ks[q].start));
     } else {
       const int64_t ld = K.total;
       f64(rmap, rows[q].len, kmap, ks[q].len, ld,
@@ -1095,14 +1091,9 @@ void product(ftcc_ctx *c, const Gemm &g, int ia, int ib, int kind) {
       q.M = b.r.len;
       q.N = b.c.len;
       q.K = b.k.len;
-      q.A = split_of(c, ia);
-      q.B = split_of(c, ib);
-      const int64_t ao = (int64_t)b.r.start * q.A.ld + b.k.start;
-      const int64_t bo = (int64_t)b.c.start * q.B.ld + b.k.start;
-      q.A.hi += ao;
-      q.A.lo += ao;
-      q.B.hi += bo;
-      q.B.lo += bo;
+      const SplitMat &sa = split_of(c, ia), &sb = split_of(c, ib);
+      q.A = sa.from((int64_t)b.r.start * sa.ld + b.k.start);
+      q.B = sb.from((int64_t)b.c.start * sb.ld + b.k.start);
       q.rmap = R.d_map + b.r.start;
       q.cmap = Cs.d_map + b.c.start;
       flops += 2.0 * b.r.count * (double)b.c.count * b.k.count * g.nb1;
@@ -3099,10 +3090,8 @@ int ftcc_gemm(ftcc_ctx *c, int M, int N, int K, int batch, double alpha,
     const size_t bbytes = 2 * (size_t)Bs.bstride * batch;
     char *buf = nullptr;
     FTCC_CHECK_HIP(hipMalloc(&buf, 2 * (abytes + bbytes)));
-    As.hi = (__bf16 *)buf;
-    As.lo = (__bf16 *)(buf + abytes);
-    Bs.hi = (__bf16 *)(buf + 2 * abytes);
-    Bs.lo = (__bf16 *)(buf + 2 * abytes + bbytes);
+    As.p = (__bf16 *)buf;
+    Bs.p = (__bf16 *)(buf + 2 * abytes);
     split_convert(A, sAm, sAk, sAb, M, K, As, batch, c->stream);
     split_convert(B, sBn, sBk, sBb, N, K, Bs, batch, c->stream);
     timed(c, true, gemm_flops(g), [&] {

@@ -108,12 +108,19 @@ size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n);
 void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
                     Scratch &scr, hipStream_t s);
 
-// Split-BF16 operand: x = hi + lo, two bf16 arrays [rows][ld] (K contiguous,
-// zero-padded to ld), batch stride in elements.
+// Split-BF16 operand: x = hi + lo in bf16, [rows][ld] (K contiguous,
+// zero-padded to ld), batch stride in elements.  Sixteen hi and their
+// sixteen lo are stored together: 64 bytes are one row's share of a K step.
 struct SplitMat {
-  __bf16 *hi = nullptr, *lo = nullptr;
+  __bf16 *p = nullptr;
   int64_t ld = 0;
   int64_t bstride = 0;
+  // place of the hi of element o of the operand; its lo is 16 further on
+  __host__ __device__ static int64_t place(int64_t o) {
+    return o + (o & ~(int64_t)15);
+  }
+  // the operand that starts at element o, a multiple of 16
+  SplitMat from(int64_t o) const { return SplitMat{p + 2 * o, ld, bstride}; }
 };
 // Spin-class ordering of a pair space (x, y), x from a set with spin labels
 // lx, y from a set with labels ly: pairs are grouped by class

@@ -2,32 +2,38 @@
 // produce its operands.
 //
 // Operands are stored in HBM already split: x = hi + lo with hi = bf16(x),
-// lo = bf16(x - hi), as two bf16 arrays with K contiguous (A as [M][ld],
-// B transposed as [N][ld]); K is zero-padded to a multiple of 32 so the
-// inner loop needs no bounds checks along K.  C = alpha * A.B + beta * C is
-// accumulated in FP32 by v_mfma_f32_32x32x16_bf16 from lo*hi + hi*lo + hi*hi
-// (in that order for every accumulator) and written as FP64.
+// lo = bf16(x - hi), with K contiguous (A as [M][ld], B transposed as
+// [N][ld]), sixteen hi and their sixteen lo side by side; K is zero-padded to
+// a multiple of 32 so the inner loop needs no bounds checks along K.
+// C = alpha * A.B + beta * C is accumulated in FP32 by
+// v_mfma_f32_32x32x16_bf16 from lo*hi + hi*lo + hi*hi (in that order for
+// every accumulator) and written as FP64.
 //
 // Tiling: a 512-thread workgroup (8 wave64s, two per SIMD) owns a 256x256
 // tile of C, each wave a 128x64 quadrant (4x2 MFMA 32x32 blocks, 128 FP32
-// accumulators per lane).  K advances in slabs of 32 through two LDS stages
-// of 64 KB; each LDS row holds the row's 32 hi values and 32 lo values as
-// eight 16-byte chunks, chunk c stored at slot c ^ ((row >> 1) & 7) so that
-// the MFMA fragment reads (32 rows at one chunk per half-wave) hit distinct
-// banks.  Slabs go from HBM straight into LDS (global_load_lds_dwordx4: each
-// lane fetches the global chunk that belongs at its LDS slot, no register
-// staging), two slabs ahead of their use, into the stage the previous slab
-// has left.  Per slab a wave reads the fragments of the next 16-deep K step
-// while the MFMAs of the current one run (fragments double-buffered in
-// registers), so one barrier per slab is the only synchronisation; the loop
-// body has no branches (the loads past the last slab re-read the last one
-// into a stage that is never read).  Rows past M (N) read the last row:
-// their products land in accumulators that are never stored.  Workgroup
-// ids are remapped so that each XCD works on a compact group of tiles
-// (shared A/B panels stay in that XCD's L2).  Against staging the slabs
-// through registers with padded LDS rows (the earlier form of this
-// kernel), 8-13% shorter launches at n = 114 shapes with bit-identical
-// results; one wave per SIMD with 128x128 wave tiles was slower.
+// accumulators per lane).  K advances in steps of 16 through a ring of five
+// LDS stages of 32 KB, all of a CU's 160 KB; an LDS row holds the 64 bytes
+// of the row's step as four 16-byte chunks, chunk c at slot
+// c ^ ((row >> 2) & 3).  Steps go from HBM straight into LDS
+// (global_load_lds_dwordx4: each lane fetches the chunk that belongs at its
+// slot), up to five ahead of their use: an L2 miss takes longer than the
+// 1.5 steps that the earlier two stages of 32 K gave it.  One barrier per
+// step.  The fragment reads of the next step and the loads are issued
+// between the MFMAs of the current one (fragments double-buffered in
+// registers): issued together after the barrier, all eight waves queue for
+// the LDS and the address unit while the matrix cores idle, and left to the
+// compiler the reads are sunk to their uses.  Rows past M (N) read the last
+// row: their products land in accumulators that are never stored.  A last
+// tile of at most 192 rows or columns runs fewer MFMAs and comes after the
+// whole tiles in the launch, to fill its last round.
+//
+// Bound: the matrix cores, 66% busy on a CU at work; the rest is the start
+// and the stores of a tile, which one workgroup per CU does not overlap.
+// The five products of a residual, ms: n = 114 17.65 -> 15.84 (1.21 PFLOP/s
+// of bf16 MFMAs; a library bf16 product reaches 1.36 at its power limit),
+// n = 66 2.32 -> 2.15, against two stages of 32 K.  Tried: the same with
+// reads and loads in one burst after the barrier 18.6 at n = 114; one wave
+// per SIMD with 128x128 wave tiles was slower.
 #include "ftcc_internal.h"
 
 #include <algorithm>
@@ -39,12 +45,19 @@ typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef float f16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int u4_t __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 256, BN = 256, BK = 32;
+constexpr int BM = 256, BN = 256, BK = 16;
 constexpr int GROUP_M = 8;
-constexpr int ROWB = 128;              // bytes per LDS row: 32 hi, 32 lo
-constexpr int OPB = BM * ROWB;         // one operand of one stage: 32 KB
+constexpr int ROWB = 4 * BK;           // bytes per LDS row: 16 hi, 16 lo
+constexpr int OPB = BM * ROWB;         // one operand of one stage: 16 KB
 constexpr int STAGEB = 2 * OPB;        // A then B
-constexpr size_t LDS_BYTES = 2 * (size_t)STAGEB;
+constexpr int NST = 5;                 // stages of the ring
+constexpr int NL = 4;                  // loads of a wave per K step
+constexpr size_t LDS_BYTES = NST * (size_t)STAGEB;
+// operand of s_waitcnt: at most vm vector loads and lgkm LDS reads (15: any)
+// in flight
+constexpr int wait_for(int vm, int lgkm) {
+  return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8);
+}
 typedef __attribute__((address_space(3))) void lds_void;
 
 // One product of a grouped launch (the spin blocks of one O(n^6) product
@@ -52,16 +65,18 @@ typedef __attribute__((address_space(3))) void lds_void;
 constexpr int MAXP = 3;
 struct SbProb {
   int M, N, Kp, tilesM, tilesN;
-  int tile0;                 // first linear tile of this problem
-  const __bf16 *Ahi, *Alo;
+  int fullM, fullN;          // tiles before a short last row, column
+  int full0, edge0;          // its first whole tile and edge tile
+  const __bf16 *A;
   int64_t lda, sAb;
-  const __bf16 *Bhi, *Blo;
+  const __bf16 *B;
   int64_t ldb, sBb;
   const int *rmap, *cmap;    // output scatter (nullptr: identity; -1 drops)
 };
 struct SbDev {
   int nprob, nb;
   int group_m;               // tile rows per band of the launch order
+  int nfull;                 // whole tiles of the launch
   SbProb pr[MAXP];
   double *C;
   int64_t sCm, sCn, sCb;
@@ -69,155 +84,217 @@ struct SbDev {
 };
 
 // Workgroup -> (problem, batch, tile m, tile n).  Consecutive workgroup ids
-// go to different XCDs, so ids are first regrouped per XCD (each XCD then
-// takes a contiguous run of linear tiles); inside a problem, tiles run in
-// GROUP_M-row bands so that an XCD's concurrent tiles share A/B panels.
+// go to different XCDs, so each XCD first takes a contiguous run of the
+// launch's whole tiles, in GROUP_M-row bands of a problem so that concurrent
+// tiles share A/B panels, and then one of the edge tiles, which are shorter
+// (see tile_product) and fill the last round of the CUs.
 __device__ inline SbProb tile_of(const SbDev &p, int &bt, int &tm, int &tn) {
-  const int nblk = gridDim.x, b = blockIdx.x;
-  const int q = nblk / 8, r = nblk % 8, x = b % 8, j = b / 8;
-  const int lid = (x < r) ? x * (q + 1) + j : r * (q + 1) + (x - r) * q + j;
+  const int nblk = gridDim.x, b = blockIdx.x, x = b % 8, j = b / 8;
+  const int fq = p.nfull / 8, fr = p.nfull % 8;
+  const int fn = fq + (x < fr ? 1 : 0), f0 = x * fq + min(x, fr);
+  const int t0 = x * (nblk / 8) + min(x, nblk % 8);
+  const bool whole = j < fn;
+  const int lid = whole ? f0 + j : (t0 - f0) + (j - fn);
   SbProb pr = p.pr[0];
-  if (p.nprob > 1 && lid >= p.pr[1].tile0) pr = p.pr[1];
-  if (p.nprob > 2 && lid >= p.pr[2].tile0) pr = p.pr[2];
-  const int local = lid - pr.tile0;
-  const int per = pr.tilesM * pr.tilesN;
+  for (int k = 1; k < MAXP; ++k)
+    if (p.nprob > k && lid >= (whole ? p.pr[k].full0 : p.pr[k].edge0))
+      pr = p.pr[k];
+  const int local = lid - (whole ? pr.full0 : pr.edge0);
+  const int fper = pr.fullM * pr.fullN;
+  const int per = whole ? fper : pr.tilesM * pr.tilesN - fper;
   bt = local / per;
   const int t = local % per;
-  const int span = p.group_m * pr.tilesN;
-  const int first_m = (t / span) * p.group_m;
-  const int gsz = min(pr.tilesM - first_m, p.group_m);
-  tm = first_m + (t % span) % gsz;
-  tn = (t % span) / gsz;
+  if (whole) {
+    const int span = p.group_m * pr.fullN;
+    const int first_m = (t / span) * p.group_m;
+    const int gsz = min(pr.fullM - first_m, p.group_m);
+    tm = first_m + (t % span) % gsz;
+    tn = (t % span) / gsz;
+  } else {
+    const int strip = (pr.tilesM - pr.fullM) * pr.tilesN;
+    tm = t < strip ? pr.fullM : t - strip;
+    tn = t < strip ? t : pr.fullN;
+  }
   return pr;
 }
 
-// LDS slot of chunk c (0-3 hi, 4-7 lo, eight bf16 each) of row r
-__device__ inline int lds_slot(int row, int c) { return c ^ ((row >> 1) & 7); }
+// LDS slot of chunk c (0, 1: hi, 2, 3: lo, eight bf16 each) of row r: the
+// sixteen lanes that read one chunk of sixteen rows hit distinct banks
+__device__ inline int lds_slot(int row, int c) { return c ^ ((row >> 2) & 3); }
 
-// One wave's share of a slab of one operand: rows [32w, 32w + 32) of the
-// tile, four loads of eight rows x eight chunks; the lane that lands at
-// slot (lane & 7) of row r fetches the chunk stored there.
-__device__ inline void load_slab(const __bf16 *hi, const __bf16 *lo,
-                                 int64_t ld, int row0, int rows, int k0,
-                                 char *lds_op, int wave, int lane) {
-  const int r8 = lane >> 3, slot = lane & 7;
+// One wave's share of a K step of one operand: rows [32w, 32w + 32) of the
+// tile in two loads of sixteen rows x four chunks; the lane that lands at
+// slot (lane & 3) of row r fetches the chunk stored there.  off: its byte
+// offsets from the tile's first row, the same in every step.
+struct Rows {
+  const __bf16 *p;   // first row of the tile
+  unsigned off[2];
+};
+__device__ inline Rows tile_rows(const __bf16 *p, int64_t ld, int row0,
+                                 int rows, int wave, int lane) {
+  Rows r;
+  r.p = p + 2 * row0 * ld;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int rowl = wave * 32 + j * 8 + r8;
-    const int c = lds_slot(rowl, slot);   // the slot map is an involution
-    int g = row0 + rowl;
-    g = g < rows ? g : rows - 1;
-    const __bf16 *src = (c < 4 ? hi : lo) + (int64_t)g * ld + k0 + 8 * (c & 3);
-    __builtin_amdgcn_global_load_lds(
-        (const void *)src, (lds_void *)(lds_op + (wave * 32 + j * 8) * ROWB),
-        16, 0, 0);
+  for (int j = 0; j < 2; ++j) {
+    const int rowl = wave * 32 + j * 16 + (lane >> 2);
+    const int c = lds_slot(rowl, lane & 3);   // the map is an involution
+    r.off[j] = (unsigned)min(rowl, rows - 1 - row0) * (unsigned)(4 * ld) +
+               16u * c;
   }
+  return r;
+}
+// load q (0, 1: A, 2, 3: B) of K step t into a stage
+__device__ inline void load_part(const Rows &A, const Rows &B, int q, int t,
+                                 char *stage, int wave) {
+  const Rows &r = q < 2 ? A : B;
+  __builtin_amdgcn_global_load_lds(
+      (const void *)((const char *)(r.p + (int64_t)t * (2 * BK)) +
+                     r.off[q & 1]),
+      (lds_void *)(stage + (q >> 1) * OPB +
+                   (wave * 32 + (q & 1) * 16) * ROWB),
+      16, 0, 0);
 }
 
 __device__ inline bf8_t lds_frag(const char *lds_op, int row, int c) {
   return *(const bf8_t *)(lds_op + row * ROWB + (lds_slot(row, c) << 4));
 }
 
-// the A (4 row blocks) and B (2 column blocks) fragments, hi and lo, of one
-// 16-deep K step (chunk c: 0 or 2, plus the lane's half)
-struct Frag {
-  bf8_t ah[4], al[4], bh[2], bl[2];
+// blocks of 32 in n rows of a last tile
+__host__ __device__ inline int edge_blocks(int n) { return (n + 31) / 32; }
+// tiles before a last one of at most EDGE blocks
+constexpr int EDGE = 6;
+inline int full_tiles(int n, int tile) {
+  const int r = n % tile;
+  return r > 0 && edge_blocks(r) <= EDGE ? n / tile : (n + tile - 1) / tile;
+}
+
+// the fragments, hi and lo, of RT row and CT column blocks of one 16-deep K
+// step (chunk c: 0 or 2, plus the lane's half)
+template <int RT, int CT> struct Frag {
+  bf8_t ah[RT], al[RT], bh[CT], bl[CT];
 };
-__device__ inline void read_frag(Frag &f, const char *As, const char *Bs,
-                                 int wm, int wn, int li, int c) {
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
-    const int row = wm * 128 + rt * 32 + li;
-    f.ah[rt] = lds_frag(As, row, c);
-    f.al[rt] = lds_frag(As, row, c + 4);
-  }
-#pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const int row = wn * 64 + ct * 32 + li;
-    f.bh[ct] = lds_frag(Bs, row, c);
-    f.bl[ct] = lds_frag(Bs, row, c + 4);
+// fragment q of the 2 (RT + CT) of a step
+template <int RT, int CT>
+__device__ inline void read_frag(Frag<RT, CT> &f, int q, const char *stage,
+                                 int wm, int wn, int li, int lg) {
+  const int h = q & 1, b = q >> 1;
+  if (b < CT) {
+    const bf8_t v =
+        lds_frag(stage + OPB, (wn * CT + b) * 32 + li, 2 * h + lg);
+    if (h) f.bl[b] = v;
+    else f.bh[b] = v;
+  } else {
+    const bf8_t v =
+        lds_frag(stage, (wm * RT + b - CT) * 32 + li, 2 * h + lg);
+    if (h) f.al[b - CT] = v;
+    else f.ah[b - CT] = v;
   }
 }
-// lo*hi + hi*lo + hi*hi, in that order for every accumulator
-__device__ inline void mfma_step(f16_t (&acc)[4][2], const Frag &f) {
+// The MFMAs of one K step, lo*hi + hi*lo + hi*hi in that order for every
+// accumulator, two accumulators in turn; other(q), q < n, is what is issued
+// between them.
+template <int RT, int CT, typename Other>
+__device__ __forceinline__ void mfma_step(f16_t (&acc)[RT][CT],
+                                          const Frag<RT, CT> &f, int n,
+                                          Other other) {
+  constexpr int NA = RT * CT, G = (NA + 1) / 2;
+  int done = 0;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+  for (int g = 0; g < G; ++g) {
+    const int upto = ((g + 1) * n + G - 1) / G;
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          f.al[rt], f.bh[ct], acc[rt][ct], 0, 0, 0);
-      acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          f.ah[rt], f.bl[ct], acc[rt][ct], 0, 0, 0);
-      acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          f.ah[rt], f.bh[ct], acc[rt][ct], 0, 0, 0);
-    }
+    for (int q = done; q < upto; ++q) other(q);
+    done = upto;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int a = 2 * g; a < (2 * g + 2 < NA ? 2 * g + 2 : NA); ++a) {
+        const int rt = a / CT, ct = a % CT;
+        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            t == 0 ? f.al[rt] : f.ah[rt], t == 1 ? f.bl[ct] : f.bh[ct],
+            acc[rt][ct], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
-__global__ __launch_bounds__(512, 1) void sbgemm_kernel(SbDev p) {
-  extern __shared__ char lds[];   // [2 stages][A | B][256 rows][128 B]
-  // the tile's output rows and columns after the scatter maps (-1: past
-  // the end or dropped), read once here, alongside the first slab's loads
-  __shared__ int emap[BM + BN];
-  int bt, tm, tn;
-  const SbProb pr = tile_of(p, bt, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  {
-    const int t = threadIdx.x;   // 512 threads: 256 rows, then 256 columns
-    if (t < BM) {
-      const int row = m0 + t;
-      emap[t] = row < pr.M ? (pr.rmap ? pr.rmap[row] : row) : -1;
-    } else {
-      const int col = n0 + t - BM;
-      emap[t] = col < pr.N ? (pr.cmap ? pr.cmap[col] : col) : -1;
-    }
-  }
-  const __bf16 *Ahi = pr.Ahi + bt * pr.sAb, *Alo = pr.Alo + bt * pr.sAb;
-  const __bf16 *Bhi = pr.Bhi + bt * pr.sBb, *Blo = pr.Blo + bt * pr.sBb;
+// One tile of C, RT x CT blocks of 32x32 a wave at block row wm RT, column
+// wn CT: 4x2 blocks on 2x4 waves for a whole tile; for a last tile with nr
+// (nc) <= 6 blocks of rows (columns), nr x 1 blocks on 1x8 waves (1 x nc on
+// 8x1), whose matrix work is nr / 8 of a whole tile's.
+template <int RT, int CT>
+__device__ __forceinline__ void tile_product(const SbDev &p, const SbProb &pr,
+                                             int bt, int m0, int n0, char *lds,
+                                             int wm, int wn) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 2, wn = wave & 3;
   const int li = lane & 31, lg = lane >> 5;
-  const int nslab = pr.Kp / BK;
+  // the tile's output rows and columns after the scatter maps (-1: past
+  // the end or dropped), one of them a thread, read here ahead of the loop
+  const int t = threadIdx.x, e = t < BM ? m0 + t : n0 + t - BM;
+  const int *map = t < BM ? pr.rmap : pr.cmap;
+  const int mapped = e < (t < BM ? pr.M : pr.N) ? (map ? map[e] : e) : -1;
+  const int nstep = pr.Kp / BK;   // even
+  const Rows A =
+      tile_rows(pr.A + 2 * bt * pr.sAb, pr.lda, m0, pr.M, wave, lane);
+  const Rows B =
+      tile_rows(pr.B + 2 * bt * pr.sBb, pr.ldb, n0, pr.N, wave, lane);
 
-  f16_t acc[4][2];
+  f16_t acc[RT][CT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
   // an empty K (a spin class without pairs) only writes beta * C
-  Frag f0, f1;
-  if (nslab > 0) {
-    load_slab(Ahi, Alo, pr.lda, m0, pr.M, 0, lds, wave, lane);
-    load_slab(Bhi, Blo, pr.ldb, n0, pr.N, 0, lds + OPB, wave, lane);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const int k1 = (nslab > 1 ? 1 : 0) * BK;
-    load_slab(Ahi, Alo, pr.lda, m0, pr.M, k1, lds + STAGEB, wave, lane);
-    load_slab(Bhi, Blo, pr.ldb, n0, pr.N, k1, lds + STAGEB + OPB, wave,
-              lane);
-    read_frag(f0, lds, lds + OPB, wm, wn, li, lg);
+  constexpr int NF = 2 * (RT + CT);
+  Frag<RT, CT> f0, f1;
+  if (nstep > 0) {
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+#pragma unroll
+      for (int q = 0; q < NL; ++q)
+        load_part(A, B, q, min(s, nstep - 1), lds + s * STAGEB, wave);
+    __builtin_amdgcn_s_waitcnt(wait_for((NST - 1) * NL, 15));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < NF; ++q) read_frag(f0, q, lds, wm, wn, li, lg);
   }
-  for (int s = 0; s < nslab; ++s) {
-    char *cur = lds + (s & 1) * STAGEB, *nxt = lds + ((s + 1) & 1) * STAGEB;
-    // second K step of slab s from LDS while the first one's MFMAs run
-    read_frag(f1, cur, cur + OPB, wm, wn, li, 2 + lg);
-    mfma_step(acc, f0);
-    // slab s + 1 has landed (every wave's loads) and every wave is done
-    // with stage s: slab s + 2 goes there, slab s + 1's first K step is read
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const int k2 = min(s + 2, nslab - 1) * BK;
-    load_slab(Ahi, Alo, pr.lda, m0, pr.M, k2, cur, wave, lane);
-    load_slab(Bhi, Blo, pr.ldb, n0, pr.N, k2, cur + OPB, wave, lane);
-    read_frag(f0, nxt, nxt + OPB, wm, wn, li, lg);
-    mfma_step(acc, f1);
+  char *cur = lds;
+  // step s: its fragments are in f, those of step s + 1 go to g
+  auto step = [&](int s, const Frag<RT, CT> &f, Frag<RT, CT> &g) {
+    // step s + 1 has landed (every wave's loads) and every wave holds its
+    // fragments of step s, whose stage takes step s + NST.  Past the last
+    // step that one is loaded again, into stages that are not read any
+    // more, which keeps the count of loads in flight constant.
+    __builtin_amdgcn_s_waitcnt(wait_for((NST - 2) * NL, 0));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    char *const nxt =
+        cur == lds + (NST - 1) * STAGEB ? lds : cur + STAGEB;
+    const int ahead = min(s + NST, nstep - 1);
+    mfma_step(acc, f, NF + NL, [&](int q) {
+      // reads and loads in turn, then what is left of either (NF >= NL)
+      if (q < 2 * NL && (q & 1)) load_part(A, B, q >> 1, ahead, cur, wave);
+      else read_frag(g, q < 2 * NL ? q >> 1 : q - NL, nxt, wm, wn, li, lg);
+    });
+    cur = nxt;
+  };
+  for (int s = 0; s < nstep; s += 2) {
+    step(s, f0, f1);
+    step(s + 1, f1, f0);
   }
-  // no load may still be writing LDS when the workgroup ends
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  // an empty K passed no barrier since the scatter maps went to LDS
-  if (nslab == 0) __syncthreads();
+  // no load may still be writing LDS when the maps take its place
+  __builtin_amdgcn_s_waitcnt(wait_for(0, 0));
+  __syncthreads();
+  int *const emap = (int *)lds;   // rows, then columns
+  emap[t] = mapped;
+  __syncthreads();
 
   // lane holds column li, rows 8*(v/4) + 4*lg + v%4 of each 32x32 block.
   // Per block, the reads of C (beta != 0) are unconditional (a dropped
@@ -226,16 +303,16 @@ __global__ __launch_bounds__(512, 1) void sbgemm_kernel(SbDev p) {
   // for all outstanding memory operations before each store.
   double *C = p.C + bt * p.sCb;
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int cc = emap[BM + wn * 64 + ct * 32 + li];
+    for (int ct = 0; ct < CT; ++ct) {
+      const int cc = emap[BM + (wn * CT + ct) * 32 + li];
       int64_t off[16];
       double res[16];
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int rr =
-            emap[wm * 128 + rt * 32 + 8 * (v >> 2) + 4 * lg + (v & 3)];
+            emap[(wm * RT + rt) * 32 + 8 * (v >> 2) + 4 * lg + (v & 3)];
         off[v] = (rr >= 0 && cc >= 0)
                      ? (int64_t)rr * p.sCm + (int64_t)cc * p.sCn
                      : (int64_t)-1;
@@ -252,6 +329,30 @@ __global__ __launch_bounds__(512, 1) void sbgemm_kernel(SbDev p) {
     }
 }
 
+__global__ __launch_bounds__(512, 1) void sbgemm_kernel(SbDev p) {
+  extern __shared__ char lds[];   // [NST stages][A | B][256 rows][64 B]
+  int bt, tm, tn;
+  const SbProb pr = tile_of(p, bt, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int wave = threadIdx.x >> 6;
+  const int nr = tm < pr.fullM ? 8 : edge_blocks(pr.M - m0);
+  const int nc = tn < pr.fullN ? 8 : edge_blocks(pr.N - n0);
+#define FTCC_EDGE(NB)                                                      \
+  if (nr <= nc) tile_product<NB, 1>(p, pr, bt, m0, n0, lds, 0, wave); \
+  else tile_product<1, NB>(p, pr, bt, m0, n0, lds, wave, 0)
+  switch (min(nr, nc)) {
+    case 1: FTCC_EDGE(1); break;
+    case 2: FTCC_EDGE(2); break;
+    case 3: FTCC_EDGE(3); break;
+    case 4: FTCC_EDGE(4); break;
+    case 5:
+    case 6: FTCC_EDGE(6); break;
+    default:
+      tile_product<4, 2>(p, pr, bt, m0, n0, lds, wave >> 2, wave & 3);
+  }
+#undef FTCC_EDGE
+}
+
 __device__ inline void split1(double v, __bf16 &hi, __bf16 &lo) {
   const float f = (float)v;
   hi = (__bf16)f;
@@ -262,12 +363,13 @@ __device__ inline void split1(double v, __bf16 &hi, __bf16 &lo) {
 // plain FP64 or FP32 (the spin-blocked operands of those modes).
 // store4 writes four consecutive elements (o a multiple of 4).
 struct SplitOut {
-  __bf16 *hi, *lo;
+  __bf16 *p;
   __device__ void operator()(int64_t o, double v) const {
     __bf16 h, l;
     split1(v, h, l);
-    hi[o] = h;
-    lo[o] = l;
+    const int64_t q = SplitMat::place(o);
+    p[q] = h;
+    p[q + 16] = l;
   }
   __device__ void store4(int64_t o, const double v[4]) const {
     typedef __bf16 b4_t __attribute__((ext_vector_type(4)));
@@ -279,8 +381,9 @@ struct SplitOut {
       h[k] = hk;
       l[k] = lk;
     }
-    *(b4_t *)(hi + o) = h;
-    *(b4_t *)(lo + o) = l;
+    const int64_t q = SplitMat::place(o);
+    *(b4_t *)(p + q) = h;
+    *(b4_t *)(p + q + 16) = l;
   }
 };
 struct F32Out {
@@ -533,7 +636,7 @@ void split_convert(const double *src, int64_t sr, int64_t sc, int64_t sb,
   bool ar;
   const PlainSrc src_ = plain(src, sr, sc, sb, ar);
   gather_launch(src_, ar, nullptr, R, nullptr, C, (int)d.ld, d.ld, d.bstride,
-                SplitOut{d.hi, d.lo}, nb, s);
+                SplitOut{d.p}, nb, s);
 }
 
 void split_gather(const double *src, int64_t sr, int64_t sc, int64_t sb,
@@ -543,14 +646,14 @@ void split_gather(const double *src, int64_t sr, int64_t sc, int64_t sb,
   bool ar;
   const PlainSrc src_ = plain(src, sr, sc, sb, ar);
   gather_launch(src_, ar, rmap, R, cmap, W, W, d.ld, d.bstride,
-                SplitOut{d.hi, d.lo}, nb, s);
+                SplitOut{d.p}, nb, s);
 }
 
 void split_rows(const double *src, int64_t sr, int64_t sb, int R, int W,
                 const SplitMat &d, int nb, hipStream_t s) {
   require(d.ld % 32 == 0 && W <= d.ld, "split operand leading dimension");
   gather_launch(PlainSrc{src, sr, 1, sb}, false, nullptr, R, nullptr, W, W,
-                d.ld, d.bstride, SplitOut{d.hi, d.lo}, nb, s);
+                d.ld, d.bstride, SplitOut{d.p}, nb, s);
 }
 
 void amp_split_gather(int kind, const double *t1, const double *t2, int nv,
@@ -559,7 +662,7 @@ void amp_split_gather(int kind, const double *t1, const double *t2, int nv,
   require(d.ld % 32 == 0 && W <= d.ld, "split operand leading dimension");
   require(rmap && cmap, "amplitude operands are gathered through pair maps");
   amp_launch(kind, t1, t2, nv, no, rmap, R, cmap, W, d.ld, d.bstride,
-             SplitOut{d.hi, d.lo}, nb, s);
+             SplitOut{d.p}, nb, s);
 }
 
 void amp_gather_plain(int kind, const double *t1, const double *t2, int nv,
@@ -585,7 +688,7 @@ void flip_ring_gather(const double *src, int nv, int no, int hv, int ho,
   if (d) {
     require(d->ld % 32 == 0 && W <= d->ld, "split operand leading dimension");
     gather_launch(src_, true, rmap, R, cmap, W, W, d->ld, d->bstride,
-                  SplitOut{d->hi, d->lo}, nb, s);
+                  SplitOut{d->p}, nb, s);
   } else if (f32) {
     gather_launch(src_, true, rmap, R, cmap, W, W, os, db,
                   F32Out{(float *)dst}, nb, s);
@@ -630,34 +733,40 @@ void sbgemm_grouped(int nprob, const SbProblem *prob, int nb, double alpha,
   p.alpha = alpha;
   p.beta = beta;
   p.nprob = 0;
-  int64_t tiles = 0;
+  int64_t tiles = 0, whole = 0;
   for (int k = 0; k < nprob; ++k) {
     const SbProblem &q = prob[k];
     if (q.M <= 0 || q.N <= 0) continue;
     require(q.A.ld % 32 == 0 && q.B.ld % 32 == 0 && q.A.ld >= q.K &&
                 q.B.ld >= q.K,
             "split operands need K padded to 32");
+    // a tile's rows lie within 32-bit byte offsets
+    require(std::max(q.A.ld, q.B.ld) < (1LL << 32) / (4 * BM),
+            "split operand rows too long");
     SbProb &d = p.pr[p.nprob++];
     d.M = q.M;
     d.N = q.N;
-    d.Kp = (int)((q.K + BK - 1) / BK * BK);
+    d.Kp = (int)((q.K + 31) / 32 * 32);
     d.tilesM = (q.M + BM - 1) / BM;
     d.tilesN = (q.N + BN - 1) / BN;
-    d.tile0 = (int)tiles;
-    d.Ahi = q.A.hi;
-    d.Alo = q.A.lo;
+    d.fullM = full_tiles(q.M, BM);
+    d.fullN = full_tiles(q.N, BN);
+    d.full0 = (int)whole;
+    d.edge0 = (int)(tiles - whole);
+    d.A = q.A.p;
     d.lda = q.A.ld;
     d.sAb = q.A.bstride;
-    d.Bhi = q.B.hi;
-    d.Blo = q.B.lo;
+    d.B = q.B.p;
     d.ldb = q.B.ld;
     d.sBb = q.B.bstride;
     d.rmap = q.rmap;
     d.cmap = q.cmap;
     tiles += (int64_t)d.tilesM * d.tilesN * nb;
+    whole += (int64_t)d.fullM * d.fullN * nb;
   }
   if (p.nprob == 0 || nb <= 0) return;
   require(tiles < (1LL << 31), "too many GEMM tiles");
+  p.nfull = (int)whole;
   hipLaunchKernelGGL(sbgemm_kernel, dim3((unsigned)tiles), dim3(512),
                      LDS_BYTES, s, p);
   FTCC_CHECK_HIP(hipGetLastError());

@@ -1,0 +1,190 @@
+"""The GPU kernels at the sizes where their tilings can go wrong: edges of
+tiles and K steps, remainders, empty and uneven spin runs, small scratch.
+Against exact integers, FP64 matrix products on the host or the oracle."""
+import numpy
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+from oracle import ftcc as oracle  # noqa: E402
+from oracle import fock_space as fs  # noqa: E402
+from test_gpu_adjoint import antisym  # noqa: E402
+from test_gpu_parity import _spin_problem, dev, rel, to_np  # noqa: E402
+
+U64, U32 = 2.0 ** -53, 2.0 ** -24
+
+
+def _gemm(M, N, K, batch, layout, precision, alpha, beta, ints=0):
+    """C = alpha A B + beta C on the engine, the host's, |A| |B| and |C|."""
+    from kelvin_amd.engine import FTEngine
+    d = dev()
+    g = torch.Generator().manual_seed(M + 3 * N + 7 * K)
+
+    def draw(*s):
+        if ints:
+            return torch.randint(-ints, ints + 1, s, generator=g).double()
+        return torch.randn(*s, generator=g, dtype=torch.float64)
+
+    def lay(x, c):
+        x = x.to(d)
+        return x if c == 'n' else \
+            x.transpose(1, 2).contiguous().transpose(1, 2)
+    A, B, C = draw(batch, M, K), draw(batch, K, N), draw(batch, M, N)
+    Cd = C.to(d)
+    eng = FTEngine(2, 2, 1)
+    eng.gemm(lay(A, layout[0]), lay(B, layout[1]), Cd, alpha=alpha, beta=beta,
+             precision=precision)
+    out = to_np(Cd)
+    eng.close()
+    return (out, (alpha * (A @ B) + beta * C).numpy(),
+            (abs(alpha) * (A.abs() @ B.abs())).numpy(),
+            (abs(beta) * C.abs()).numpy())
+
+
+@pytest.mark.parametrize("layout", ["nn", "tn", "nt", "tt"])
+@pytest.mark.parametrize("M,N,K,batch", [
+    (1, 1, 1, 1), (15, 130, 4, 2), (31, 65, 32, 1), (33, 64, 33, 3),
+    (48, 129, 48, 1), (49, 63, 49, 2), (64, 31, 64, 1), (130, 16, 31, 2),
+    (127, 33, 47, 1), (66, 48, 64, 3), (200, 50, 1, 1), (65, 66, 63, 2),
+    (65, 66, 65, 2),                     # K one past the short-K kernel
+    (4096, 4100, 5, 1),                  # more 64x64 tiles than it takes
+    (20, 30, 3000, 1), (300, 260, 900, 2)])   # split K, many and few sums
+def test_gemm_tile_and_k_edges(M, N, K, batch, layout):
+    """Rounding of two FP64 sums of K products: 2 (K + 3) u |A| |B|."""
+    out, ref, ab, c = _gemm(M, N, K, batch, layout, "fp64", 0.75, -0.5)
+    assert (numpy.abs(out - ref) <= 2 * (K + 3) * U64 * (ab + c)).all()
+
+
+@pytest.mark.parametrize("M,N,K,batch", [
+    (1, 1, 1, 1), (32, 257, 16, 2), (33, 256, 17, 1), (64, 300, 32, 1),
+    (65, 512, 33, 3), (96, 96, 64, 1), (128, 289, 80, 1), (129, 257, 96, 1),
+    (160, 300, 95, 1), (192, 520, 160, 2), (193, 257, 48, 1),
+    (224, 224, 64, 1), (225, 300, 31, 1), (255, 511, 128, 1),
+    (256, 256, 161, 1), (257, 64, 64, 1), (300, 128, 40, 1),
+    (520, 192, 200, 9), (300, 32, 96, 2), (511, 416, 64, 9)])
+def test_split_product_tile_and_k_edges(M, N, K, batch):
+    """Integers below 2^8 are exact in bf16 and their sums in FP32: equal to
+    the last bit.  Normal numbers: the split leaves 2^-18 of an operand, the
+    dropped lo*lo 2^-18 of a product, FP32 sums of 3 K terms."""
+    out, ref, ab, c = _gemm(M, N, K, batch, "nt", "bf16x3", 1.0, 0.0, ints=9)
+    assert numpy.array_equal(out, ref)
+    out, ref, ab, c = _gemm(M, N, K, batch, "nt", "bf16x3", 0.5, 2.0)
+    bound = (3 * 2.0 ** -17 + 3 * (K + 1) * U32) * ab + 4 * U64 * c
+    assert (numpy.abs(out - ref) <= bound).all()
+
+
+# (alpha, beta) occupied and virtual orbitals: (v, o) classes of 31, 32, 33,
+# 64, 65 pairs, runs of 31 to 33 orbitals, unequal and empty runs
+_RUNS = [((1, 2), (31, 16)), ((3, 4), (11, 8)), ((5, 5), (13, 13)),
+         ((2, 8), (4, 8)), ((3, 0), (5, 4)), ((33, 2), (2, 3)),
+         ((2, 1), (33, 32)), ((4, 4), (8, 8)), ((1, 1), (1, 1))]
+
+
+def _run_problem(runs, ng, rng):
+    (oa, ob), (va, vb) = runs
+    lab = numpy.repeat([0, 1, 0, 1], [oa, ob, va, vb])
+    return (oa + ob, va + vb,
+            _spin_problem(oa + ob, va + vb, ng, lab, rng))
+
+
+def _run_engine(F, I, no, nv, ng, lo, lv, prec):
+    from kelvin_amd.engine import FTEngine
+    from kelvin_amd.ov_blocks import one_e_blocks, two_e_blocks
+    eng = FTEngine(no, nv, ng, precision=prec)
+    eng.set_blocks(one_e_blocks(**{k: F[k] for k in ('oo', 'ov', 'vo', 'vv')}),
+                   two_e_blocks(**{k: I[k] for k in I}))
+    eng.set_denominators(numpy.ones((nv, no)), numpy.ones((nv, nv, no, no)))
+    eng.set_grid(numpy.zeros(ng), numpy.zeros((ng, ng)))
+    eng.set_spin(lo, lv)
+    return eng
+
+
+@pytest.mark.parametrize("workspace", [None, "0.0001"])
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5),
+                                      ("bf16x3", 2e-4)])
+@pytest.mark.parametrize("runs", _RUNS)
+def test_blocked_residual_at_class_and_run_edges(prec, tol, runs, workspace,
+                                                 monkeypatch):
+    """Products, grouped contractions and the doubles assembly of the
+    spin-blocked residual, all grid points at once and one at a time; the
+    tolerances of the residual tests of these precisions."""
+    d = dev()
+    ng = 2
+    if workspace:
+        monkeypatch.setenv("FTCC_WORKSPACE_GB", workspace)
+    rng = numpy.random.default_rng(sum(map(sum, runs)))
+    no, nv, (F, I, t1, t2, lo, lv) = _run_problem(runs, ng, rng)
+    ref1, ref2 = oracle.residual_tbar(F, I, t1, t2)
+    eng = _run_engine(F, I, no, nv, ng, lo, lv, prec)
+    T1, T2 = (torch.as_tensor(x, device=d) for x in (t1, t2))
+    b1, b2 = torch.empty_like(T1), torch.empty_like(T2)
+    eng.residual(T1, T2, b1, b2)
+    assert rel(to_np(b1), ref1) < tol
+    assert rel(to_np(b2), ref2) < tol
+    eng.close()
+
+
+@pytest.mark.parametrize("workspace,cache", [(None, "64"), (None, "0"),
+                                             ("0.0001", "0")])
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("bf16x3", 2e-4)])
+@pytest.mark.parametrize("runs", [r for r in _RUNS if sum(r[1]) < 60])
+def test_blocked_adjoint_at_class_and_run_edges(prec, tol, runs, workspace,
+                                                cache, monkeypatch):
+    """The transposed residual over spin blocks against the oracle's, with
+    the intermediates kept and rebuilt, and with little scratch; tolerances
+    as for the residual."""
+    d = dev()
+    ng = 3
+    monkeypatch.setenv("FTCC_ADJOINT_CACHE_GB", cache)
+    if workspace:
+        monkeypatch.setenv("FTCC_WORKSPACE_GB", workspace)
+    rng = numpy.random.default_rng(7 + sum(map(sum, runs)))
+    no, nv, (F, I, t1, t2, lo, lv) = _run_problem(runs, ng, rng)
+    v1 = rng.normal(size=t1.shape) * (lv[:, None] == lo[None, :])
+    v2 = antisym(rng.normal(size=t2.shape)) * (
+        (lv[:, None, None, None] + lv[None, :, None, None]) ==
+        (lo[None, None, :, None] + lo[None, None, None, :]))
+    ref1, ref2 = numpy.empty_like(v1), numpy.empty_like(v2)
+    for y in range(ng):
+        g1, g2 = oracle.stanton_rhs_transpose(F, I, t1[y], t2[y], v1[y],
+                                              v2[y])
+        ref1[y], ref2[y] = g1, oracle.antisymmetrize(g2)
+    eng = _run_engine(F, I, no, nv, ng, lo, lv, "fp64")
+    T1, T2, V1, V2 = (torch.as_tensor(x, device=d) for x in (t1, t2, v1, v2))
+    eng.adjoint_begin(T1, T2)
+    eng.adjoint_precision(prec)
+    G1, G2 = eng.empty_amplitudes()
+    eng.adjoint_apply(V1, V2, G1, G2)
+    eng.adjoint_end()
+    assert rel(to_np(G1), ref1) < tol
+    assert rel(to_np(G2), ref2) < tol
+    eng.close()
+
+
+@pytest.mark.parametrize("quad", ['lin', 'mid', 'L'])
+@pytest.mark.parametrize("ng", [3, 5, 7, 9, 17, 33])
+def test_adjoint_recurrence_lengths(quad, ng):
+    """Batches of eight slices, remainders and grids shorter than one:
+    sums of ng terms of at most unit weight, a few ng u."""
+    from kelvin_amd import quadrature
+    from kelvin_amd.engine import FTEngine
+    d = dev()
+    rng = numpy.random.default_rng(ng)
+    n = 3
+    ti, g, G = quadrature.ft_quad(ng, 4.0, quad)
+    en = numpy.sort(rng.uniform(-1, 1, n))
+    eng = FTEngine(n, n, ng)
+    eri = fs.random_antisym(n, rng, hermitian=True) * 0.1
+    eng.set_system(en, numpy.diag(en), eri, 4.0, 0.0)
+    eng.set_grid(ti, G)
+    l1, l2 = rng.normal(size=(ng, n, n)), rng.normal(size=(ng, n, n, n, n))
+    L1, L2 = (torch.as_tensor(x, device=d) for x in (l1, l2))
+    O1, O2 = eng.empty_amplitudes()
+    eng.integrate_adjoint(L1, L2, O1, O2)
+    assert rel(to_np(O1), oracle.int_adjoint(
+        ng, l1, ti, oracle.D1(en, en), G)) < 1e-13
+    assert rel(to_np(O2), oracle.int_adjoint(
+        ng, l2, ti, oracle.D2(en, en), G)) < 1e-13
+    eng.close()

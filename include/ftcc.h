@@ -408,8 +408,9 @@ int ftcc_workspace_bytes(const ftcc_ctx *ctx, int64_t *bytes);
 int ftcc_profile_enable(ftcc_ctx *ctx, int on);
 int ftcc_profile_read(ftcc_ctx *ctx, int64_t *launches, double *ms,
                       double *flops);
-/* Launch plan of the generic GEMMs (the O(n^5) terms, and everything in the
- * FP64/FP32 modes): tile_policy 0 takes 64x64 tiles, 1 128x128 unless a
+/* Launch plan of the generic GEMMs (the O(n^5) terms, and the products of
+ * dense FP64/FP32 contexts): tile_policy 0 takes 64x64 tiles (in FP64 as few
+ * 16s as hold a side for K of at most 64), 1 128x128 unless a
  * dimension is at most 64, 2 the best of 128x64, 64x128 and 64x64 by their
  * estimated time; K is split at
  * most until a launch has split_target workgroups (default 1024).

@@ -31,8 +31,11 @@
 //   Zv[a,m,i,j] = sum_ef vovv[a,m,e,f] tau[e,f,i,j]
 // and the Fock-type Fme, Fae, Fmi, Fbe, Fmj.  One application costs five
 // O(n^6) products per grid point (two ladders, three rings) and O(n^5)
-// contractions, all in FP64 on the GEMM engine (dense operands; every
-// index is addressed through its own stride).
+// contractions, for as many grid points a launch as the workspace holds.
+// On a spin-blocked system the products run on packed copies of their
+// operands (AdjOp: FP64, or split-bf16 where chosen) and the doubles are
+// projected over pair tiles; otherwise everything goes through the GEMM
+// engine, every index addressed through its own stride.
 #include "ftcc_ctx.h"
 
 #include <math.h>

@@ -323,7 +323,7 @@ int ftcc_density1(ftcc_ctx *ctx, const double *T1_dev, const double *T2_dev,
                   double *pba_dev, double *pji_dev, double *pai_dev);
 /* Contraction precision of the large blocks of ftcc_adjoint_apply:
  * FTCC_PREC_FP64 (default) or FTCC_PREC_BF16X3 (the low-precision phase of
- * a refined lambda iteration).  Unbatched blocks of at least
+ * a refined lambda iteration).  Products and blocks of at least
  * FTCC_ADJOINT_LOWP_MIN_GFLOP GFLOP (environment, read by this call; default
  * 10) run split-bf16.  No counterpart in the reference (its lambda equations
  * are FP64 numpy). */

@@ -1193,6 +1193,9 @@ bool try_spin(ftcc_ctx *c, const std::vector<int> &lo,
     bad += c->host_red[2];
   }
   if (bad != 0.0) return false;
+  // the operand copies were carved for the class lengths of the old spaces
+  // and gathered through their maps: the next residual lays them out anew
+  c->arena_owner = 0;
   for (PairSpace *ps :
        {&c->ps_vv, &c->ps_oo, &c->ps_vo, &c->ps_vvp, &c->ps_oop}) {
     dfree(c, ps->d_map);

@@ -126,6 +126,45 @@ def test_blocked_residual_at_class_and_run_edges(prec, tol, runs, workspace,
     eng.close()
 
 
+# compositions of one (no, nv): the classes of the second need longer operand
+# slots than those of the first, a longer operand set in the third pair
+_RELABEL = [[((3, 4), (11, 8)), ((3, 4), (10, 9))],
+            [((7, 7), (12, 12)), ((8, 6), (11, 13)), ((7, 7), (12, 12))],
+            [((2, 2), (4, 4)), ((4, 0), (3, 5)), ((1, 3), (6, 2))]]
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5),
+                                      ("bf16x3", 2e-4)])
+@pytest.mark.parametrize("runs", _RELABEL)
+def test_one_engine_takes_other_compositions(prec, tol, runs):
+    """One engine given system after system of the same (no, nv) that divide
+    differently between the spins, then other labels of the same blocks (the
+    spins exchanged: no runs any more); the tolerances of the residual."""
+    from kelvin_amd.ov_blocks import one_e_blocks, two_e_blocks
+    d = dev()
+    ng = 2
+    rng = numpy.random.default_rng(sum(map(sum, runs[0])))
+    eng = None
+    for k, r in enumerate(runs):
+        no, nv, (F, I, t1, t2, lo, lv) = _run_problem(r, ng, rng)
+        if eng is None:
+            eng = _run_engine(F, I, no, nv, ng, lo, lv, prec)
+        else:
+            eng.set_blocks(
+                one_e_blocks(**{k: F[k] for k in ('oo', 'ov', 'vo', 'vv')}),
+                two_e_blocks(**{k: I[k] for k in I}))
+            eng.set_spin(lo, lv)
+        ref1, ref2 = oracle.residual_tbar(F, I, t1, t2)
+        T1, T2 = (torch.as_tensor(x, device=d) for x in (t1, t2))
+        for labels in ((lo, lv), (1 - lo, 1 - lv)):
+            eng.set_spin(*labels)
+            b1, b2 = torch.empty_like(T1), torch.empty_like(T2)
+            eng.residual(T1, T2, b1, b2)
+            assert rel(to_np(b1), ref1) < tol, (k, labels)
+            assert rel(to_np(b2), ref2) < tol, (k, labels)
+    eng.close()
+
+
 @pytest.mark.parametrize("workspace,cache", [(None, "64"), (None, "0"),
                                              ("0.0001", "0")])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("bf16x3", 2e-4)])

@@ -298,7 +298,8 @@ int ftcc_defect(ftcc_ctx *ctx, const double *T1_dev, const double *T2_dev,
  * them unchanged until ftcc_adjoint_end) and build the amplitude-only
  * intermediates of J^T for as many grid points as FTCC_ADJOINT_CACHE_GB
  * (default 64) holds; the others rebuild theirs at each application.
- * Releases the residual workspace of the forward iteration. */
+ * Releases the residual workspace of the forward iteration.  After other
+ * spin labels the next application builds them again. */
 int ftcc_adjoint_begin(ftcc_ctx *ctx, const double *T1_dev,
                        const double *T2_dev);
 /* Grid points whose intermediates are kept. */

@@ -1124,8 +1124,10 @@ struct Adjoint {
   const double *T1 = nullptr, *T2 = nullptr;   // the checkpoint
   int ng = 0;
   int nb = 1;                    // grid points of one application's launches
-  // the O(n^6) products run on spin-blocked, packed operand copies
+  // the O(n^6) products run on spin-blocked, packed operand copies, sized by
+  // the pair spaces of this building of theirs (ftcc_ctx::spaces_built)
   bool blocked = false;
+  int64_t spaces = 0;
   AdjSlice cache;                // grid points [0, cache.n) are kept
   AdjSlice work;                 // intermediates of uncached grid points
   // buffers of nb grid points (prepare_points and apply_points each say
@@ -1763,6 +1765,61 @@ __global__ void density1_out_kernel(const double *s_vo, const double *s_vv,
   }
 }
 
+// the products of J^T run on blocked operand copies under the present labels
+bool adjoint_blocked(const ftcc_ctx *c) {
+  return c->spin && c->spin5 && c->pack;
+}
+
+// The workspace of J^T at the amplitudes T1, T2 and its kept intermediates
+void build_adjoint(ftcc_ctx *c, const double *T1, const double *T2) {
+  drop_graph(c);
+  // the forward residual's operand buffers are rebuilt when next needed
+  free_workspace(c);
+  adjoint_release(c);
+  double budget_gb = 64.0, work_gb = 120.0;
+  if (const char *env = getenv("FTCC_ADJOINT_CACHE_GB"))
+    budget_gb = atof(env);
+  if (const char *env = getenv("FTCC_WORKSPACE_GB")) work_gb = atof(env);
+  const bool blocked = adjoint_blocked(c);
+  const int keep = (int)std::max<int64_t>(
+      0, std::min<int64_t>(c->ng, (int64_t)(budget_gb * (1LL << 30)) /
+                                      slice_bytes(c, blocked)));
+  // grid points per application: as many as a quarter of the budget of
+  // the residual workspace (released above) holds, one at least; they
+  // share their launches (at n = 66 and eight grid points an application
+  // took 3720 launches one point at a time, most of them too small to
+  // fill the device)
+  const int64_t per = buffer_bytes(c, blocked) +
+                      (keep < c->ng ? slice_bytes(c, blocked) : 0);
+  int nb = (int)std::max<int64_t>(
+      1, std::min<int64_t>(c->ng, (int64_t)(work_gb * 0.25 * (1LL << 30)) /
+                                      per));
+  Adjoint *A = nullptr;
+  for (;; nb = (nb + 1) / 2) {
+    A = adjoint_ws(c);
+    A->blocked = blocked;
+    A->spaces = c->spaces_built;
+    try {
+      alloc_apply_buffers(c, A, nb, keep < c->ng);
+      alloc_slice(c, A, A->cache, keep);
+      break;
+    } catch (const Error &e) {
+      if (e.code != FTCC_ENOMEM || nb == 1) throw;
+      adjoint_release(c);   // less memory free than that: fewer at a time
+      (void)hipGetLastError();
+    }
+  }
+  A->T1 = T1;
+  A->T2 = T2;
+  A->ng = c->ng;
+  const int64_t VO = (int64_t)c->nv * c->no;
+  if (blocked) put_op(c, op_cross(c), c->oovv_ring, VO, 1, 0, A->ring, 1);
+  for (int y = 0; y < keep; y += nb)
+    prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
+                   at_point(c, A, A->cache, y), std::min(nb, keep - y));
+  FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
+}
+
 }  // namespace
 
 extern "C" {
@@ -1771,51 +1828,7 @@ int ftcc_adjoint_begin(ftcc_ctx *c, const double *T1, const double *T2) {
   return guarded(c, [&] {
     check_ready(c);
     require(T1 && T2, "null amplitude pointer");
-    drop_graph(c);
-    // the forward residual's operand buffers are rebuilt when next needed
-    free_workspace(c);
-    adjoint_release(c);
-    double budget_gb = 64.0, work_gb = 120.0;
-    if (const char *env = getenv("FTCC_ADJOINT_CACHE_GB"))
-      budget_gb = atof(env);
-    if (const char *env = getenv("FTCC_WORKSPACE_GB")) work_gb = atof(env);
-    const bool blocked = c->spin && c->spin5 && c->pack;
-    const int keep = (int)std::max<int64_t>(
-        0, std::min<int64_t>(c->ng, (int64_t)(budget_gb * (1LL << 30)) /
-                                        slice_bytes(c, blocked)));
-    // grid points per application: as many as a quarter of the budget of
-    // the residual workspace (released above) holds, one at least; they
-    // share their launches (at n = 66 and eight grid points an application
-    // took 3720 launches one point at a time, most of them too small to
-    // fill the device)
-    const int64_t per = buffer_bytes(c, blocked) +
-                        (keep < c->ng ? slice_bytes(c, blocked) : 0);
-    int nb = (int)std::max<int64_t>(
-        1, std::min<int64_t>(c->ng, (int64_t)(work_gb * 0.25 * (1LL << 30)) /
-                                        per));
-    Adjoint *A = nullptr;
-    for (;; nb = (nb + 1) / 2) {
-      A = adjoint_ws(c);
-      A->blocked = blocked;
-      try {
-        alloc_apply_buffers(c, A, nb, keep < c->ng);
-        alloc_slice(c, A, A->cache, keep);
-        break;
-      } catch (const Error &e) {
-        if (e.code != FTCC_ENOMEM || nb == 1) throw;
-        adjoint_release(c);   // less memory free than that: fewer at a time
-        (void)hipGetLastError();
-      }
-    }
-    A->T1 = T1;
-    A->T2 = T2;
-    A->ng = c->ng;
-    const int64_t VO = (int64_t)c->nv * c->no;
-    if (blocked) put_op(c, op_cross(c), c->oovv_ring, VO, 1, 0, A->ring, 1);
-    for (int y = 0; y < keep; y += nb)
-      prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
-                     at_point(c, A, A->cache, y), std::min(nb, keep - y));
-    FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
+    build_adjoint(c, T1, T2);
   });
 }
 
@@ -1836,8 +1849,11 @@ int ftcc_adjoint_apply(ftcc_ctx *c, const double *Lt1, const double *Lt2,
             FTCC_ESTATE);
     require(Lt1 && Lt2 && G1 && G2, "null pointer");
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
-    require(!A->blocked || (c->spin && c->spin5 && c->pack),
-            "the spin labels changed since ftcc_adjoint_begin", FTCC_ESTATE);
+    // other spin labels since: the operand copies have other sizes now
+    if (A->blocked && (!adjoint_blocked(c) || A->spaces != c->spaces_built)) {
+      build_adjoint(c, A->T1, A->T2);
+      A = c->adj;
+    }
     if (A->blocked && (low_product(c, 3, 3) || low_product(c, 4, 2) ||
                        low_product(c, 2, 4)))
       ensure_lowp(c, A);

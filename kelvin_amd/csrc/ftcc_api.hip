@@ -1196,6 +1196,7 @@ bool try_spin(ftcc_ctx *c, const std::vector<int> &lo,
   // the operand copies were carved for the class lengths of the old spaces
   // and gathered through their maps: the next residual lays them out anew
   c->arena_owner = 0;
+  ++c->spaces_built;   // (and so does the adjoint)
   for (PairSpace *ps :
        {&c->ps_vv, &c->ps_oo, &c->ps_vo, &c->ps_vvp, &c->ps_oop}) {
     dfree(c, ps->d_map);

@@ -168,6 +168,7 @@ struct ftcc_ctx {
   // the result: packed (e,f) and (m,n) spaces, used for their K index
   int pack = 0;
   PairSpace ps_vvp, ps_oop;
+  int64_t spaces_built = 0;   // times the spaces were (re)built
   double *b64[10] = {};            // FP64 blocked operands (fp64/fp32 modes)
   int b64_layout = -1;
   int b64_nb = 0;

@@ -185,11 +185,7 @@ def test_blocked_adjoint_at_class_and_run_edges(prec, tol, runs, workspace,
     v2 = antisym(rng.normal(size=t2.shape)) * (
         (lv[:, None, None, None] + lv[None, :, None, None]) ==
         (lo[None, None, :, None] + lo[None, None, None, :]))
-    ref1, ref2 = numpy.empty_like(v1), numpy.empty_like(v2)
-    for y in range(ng):
-        g1, g2 = oracle.stanton_rhs_transpose(F, I, t1[y], t2[y], v1[y],
-                                              v2[y])
-        ref1[y], ref2[y] = g1, oracle.antisymmetrize(g2)
+    ref1, ref2 = _adjoint_reference(F, I, t1, t2, v1, v2)
     eng = _run_engine(F, I, no, nv, ng, lo, lv, "fp64")
     T1, T2, V1, V2 = (torch.as_tensor(x, device=d) for x in (t1, t2, v1, v2))
     eng.adjoint_begin(T1, T2)
@@ -199,6 +195,52 @@ def test_blocked_adjoint_at_class_and_run_edges(prec, tol, runs, workspace,
     eng.adjoint_end()
     assert rel(to_np(G1), ref1) < tol
     assert rel(to_np(G2), ref2) < tol
+    eng.close()
+
+
+def _adjoint_reference(F, I, t1, t2, v1, v2):
+    ref1, ref2 = numpy.empty_like(v1), numpy.empty_like(v2)
+    for y in range(len(v1)):
+        g1, g2 = oracle.stanton_rhs_transpose(F, I, t1[y], t2[y], v1[y],
+                                              v2[y])
+        ref1[y], ref2[y] = g1, oracle.antisymmetrize(g2)
+    return ref1, ref2
+
+
+@pytest.mark.parametrize("cache", ["64", "0"])
+def test_adjoint_after_other_labels(cache, monkeypatch):
+    """Three kinds of orbitals that every block conserves; the second kind
+    counts as beta or as alpha, so that the pair classes of one problem have
+    two sets of lengths (128 and 192 ring pairs).  J^T after each relabelling
+    and with blocking off, against the oracle; tolerance of the adjoint."""
+    d = dev()
+    ng, o, v = 3, (4, 2, 1), (7, 4, 2)
+    monkeypatch.setenv("FTCC_ADJOINT_CACHE_GB", cache)
+    rng = numpy.random.default_rng(11)
+    no, nv = sum(o), sum(v)
+    kind = numpy.repeat([0, 1, 2, 0, 1, 2], o + v)
+    # equal sums of 4^kind: the same kinds on both sides of a block
+    F, I, t1, t2, _, _ = _spin_problem(no, nv, ng, 4 ** kind, rng)
+    ko, kv = 4 ** kind[:no], 4 ** kind[no:]
+    v1 = rng.normal(size=t1.shape) * (kv[:, None] == ko[None, :])
+    v2 = antisym(rng.normal(size=t2.shape)) * (
+        (kv[:, None, None, None] + kv[None, :, None, None]) ==
+        (ko[None, None, :, None] + ko[None, None, None, :]))
+    ref1, ref2 = _adjoint_reference(F, I, t1, t2, v1, v2)
+    as_beta, as_alpha = (kind >= 1).astype(int), (kind >= 2).astype(int)
+    eng = _run_engine(F, I, no, nv, ng, as_beta[:no], as_beta[no:], "fp64")
+    T1, T2, V1, V2 = (torch.as_tensor(x, device=d) for x in (t1, t2, v1, v2))
+    eng.adjoint_begin(T1, T2)
+    for lab in (as_beta, as_alpha, None, as_beta, 1 - as_alpha):
+        if lab is None:
+            eng.set_spin(None, None)
+        else:
+            eng.set_spin(lab[:no], lab[no:])
+        G1, G2 = eng.empty_amplitudes()
+        eng.adjoint_apply(V1, V2, G1, G2)
+        assert rel(to_np(G1), ref1) < 1e-12, lab
+        assert rel(to_np(G2), ref2) < 1e-12, lab
+    eng.adjoint_end()
     eng.close()
 
 

@@ -578,9 +578,11 @@ void run_spin(ftcc_ctx *c, const Gemm &base, int prec,
     }
     if (K == 0) {
       if (!writes_all || !first) continue;
-      g.K = 0;   // C = beta * C + gamma * D only
+      // C = beta * C + gamma * D only; K over several indices stays that, so
+      // that the block can share a launch with the others of its output
+      g.K = 0;
       g.K1 = 1;
-      g.K2 = 0;
+      g.K2 = nk >= 2 ? 1 : 0;
     }
     items.push_back(g);
     item_blk.push_back(cb);

@@ -79,7 +79,8 @@ def test_split_product_tile_and_k_edges(M, N, K, batch):
 # 64, 65 pairs, runs of 31 to 33 orbitals, unequal and empty runs
 _RUNS = [((1, 2), (31, 16)), ((3, 4), (11, 8)), ((5, 5), (13, 13)),
          ((2, 8), (4, 8)), ((3, 0), (5, 4)), ((33, 2), (2, 3)),
-         ((2, 1), (33, 32)), ((4, 4), (8, 8)), ((1, 1), (1, 1))]
+         ((2, 1), (33, 32)), ((4, 4), (8, 8)), ((1, 1), (1, 1)),
+         ((0, 3), (5, 4)), ((3, 2), (0, 4)), ((0, 2), (0, 5))]
 
 
 def _run_problem(runs, ng, rng):

@@ -721,7 +721,10 @@ int64_t split_elems(const ftcc_ctx *c, int id) {
 int64_t carve_len(int64_t doubles) { return (doubles + 31) / 32 * 32; }
 
 // arena doubles of the operand set of precision `prec` at chunk nb (0: the
-// dense FP64/FP32 layout reads its operands in place)
+// dense FP64/FP32 layout reads its operands in place).  The spin-blocked
+// FP64 and FP32 sets have the same slots, of FP64 size: with FP32 slots of
+// half the size, the FP64 steps after an FP32 start found room for half the
+// chunk only.
 int64_t operand_doubles(const ftcc_ctx *c, int prec, int nb) {
   int64_t tot = 0;
   for (int id = 0; id < NOPS; ++id) {
@@ -731,8 +734,7 @@ int64_t operand_doubles(const ftcc_ctx *c, int prec, int nb) {
       const int64_t elems = rows * split_ld(space_len(c, op_k(c, id))) * slots;
       tot += 2 * carve_len((elems + 3) / 4 + 1);   // four bf16 per double
     } else if (c->spin) {
-      const int64_t elems = rows * space_len(c, op_k(c, id)) * slots;
-      tot += carve_len(prec == FTCC_PREC_FP32 ? (elems + 1) / 2 : elems);
+      tot += carve_len(rows * space_len(c, op_k(c, id)) * slots);
     }
   }
   return tot;
@@ -785,23 +787,24 @@ void ensure_split_buffers(ftcc_ctx *c) {
 }
 
 // Spin-blocked operand buffers of the FP64 and FP32 modes (elements of that
-// type), carved from the arena (the other precision's copies there are given
-// up).
+// type in the same slots), carved from the arena (the split copies there are
+// given up; after a switch between the two, those that depend on the
+// integrals only are gathered again in the other type).
 void ensure_b64_buffers(ftcc_ctx *c) {
-  const bool f32 = c->prec == FTCC_PREC_FP32;
-  const int owner = f32 ? 3 : 2;
-  if (c->arena_owner == owner && c->b64_layout == op_layout(c) &&
-      c->b64_nb == c->nb)
+  const int owner = c->prec == FTCC_PREC_FP32 ? 3 : 2;
+  if (c->arena_owner >= 2 && c->b64_layout == op_layout(c) &&
+      c->b64_nb == c->nb) {
+    if (c->arena_owner != owner) c->b64_fixed_valid = false;
+    c->arena_owner = owner;
     return;
+  }
   double *p = operand_arena(c, operand_doubles(c, c->prec, c->nb));
   for (int id = 0; id < NOPS; ++id) split_of(c, id) = SplitMat();
   c->split_layout = -1;
   for (int id = 0; id < NOPS; ++id) {
     c->b64[id] = p;
-    const int64_t elems = (int64_t)space_len(c, op_rows(c, id)) *
-                          space_len(c, op_k(c, id)) *
-                          (OP_FIXED[id] ? 1 : c->nb);
-    p += carve_len(f32 ? (elems + 1) / 2 : elems);
+    p += carve_len((int64_t)space_len(c, op_rows(c, id)) *
+                   space_len(c, op_k(c, id)) * (OP_FIXED[id] ? 1 : c->nb));
   }
   c->arena_owner = owner;
   c->b64_layout = op_layout(c);
@@ -1301,8 +1304,8 @@ int chunk_for_budget(const ftcc_ctx *c) {
   const int64_t sm = std::max<int64_t>(VV, std::max<int64_t>(VO, OO));
   // five n^4 intermediates (seven in the dense layout, which also forms tau
   // and t2r), Wmnij/Wabef/U, and the seven per-slot product operands of the
-  // current precision: split into bf16 pairs (bf16x3) or as FP64
-  // spin-blocked copies (FP64/FP32 spin layout), one set at a time
+  // current precision: split into bf16 pairs (bf16x3) or as spin-blocked
+  // copies in slots of FP64 size (FP64/FP32 spin layout), one set at a time
   const int64_t operands =
       c->prec == FTCC_PREC_BF16X3
           ? 4 * 7 *

@@ -105,9 +105,10 @@ struct ftcc_ctx {
   bool split_fixed_valid = false;
   int split_layout = -1;        // spin state the split buffers are sized for
   int split_nb = 0;             // and the chunk
-  // the product operands of either precision (split-bf16 pairs or FP64
-  // blocked copies, one set at a time) are carved from one allocation, so a
-  // precision switch allocates nothing: owner 0 none, 1 split, 2 FP64
+  // the product operands of the three precisions (split-bf16 pairs, or FP64
+  // or FP32 blocked copies, one set at a time) are carved from one
+  // allocation, so a precision switch allocates nothing: owner 0 none,
+  // 1 split, 2 FP64, 3 FP32
   double *arena = nullptr;
   int64_t arena_doubles = 0;
   int arena_owner = 0;
@@ -169,7 +170,7 @@ struct ftcc_ctx {
   int pack = 0;
   PairSpace ps_vvp, ps_oop;
   int64_t spaces_built = 0;   // times the spaces were (re)built
-  double *b64[10] = {};            // FP64 blocked operands (fp64/fp32 modes)
+  double *b64[10] = {};            // blocked operands (fp64/fp32 modes)
   int b64_layout = -1;
   int b64_nb = 0;
   bool b64_fixed_valid = false;

@@ -166,6 +166,30 @@ def test_one_engine_takes_other_compositions(prec, tol, runs):
     eng.close()
 
 
+@pytest.mark.parametrize("first", ["fp64", "fp32"])
+def test_precision_switches_keep_the_chunk(first):
+    """FP32 and FP64 residuals in turn on one engine: the chunk stays (all
+    grid points here) and every result is that of its precision; tolerances
+    of the residual."""
+    d = dev()
+    ng = 6
+    rng = numpy.random.default_rng(3)
+    no, nv, (F, I, t1, t2, lo, lv) = _run_problem(((5, 5), (13, 13)), ng, rng)
+    ref1, ref2 = oracle.residual_tbar(F, I, t1, t2)
+    eng = _run_engine(F, I, no, nv, ng, lo, lv, first)
+    T1, T2 = (torch.as_tensor(x, device=d) for x in (t1, t2))
+    b1, b2 = torch.empty_like(T1), torch.empty_like(T2)
+    for prec in (first, "fp64", "fp32", "fp64", "bf16x3", "fp32", "fp64"):
+        eng.set_precision(prec)
+        eng.residual(T1, T2, b1, b2)
+        tol = {"fp64": 1e-12, "fp32": 1e-5, "bf16x3": 2e-4}[prec]
+        assert rel(to_np(b1), ref1) < tol, prec
+        assert rel(to_np(b2), ref2) < tol, prec
+        if prec != "bf16x3":
+            assert eng.chunk() == ng, prec
+    eng.close()
+
+
 @pytest.mark.parametrize("workspace,cache", [(None, "64"), (None, "0"),
                                              ("0.0001", "0")])
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("bf16x3", 2e-4)])

@@ -30,7 +30,8 @@ typedef struct ftcc_ctx ftcc_ctx;
  * (Fermi factors, propagators, quadrature, damping, norms, energies) is FP64 */
 enum {
   FTCC_PREC_FP64 = 0,   /* FP64 operands, FP64 MFMA                          */
-  FTCC_PREC_FP32 = 1,   /* operands rounded to FP32, FP32 MFMA and accum.     */
+  FTCC_PREC_FP32 = 1,   /* operands rounded to FP32, FP32 MFMA; sums of 128   */
+                        /* terms in FP32, added up in FP64 (wide tiles: FP32) */
   FTCC_PREC_BF16X3 = 2  /* x = hi+lo in bf16; hi*hi+hi*lo+lo*hi, FP32 accum.  */
 };
 
@@ -411,10 +412,11 @@ int ftcc_profile_read(ftcc_ctx *ctx, int64_t *launches, double *ms,
                       double *flops);
 /* Launch plan of the generic GEMMs (the O(n^5) terms, and the products of
  * dense FP64/FP32 contexts): tile_policy 0 takes 64x64 tiles (in FP64 as few
- * 16s as hold a side for K of at most 64), 1 128x128 unless a
- * dimension is at most 64, 2 the best of 128x64, 64x128 and 64x64 by their
- * estimated time; K is split at
- * most until a launch has split_target workgroups (default 1024).
+ * 16s as hold a side for K of at most 64, in FP32 128x128 for large products
+ * with little padding), 1 128x128 unless a dimension is at most 64, 2 the best
+ * of 128x64, 64x128 and 64x64 by their estimated time (FP32: 1 and 2 where a
+ * product has 1024 of those tiles, else 64x64); K is split at most until a
+ * launch has split_target workgroups (default 1024).
  * Results are the same up to the summation order of split K.  No
  * counterpart in the reference (the tile autotuner of the batch sets it). */
 int ftcc_set_gemm_plan(ftcc_ctx *ctx, int tile_policy, int split_target);

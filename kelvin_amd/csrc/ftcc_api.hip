@@ -319,7 +319,7 @@ void run_group(ftcc_ctx *c, const Gemm *g0, const int *cblk0, int n, int prec,
         cblk[m] = cblk0[order[at]];
       }
     }
-    ensure_partial(c, gemm_group_scratch(g, cblk, m));
+    ensure_partial(c, gemm_group_scratch(g, cblk, m, prec));
     c->cur_line = c->site_override ? c->site_override : line;
     c->cur_M = g[0].M;
     c->cur_N = g[0].N;

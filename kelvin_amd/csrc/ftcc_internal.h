@@ -97,6 +97,12 @@ struct Scratch {
   size_t lowp_bytes = 0;
 };
 
+// FP32 products add at most FOLD_K of K in FP32 and those sums in FP64, so
+// that their rounding does not grow with K (products of fewer than 1024
+// tiles had it so by their split K, of 128 to 255 of K each).  The generic
+// engine's launches of more wide tiles keep one FP32 sum (gemm.hip).
+constexpr int FOLD_K = 128;
+
 // Up to GEMM_GROUP products in one launch, n >= 1, of equal operand layouts
 // (gemm_groupable) and batch.  cblk names each product's output: products of
 // equal cblk are added up in the order given (equal M, N and C; alpha, beta
@@ -104,7 +110,8 @@ struct Scratch {
 constexpr int GEMM_GROUP = 8;
 bool gemm_groupable(const Gemm &x, const Gemm &y);
 // doubles of Scratch::partial that gemm_run_group needs
-size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n);
+size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n,
+                          int precision);
 void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
                     Scratch &scr, hipStream_t s);
 

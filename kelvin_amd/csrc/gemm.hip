@@ -302,6 +302,26 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmGroup grp) {
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < CT; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  // FP32 sums run over at most FOLD_K of K and are added up in FP64 (not on
+  // the wide tiles: plan_of)
+  constexpr bool FOLD = sizeof(T) == 4 && TM == 64 && TN == 64;
+  d4_t sum[FOLD ? RT : 1][FOLD ? CT : 1];
+  if (FOLD) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) sum[i][j] = d4_t{0, 0, 0, 0};
+  }
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sum[i][j][v] += (double)acc[i][j][v];
+        acc[i][j] = acc_t{0, 0, 0, 0};
+      }
+  };
 
   double ra[TM / 16], rb[TN / 16];
   tile_offsets<TM, TN>(p, m0, n0, aoff, boff);
@@ -337,11 +357,17 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmGroup grp) {
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
           acc[rt][ct] = Mma<T>::op(a[rt][kk], b[ct][kk], acc[rt][ct]);
+    if (FOLD && (s + 1) % (FOLD_K / BK) == 0) fold();
     if (s + 1 < nslab)
       store_slab<T, A_MFAST, B_NFAST, TM, TN>(As[DB ? buf ^ 1 : 0],
                                               Bs[DB ? buf ^ 1 : 0], ra, rb);
     __syncthreads();
   }
+
+  if (FOLD) fold();
+  auto result = [&](int rt, int ct, int v) {
+    return FOLD ? sum[rt][ct][v] : (double)acc[rt][ct][v];
+  };
 
   // epilogue: lane holds column li of each 16x16 block, rows Mma<T>::crow.
   // Output offsets of the tile's rows and columns (after the scatter maps;
@@ -398,7 +424,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmGroup grp) {
           const int lr = wm * (TM / 2) + rt * 16 + Mma<T>::crow(lg, v);
           const bool ok = crow[lr] >= 0 && ccol[lc] >= 0;
           oc[ct][v] = ok ? crow[lr] + ccol[lc] : -1;
-          res[ct][v] = p.alpha * (double)acc[rt][ct][v];
+          res[ct][v] = p.alpha * result(rt, ct, v);
         }
       if (D) {
 #pragma unroll
@@ -434,7 +460,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_mfma_kernel(GemmGroup grp) {
         for (int v = 0; v < 4; ++v) {
           const int lr = wm * (TM / 2) + rt * 16 + Mma<T>::crow(lg, v);
           if (m0 + lr < p.M && n0 + lc < p.N)
-            P[(int64_t)(m0 + lr) * p.N + n0 + lc] = (double)acc[rt][ct][v];
+            P[(int64_t)(m0 + lr) * p.N + n0 + lc] = result(rt, ct, v);
         }
       }
     }
@@ -691,13 +717,20 @@ __global__ __launch_bounds__(256) void reduce_few_kernel(GemmGroup grp) {
 // size measured but one 4096^3 (TFLOP/s FP64, 64x64 | 128x64 | 128x128: 11
 // of 1458^3 51 | 48 | 42; 3249^3 48 | 44 | 43; 15 of 722^3 42 | 36 | 30;
 // 4096^3 54 | 53 | 55), and for the short-K terms, whose groups it shortens
-// by 4% of a step at n = 66; the wider ones are left to the autotuner.  Per CU a workgroup's slab takes the time of its
-// MFMAs, and a CU works through its workgroups of a launch at that rate or
+// by 4% of a step at n = 66; the wider ones are left to the autotuner.  Per
+// CU a workgroup's slab takes the time of its MFMAs, and a CU works through its workgroups of a launch at that rate or
 // at that of the load latency of its resident ones, whichever is longer;
 // partial sums (splits of K, and products of one output) add their write
 // and read.  (Splitting every launch of fewer than 1024 workgroups, as this
 // rule did before, spent half of an FP64 step at n = 54 in the sums of
 // partials: 7.4 of 14.4 ms.)
+//   FP32: 64x64 too, except that one product of at least 1024 128x128 tiles
+// with at most 6% of padding takes those, as policy 1 (2: the narrower one
+// by the aspect) does from 1024 on: a wide tile has no registers for the FP64
+// sums of its accumulators, which at that many tiles run over all of K.
+// (TFLOP/s and error of the result, 128x128 | 64x64: 4096^3 82 1.1e-6 | 76
+// 2.0e-7; 4356^3, 5% of padding, 78 1.2e-6 | 72 2.0e-7; four of 2178^3, 11%,
+// 64 8.3e-7 | 64 2.0e-7; the sums themselves cost a 64x64 tile 2 to 4%.)
 struct Plan {
   Tile t;
   int kc;   // K of a split, whole slabs
@@ -731,7 +764,7 @@ double estimate_us(const Gemm *g, const int *cblk, int n, Tile t, int kc) {
                                  std::ceil(b / (256.0 * occ)) * lat);
   return us + (sum > 0.0 ? 4.0 + sum : 0.0);
 }
-Plan plan_of(const Gemm *g, const int *cblk, int n) {
+Plan plan_of(const Gemm *g, const int *cblk, int n, bool f32) {
   const int pol = g[0].tile_policy;
   const Tile cand[4] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
   int M = 0, N = 0, K = 0;
@@ -742,14 +775,22 @@ Plan plan_of(const Gemm *g, const int *cblk, int n) {
   }
   const int whole = std::max(1, (K + BK - 1) / BK) * BK;
   Plan best{{64, 64}, whole};
+  if (f32 && n == 1 && M > 64 && N > 64) {
+    const Tile t = pol != 2 ? cand[0] : M >= N ? cand[1] : cand[2];
+    const int64_t tiles = tiles_of(g[0], t);
+    const bool tight = (double)M * N * g[0].nb1 * g[0].nb2 >=
+                       0.94 * (double)tiles * t.m * t.n;
+    if (tiles >= 1024 && (pol != 0 || tight)) return Plan{t, whole};
+  }
   double us = 1e300;
   for (const Tile &t : cand) {
+    if (f32 && t.m * t.n > 64 * 64) continue;
     // the wide policies take no 128-wide tile for a side of at most 64
     if ((M <= 64 && t.m > 64) || (N <= 64 && t.n > 64)) continue;
     const bool full = t.m >= std::min(128, (M + 63) / 64 * 64) &&
                       t.n >= std::min(128, (N + 63) / 64 * 64);
     if (pol == 0 && t.m * t.n > 64 * 64) continue;
-    if (pol == 1 && !full) continue;
+    if (pol == 1 && !f32 && !full) continue;
     if (pol == 2 && t.m * t.n == 128 * 128) continue;
     int64_t blocks = 0;
     for (int k = 0; k < n; ++k) blocks += tiles_of(g[k], t);
@@ -936,8 +977,9 @@ bool gemm_groupable(const Gemm &x, const Gemm &y) {
          (x.K2 > 0) == (y.K2 > 0) && x.nb1 == y.nb1 && x.nb2 == y.nb2;
 }
 
-size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n) {
-  const Plan pl = plan_of(g, cblk, n);
+size_t gemm_group_scratch(const Gemm *g, const int *cblk, int n,
+                          int precision) {
+  const Plan pl = plan_of(g, cblk, n, precision == FTCC_PREC_FP32);
   size_t need = 0;
   for (int k = 0; k < n; ++k) {
     const int sp = splits_of(g[k], pl.kc);
@@ -954,7 +996,7 @@ void gemm_run_group(const Gemm *g, const int *cblk, int n, int precision,
   require(precision == FTCC_PREC_FP64 || precision == FTCC_PREC_FP32,
           "the generic GEMM runs FP64 or FP32 (bf16x3 uses sbgemm)");
   require(n >= 1 && n <= GEMM_GROUP, "GEMM group size");
-  const Plan pl = plan_of(g, cblk, n);
+  const Plan pl = plan_of(g, cblk, n, precision == FTCC_PREC_FP32);
   // K of one index and at most 64, each output of one product: the short-K
   // kernel (in FP64, the precision of those terms, and under the default
   // launch plan)

@@ -148,6 +148,25 @@ __global__ __launch_bounds__(256, 2) void pgemm_kernel(Dev<T> p) {
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < RT; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  // FP32: the sums folded so far
+  constexpr bool FOLD = sizeof(T) == 4;
+  d4_t sum[FOLD ? RT : 1][FOLD ? RT : 1];
+  if (FOLD) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < RT; ++j) sum[i][j] = d4_t{0, 0, 0, 0};
+  }
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < RT; ++j) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sum[i][j][v] += (double)acc[i][j][v];
+        acc[i][j] = acc_t{0, 0, 0, 0};
+      }
+  };
 
   // the maps above are read after a barrier even when K is empty, and their
   // loads are not counted by the waits below
@@ -193,11 +212,13 @@ __global__ __launch_bounds__(256, 2) void pgemm_kernel(Dev<T> p) {
 #pragma unroll
         for (int ct = 0; ct < RT; ++ct)
           acc[rt][ct] = Mma<T>::op(a[rt][k], b[ct][k], acc[rt][ct]);
+    if (FOLD && (s + 1) % (FOLD_K / (ROWB / (int)sizeof(T))) == 0) fold();
     cur = cur + 1 == NST ? 0 : cur + 1;
     nxt = nxt + 1 == NST ? 0 : nxt + 1;
   }
   // no load may still be writing LDS when the workgroup ends
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (FOLD) fold();
 
   // lane holds column li of each block.  Reads of C (beta != 0) are
   // unconditional (a dropped element reads element 0) and every value is
@@ -216,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void pgemm_kernel(Dev<T> p) {
         off[ct][v] = (rr >= 0 && cc >= 0)
                          ? (int64_t)rr * p.sCm + (int64_t)cc * p.sCn
                          : (int64_t)-1;
-        res[ct][v] = p.alpha * (double)acc[rt][ct][v];
+        res[ct][v] = p.alpha * (FOLD ? sum[rt][ct][v] : (double)acc[rt][ct][v]);
       }
     }
     if (p.beta != 0.0) {

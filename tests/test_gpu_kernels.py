@@ -75,6 +75,63 @@ def test_split_product_tile_and_k_edges(M, N, K, batch):
     assert (numpy.abs(out - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("layout", ["nn", "tn", "nt", "tt"])
+@pytest.mark.parametrize("M,N,K,batch", [(70, 65, 127, 1), (64, 64, 129, 2),
+                                         (33, 130, 4100, 1),
+                                         (260, 300, 1000, 3)])
+def test_fp32_products_add_up_in_fp64(M, N, K, batch, layout):
+    """Products of 1 and 1 + 2^-17: sums of 128 of them are exact in FP32 and
+    of any number in FP64, while one FP32 sum loses the 2^-17 from 256 terms
+    on.  Equal to the last bit."""
+    from kelvin_amd.engine import FTEngine
+    d = dev()
+    x = 1.0 + 2.0 ** -17
+
+    def ones(r, c, t):
+        a = torch.ones(batch, c, r, dtype=torch.float64, device=d)
+        return a.transpose(1, 2) if t == "t" else a.reshape(batch, r, c)
+    eng = FTEngine(2, 2, 1)
+    C = torch.zeros(batch, M, N, dtype=torch.float64, device=d)
+    eng.gemm(ones(M, K, layout[0]), x * ones(K, N, layout[1]), C,
+             precision="fp32")
+    assert bool((C == K * x).all())
+    eng.close()
+
+
+def test_fp32_residual_adds_up_in_fp64():
+    """The same through a ring product of the spin-blocked residual: only
+    <mb||ej> of four beta indices (1 + 2^-17) and opposite-spin amplitudes
+    (1), so that R2 is a sum of 1024 equal terms."""
+    from kelvin_amd.engine import FTEngine
+    from kelvin_amd.engine import ONE_E, TWO_E
+    from kelvin_amd.ov_blocks import one_e_blocks, two_e_blocks
+    d = dev()
+    n, h = 64, 32
+    x = 1.0 + 2.0 ** -17
+    F = {k: torch.zeros(n, n, dtype=torch.float64, device=d) for k in ONE_E}
+    I = {k: torch.zeros(n, n, n, n, dtype=torch.float64, device=d)
+         for k in TWO_E}
+    I["vovo"][h:, h:, h:, h:] = -x
+    t1 = torch.zeros(1, n, n, dtype=torch.float64, device=d)
+    t2 = torch.zeros(1, n, n, n, n, dtype=torch.float64, device=d)
+    for a, b, s in ((0, h, 1.0), (h, 0, -1.0)):
+        t2[:, a:a + h, b:b + h, :h, h:] = s
+        t2[:, a:a + h, b:b + h, h:, :h] = -s
+    eng = FTEngine(n, n, 1, precision="fp32")
+    eng.set_blocks(one_e_blocks(**F), two_e_blocks(**I))
+    eng.set_denominators(torch.ones(n, n, dtype=torch.float64, device=d),
+                         torch.ones(n, n, n, n, dtype=torch.float64,
+                                    device=d))
+    eng.set_grid(numpy.zeros(1), numpy.zeros((1, 1)))
+    lab = numpy.repeat([0, 1], h)
+    eng.set_spin(lab, lab)
+    b1, b2 = torch.empty_like(t1), torch.empty_like(t2)
+    eng.residual(t1, t2, b1, b2)
+    r = b2[0, :h, h:, :h, h:]
+    assert bool((r.abs() == h * h * x).all())
+    eng.close()
+
+
 # (alpha, beta) occupied and virtual orbitals: (v, o) classes of 31, 32, 33,
 # 64, 65 pairs, runs of 31 to 33 orbitals, unequal and empty runs
 _RUNS = [((1, 2), (31, 16)), ((3, 4), (11, 8)), ((5, 5), (13, 13)),

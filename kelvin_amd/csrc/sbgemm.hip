@@ -125,28 +125,30 @@ __device__ inline int lds_slot(int row, int c) { return c ^ ((row >> 2) & 3); }
 // One wave's share of a K step of one operand: rows [32w, 32w + 32) of the
 // tile in two loads of sixteen rows x four chunks; the lane that lands at
 // slot (lane & 3) of row r fetches the chunk stored there.  off: its byte
-// offsets from the tile's first row, the same in every step.
-struct Rows {
+// offsets from the tile's first row, the same in every step (Off: 32 bits
+// hold them for rows of less than 2^22 elements).
+template <typename Off> struct Rows {
   const __bf16 *p;   // first row of the tile
-  unsigned off[2];
+  Off off[2];
 };
-__device__ inline Rows tile_rows(const __bf16 *p, int64_t ld, int row0,
-                                 int rows, int wave, int lane) {
-  Rows r;
+template <typename Off>
+__device__ inline Rows<Off> tile_rows(const __bf16 *p, int64_t ld, int row0,
+                                      int rows, int wave, int lane) {
+  Rows<Off> r;
   r.p = p + 2 * row0 * ld;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int rowl = wave * 32 + j * 16 + (lane >> 2);
     const int c = lds_slot(rowl, lane & 3);   // the map is an involution
-    r.off[j] = (unsigned)min(rowl, rows - 1 - row0) * (unsigned)(4 * ld) +
-               16u * c;
+    r.off[j] = (Off)min(rowl, rows - 1 - row0) * (Off)(4 * ld) + 16u * c;
   }
   return r;
 }
 // load q (0, 1: A, 2, 3: B) of K step t into a stage
-__device__ inline void load_part(const Rows &A, const Rows &B, int q, int t,
-                                 char *stage, int wave) {
-  const Rows &r = q < 2 ? A : B;
+template <typename Off>
+__device__ inline void load_part(const Rows<Off> &A, const Rows<Off> &B,
+                                 int q, int t, char *stage, int wave) {
+  const Rows<Off> &r = q < 2 ? A : B;
   __builtin_amdgcn_global_load_lds(
       (const void *)((const char *)(r.p + (int64_t)t * (2 * BK)) +
                      r.off[q & 1]),
@@ -223,7 +225,7 @@ __device__ __forceinline__ void mfma_step(f16_t (&acc)[RT][CT],
 // wn CT: 4x2 blocks on 2x4 waves for a whole tile; for a last tile with nr
 // (nc) <= 6 blocks of rows (columns), nr x 1 blocks on 1x8 waves (1 x nc on
 // 8x1), whose matrix work is nr / 8 of a whole tile's.
-template <int RT, int CT>
+template <int RT, int CT, typename Off = unsigned>
 __device__ __forceinline__ void tile_product(const SbDev &p, const SbProb &pr,
                                              int bt, int m0, int n0, char *lds,
                                              int wm, int wn) {
@@ -235,10 +237,10 @@ __device__ __forceinline__ void tile_product(const SbDev &p, const SbProb &pr,
   const int *map = t < BM ? pr.rmap : pr.cmap;
   const int mapped = e < (t < BM ? pr.M : pr.N) ? (map ? map[e] : e) : -1;
   const int nstep = pr.Kp / BK;   // even
-  const Rows A =
-      tile_rows(pr.A + 2 * bt * pr.sAb, pr.lda, m0, pr.M, wave, lane);
-  const Rows B =
-      tile_rows(pr.B + 2 * bt * pr.sBb, pr.ldb, n0, pr.N, wave, lane);
+  const Rows<Off> A =
+      tile_rows<Off>(pr.A + 2 * bt * pr.sAb, pr.lda, m0, pr.M, wave, lane);
+  const Rows<Off> B =
+      tile_rows<Off>(pr.B + 2 * bt * pr.sBb, pr.ldb, n0, pr.N, wave, lane);
 
   f16_t acc[RT][CT];
 #pragma unroll
@@ -351,6 +353,17 @@ __global__ __launch_bounds__(512, 1) void sbgemm_kernel(SbDev p) {
       tile_product<4, 2>(p, pr, bt, m0, n0, lds, wave >> 2, wave & 3);
   }
 #undef FTCC_EDGE
+}
+
+// The same for longer rows, whose offsets take 64 bits (whole tiles only:
+// the launch has no edge tiles)
+__global__ __launch_bounds__(512, 1) void sbgemm_long_kernel(SbDev p) {
+  extern __shared__ char lds[];
+  int bt, tm, tn;
+  const SbProb pr = tile_of(p, bt, tm, tn);
+  const int wave = threadIdx.x >> 6;
+  tile_product<4, 2, uint64_t>(p, pr, bt, tm * BM, tn * BN, lds, wave >> 2,
+                               wave & 3);
 }
 
 __device__ inline void split1(double v, __bf16 &hi, __bf16 &lo) {
@@ -715,8 +728,10 @@ void sbgemm_grouped(int nprob, const SbProblem *prob, int nb, double alpha,
                     double beta, double *C, int64_t sCm, int64_t sCn,
                     int64_t sCb, hipStream_t s) {
   require(nprob >= 1 && nprob <= MAXP, "1 to 3 problems per grouped launch");
-  static std::once_flag attr;
+  static std::once_flag attr, attr_long;
   set_max_lds_once(attr, (const void *)sbgemm_kernel, (int)LDS_BYTES);
+  set_max_lds_once(attr_long, (const void *)sbgemm_long_kernel,
+                   (int)LDS_BYTES);
   // band height of the launch order (FTCC_SB_GROUP_M tunes it)
   static const int group_m = [] {
     const char *e = getenv("FTCC_SB_GROUP_M");
@@ -733,24 +748,25 @@ void sbgemm_grouped(int nprob, const SbProblem *prob, int nb, double alpha,
   p.alpha = alpha;
   p.beta = beta;
   p.nprob = 0;
-  int64_t tiles = 0, whole = 0;
+  int64_t tiles = 0, whole = 0, ld = 0;
+  for (int k = 0; k < nprob; ++k)
+    ld = std::max(ld, std::max(prob[k].A.ld, prob[k].B.ld));
+  // a tile's rows beyond 32-bit byte offsets
+  const bool far = ld >= (1LL << 32) / (4 * BM);
   for (int k = 0; k < nprob; ++k) {
     const SbProblem &q = prob[k];
     if (q.M <= 0 || q.N <= 0) continue;
     require(q.A.ld % 32 == 0 && q.B.ld % 32 == 0 && q.A.ld >= q.K &&
                 q.B.ld >= q.K,
             "split operands need K padded to 32");
-    // a tile's rows lie within 32-bit byte offsets
-    require(std::max(q.A.ld, q.B.ld) < (1LL << 32) / (4 * BM),
-            "split operand rows too long");
     SbProb &d = p.pr[p.nprob++];
     d.M = q.M;
     d.N = q.N;
     d.Kp = (int)((q.K + 31) / 32 * 32);
     d.tilesM = (q.M + BM - 1) / BM;
     d.tilesN = (q.N + BN - 1) / BN;
-    d.fullM = full_tiles(q.M, BM);
-    d.fullN = full_tiles(q.N, BN);
+    d.fullM = far ? d.tilesM : full_tiles(q.M, BM);
+    d.fullN = far ? d.tilesN : full_tiles(q.N, BN);
     d.full0 = (int)whole;
     d.edge0 = (int)(tiles - whole);
     d.A = q.A.p;
@@ -767,8 +783,8 @@ void sbgemm_grouped(int nprob, const SbProblem *prob, int nb, double alpha,
   if (p.nprob == 0 || nb <= 0) return;
   require(tiles < (1LL << 31), "too many GEMM tiles");
   p.nfull = (int)whole;
-  hipLaunchKernelGGL(sbgemm_kernel, dim3((unsigned)tiles), dim3(512),
-                     LDS_BYTES, s, p);
+  hipLaunchKernelGGL(far ? sbgemm_long_kernel : sbgemm_kernel,
+                     dim3((unsigned)tiles), dim3(512), LDS_BYTES, s, p);
   FTCC_CHECK_HIP(hipGetLastError());
 }
 

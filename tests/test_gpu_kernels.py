@@ -75,6 +75,27 @@ def test_split_product_tile_and_k_edges(M, N, K, batch):
     assert (numpy.abs(out - ref) <= bound).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 2, 2 ** 22 + 5),
+                                   (2, 35, 2 ** 22 - 64)])
+def test_split_product_of_long_rows(M, N, K):
+    """Rows of 2^22 elements and more (and the longest below them): sums of
+    few ones and twos, exact."""
+    from kelvin_amd.engine import FTEngine
+    d = dev()
+    g = torch.Generator().manual_seed(K)
+    A = torch.randint(-1, 2, (M, K), generator=g, dtype=torch.int8)
+    B = torch.randint(-1, 2, (N, K), generator=g, dtype=torch.int8)
+    A[:, 0], B[:, 0], A[:, -1], B[:, -1] = 2, 1, 1, 2
+    A, B = A.to(d).double(), B.to(d).double()
+    ref = A @ B.t()
+    assert float(ref.abs().max()) < 2 ** 22
+    C = torch.zeros(M, N, dtype=torch.float64, device=d)
+    eng = FTEngine(2, 2, 1)
+    eng.gemm(A, B.t(), C, precision="bf16x3")
+    assert torch.equal(C, ref)
+    eng.close()
+
+
 @pytest.mark.parametrize("layout", ["nn", "tn", "nt", "tt"])
 @pytest.mark.parametrize("M,N,K,batch", [(70, 65, 127, 1), (64, 64, 129, 2),
                                          (33, 130, 4100, 1),

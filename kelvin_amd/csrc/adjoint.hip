@@ -1128,6 +1128,8 @@ struct Adjoint {
   // the pair spaces of this building of theirs (ftcc_ctx::spaces_built)
   bool blocked = false;
   int64_t spaces = 0;
+  // precision that the kept intermediates were built in
+  int prec = FTCC_PREC_FP64;
   AdjSlice cache;                // grid points [0, cache.n) are kept
   AdjSlice work;                 // intermediates of uncached grid points
   // buffers of nb grid points (prepare_points and apply_points each say
@@ -1799,6 +1801,7 @@ void build_adjoint(ftcc_ctx *c, const double *T1, const double *T2) {
     A = adjoint_ws(c);
     A->blocked = blocked;
     A->spaces = c->spaces_built;
+    A->prec = c->adj_prec;
     try {
       alloc_apply_buffers(c, A, nb, keep < c->ng);
       alloc_slice(c, A, A->cache, keep);
@@ -1818,6 +1821,19 @@ void build_adjoint(ftcc_ctx *c, const double *T1, const double *T2) {
     prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
                    at_point(c, A, A->cache, y), std::min(nb, keep - y));
   FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
+}
+
+// The same again in the course of an application, whose precision may be
+// another than that of ftcc_adjoint_begin: the kept intermediates keep theirs.
+void rebuild_adjoint(ftcc_ctx *c) {
+  struct Restore {
+    ftcc_ctx *c;
+    int prec;
+    ~Restore() { c->adj_prec = prec; }
+  } restore{c, c->adj_prec};
+  const double *T1 = c->adj->T1, *T2 = c->adj->T2;
+  c->adj_prec = c->adj->prec;
+  build_adjoint(c, T1, T2);
 }
 
 }  // namespace
@@ -1851,7 +1867,7 @@ int ftcc_adjoint_apply(ftcc_ctx *c, const double *Lt1, const double *Lt2,
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
     // other spin labels since: the operand copies have other sizes now
     if (A->blocked && (!adjoint_blocked(c) || A->spaces != c->spaces_built)) {
-      build_adjoint(c, A->T1, A->T2);
+      rebuild_adjoint(c);
       A = c->adj;
     }
     if (A->blocked && (low_product(c, 3, 3) || low_product(c, 4, 2) ||

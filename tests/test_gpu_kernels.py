@@ -343,6 +343,17 @@ def test_adjoint_after_other_labels(cache, monkeypatch):
         eng.adjoint_apply(V1, V2, G1, G2)
         assert rel(to_np(G1), ref1) < 1e-12, lab
         assert rel(to_np(G2), ref2) < 1e-12, lab
+    # kept intermediates stay FP64 when rebuilt by a low-precision application
+    monkeypatch.setenv("FTCC_ADJOINT_LOWP_MIN_GFLOP", "0")
+    eng.adjoint_end()
+    eng.set_spin(as_beta[:no], as_beta[no:])
+    eng.adjoint_begin(T1, T2)
+    eng.set_spin(as_alpha[:no], as_alpha[no:])
+    for prec, tol in (("bf16x3", 2e-4), ("fp64", 1e-12)):
+        eng.adjoint_precision(prec)
+        eng.adjoint_apply(V1, V2, G1, G2)
+        assert rel(to_np(G1), ref1) < tol, prec
+        assert rel(to_np(G2), ref2) < tol, prec
     eng.adjoint_end()
     eng.close()
 

@@ -398,7 +398,9 @@ int ftcc_step_graph(ftcc_ctx *ctx, double *T1old_dev, double *T2old_dev,
                     double *T1bar_dev, double *T2bar_dev, double beta,
                     double damp, uint64_t skip_mask, double out5[5]);
 
-/* Device bytes held by the context (integrals + workspace). */
+/* Device bytes held by the context (integrals + workspace).  Under
+ * FTCC_CONTEXT_GB (GiB, environment; default no limit) an allocation past that
+ * much fails with FTCC_ENOMEM, as on a device without room for it. */
 int ftcc_workspace_bytes(const ftcc_ctx *ctx, int64_t *bytes);
 
 /* Kernel timing with HIP events on the context's stream (no counterpart in

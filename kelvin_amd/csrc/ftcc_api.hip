@@ -38,6 +38,10 @@ constexpr int MAX_PARTIAL_BLOCKS = 8192;
 
 double *dalloc(ftcc_ctx *c, int64_t n) {
   if (n <= 0) n = 1;
+  if (const char *env = getenv("FTCC_CONTEXT_GB"))
+    if ((double)(c->bytes + 8 * n) > atof(env) * (double)(1LL << 30))
+      throw Error(FTCC_ENOMEM, std::to_string(8 * n) +
+                                   " bytes exceed FTCC_CONTEXT_GB");
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, sizeof(double) * (size_t)n);
   if (e != hipSuccess)
@@ -142,18 +146,23 @@ Gemm mk(int M, int N, int K, double alpha, double beta, const double *A,
 }
 
 void ensure_partial(ftcc_ctx *c, size_t need) {
-  if (need > c->scr.partial_elems) {
-    // grow: allocation happens outside the kernel stream order, so drain it
-    FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
-    if (c->scr.partial) {
-      auto it = std::find(c->allocs.begin(), c->allocs.end(),
-                          (void *)c->scr.partial);
-      if (it != c->allocs.end()) c->allocs.erase(it);
-      c->bytes -= 8 * (int64_t)c->scr.partial_elems;
-      FTCC_CHECK_HIP(hipFree(c->scr.partial));
-    }
-    c->scr.partial = dalloc(c, (int64_t)need);
-    c->scr.partial_elems = need;
+  if (need <= c->scr.partial_elems) return;
+  // grow: allocation happens outside the kernel stream order, so drain it
+  FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
+  const size_t old = c->scr.partial_elems;
+  auto take = [&](size_t n) {
+    dfree(c, c->scr.partial);
+    c->scr.partial = nullptr;
+    c->scr.partial_elems = 0;
+    c->scr.partial = dalloc(c, (int64_t)n);
+    c->scr.partial_elems = n;
+  };
+  try {
+    take(need);
+  } catch (const Error &) {
+    (void)hipGetLastError();
+    take(old);   // what other calls count on
+    throw;
   }
 }
 

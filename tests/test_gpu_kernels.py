@@ -75,6 +75,33 @@ def test_split_product_tile_and_k_edges(M, N, K, batch):
     assert (numpy.abs(out - ref) <= bound).all()
 
 
+def test_engine_goes_on_after_a_failed_growth(monkeypatch):
+    """A split product whose partial sums find no room fails with ENOMEM; the
+    buffer that was there serves the next one."""
+    from kelvin_amd._lib import FTCCError
+    from kelvin_amd.engine import FTEngine
+    d = dev()
+    eng = FTEngine(2, 2, 1)
+
+    def product(M, K):
+        A = torch.randn(M, K, dtype=torch.float64, device=d)
+        B = torch.randn(K, M, dtype=torch.float64, device=d)
+        C = torch.zeros(M, M, dtype=torch.float64, device=d)
+        eng.gemm(A, B, C, precision="fp64")
+        assert bool(((C - A @ B).abs() <=
+                     2 * (K + 3) * U64 * (A.abs() @ B.abs())).all())
+    held = eng.workspace_bytes()
+    monkeypatch.setenv("FTCC_CONTEXT_GB", repr((held + 4096) / 2.0 ** 30))
+    with pytest.raises(FTCCError, match="FTCC_CONTEXT_GB"):
+        product(512, 16384)
+    assert eng.workspace_bytes() == held
+    product(30, 3000)
+    monkeypatch.delenv("FTCC_CONTEXT_GB")
+    product(512, 16384)
+    assert eng.workspace_bytes() > held
+    eng.close()
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 2, 2 ** 22 + 5),
                                    (2, 35, 2 ** 22 - 64)])
 def test_split_product_of_long_rows(M, N, K):

@@ -300,7 +300,8 @@ int ftcc_defect(ftcc_ctx *ctx, const double *T1_dev, const double *T2_dev,
  * intermediates of J^T for as many grid points as FTCC_ADJOINT_CACHE_GB
  * (default 64) holds; the others rebuild theirs at each application.
  * Releases the residual workspace of the forward iteration.  After other
- * spin labels the next application builds them again. */
+ * spin labels, or where the memory does not suffice for as many grid points
+ * at a time, the next application builds them again. */
 int ftcc_adjoint_begin(ftcc_ctx *ctx, const double *T1_dev,
                        const double *T2_dev);
 /* Grid points whose intermediates are kept. */

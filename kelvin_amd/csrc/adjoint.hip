@@ -1143,7 +1143,7 @@ struct Adjoint {
   // ring integrals
   double *vB = nullptr, *vA = nullptr, *vR = nullptr, *gwA = nullptr,
          *ring = nullptr;
-  // split-bf16 copies for the low-precision form (lowp_arena): made at each
+  // split-bf16 copies for the low-precision form (ensure_lowp): made at each
   // application
   double *lowp = nullptr;
   double *partials = nullptr;
@@ -1772,8 +1772,22 @@ bool adjoint_blocked(const ftcc_ctx *c) {
   return c->spin && c->spin5 && c->pack;
 }
 
-// The workspace of J^T at the amplitudes T1, T2 and its kept intermediates
-void build_adjoint(ftcc_ctx *c, const double *T1, const double *T2) {
+// Give back the operand copies that the contractions keep between calls; each
+// grows again to what it needs.
+void release_scratch(ftcc_ctx *c) {
+  FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
+  dfree(c, c->pack_buf);
+  c->pack_buf = nullptr;
+  c->pack_elems = 0;
+  dfree(c, c->lp_buf);
+  c->lp_buf = nullptr;
+  c->lp_doubles = 0;
+}
+
+// The workspace of J^T at the amplitudes T1, T2 and its kept intermediates,
+// for applications to at most `most` grid points at a time
+void build_adjoint(ftcc_ctx *c, const double *T1, const double *T2,
+                   int most) {
   drop_graph(c);
   // the forward residual's operand buffers are rebuilt when next needed
   free_workspace(c);
@@ -1794,38 +1808,38 @@ void build_adjoint(ftcc_ctx *c, const double *T1, const double *T2) {
   const int64_t per = buffer_bytes(c, blocked) +
                       (keep < c->ng ? slice_bytes(c, blocked) : 0);
   int nb = (int)std::max<int64_t>(
-      1, std::min<int64_t>(c->ng, (int64_t)(work_gb * 0.25 * (1LL << 30)) /
-                                      per));
-  Adjoint *A = nullptr;
+      1, std::min<int64_t>(most, (int64_t)(work_gb * 0.25 * (1LL << 30)) /
+                                     per));
+  const int64_t VO = (int64_t)c->nv * c->no;
   for (;; nb = (nb + 1) / 2) {
-    A = adjoint_ws(c);
+    Adjoint *A = adjoint_ws(c);
     A->blocked = blocked;
     A->spaces = c->spaces_built;
     A->prec = c->adj_prec;
     try {
       alloc_apply_buffers(c, A, nb, keep < c->ng);
       alloc_slice(c, A, A->cache, keep);
+      if (blocked) put_op(c, op_cross(c), c->oovv_ring, VO, 1, 0, A->ring, 1);
+      for (int y = 0; y < keep; y += nb)
+        prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
+                       at_point(c, A, A->cache, y), std::min(nb, keep - y));
+      A->T1 = T1;
+      A->T2 = T2;
+      A->ng = c->ng;
       break;
     } catch (const Error &e) {
       if (e.code != FTCC_ENOMEM || nb == 1) throw;
       adjoint_release(c);   // less memory free than that: fewer at a time
+      release_scratch(c);
       (void)hipGetLastError();
     }
   }
-  A->T1 = T1;
-  A->T2 = T2;
-  A->ng = c->ng;
-  const int64_t VO = (int64_t)c->nv * c->no;
-  if (blocked) put_op(c, op_cross(c), c->oovv_ring, VO, 1, 0, A->ring, 1);
-  for (int y = 0; y < keep; y += nb)
-    prepare_points(c, A, T1 + y * VO, T2 + y * VO * VO,
-                   at_point(c, A, A->cache, y), std::min(nb, keep - y));
   FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
 }
 
 // The same again in the course of an application, whose precision may be
 // another than that of ftcc_adjoint_begin: the kept intermediates keep theirs.
-void rebuild_adjoint(ftcc_ctx *c) {
+void rebuild_adjoint(ftcc_ctx *c, int most) {
   struct Restore {
     ftcc_ctx *c;
     int prec;
@@ -1833,7 +1847,7 @@ void rebuild_adjoint(ftcc_ctx *c) {
   } restore{c, c->adj_prec};
   const double *T1 = c->adj->T1, *T2 = c->adj->T2;
   c->adj_prec = c->adj->prec;
-  build_adjoint(c, T1, T2);
+  build_adjoint(c, T1, T2, most);
 }
 
 }  // namespace
@@ -1844,7 +1858,7 @@ int ftcc_adjoint_begin(ftcc_ctx *c, const double *T1, const double *T2) {
   return guarded(c, [&] {
     check_ready(c);
     require(T1 && T2, "null amplitude pointer");
-    build_adjoint(c, T1, T2);
+    build_adjoint(c, T1, T2, c->ng);
   });
 }
 
@@ -1867,20 +1881,31 @@ int ftcc_adjoint_apply(ftcc_ctx *c, const double *Lt1, const double *Lt2,
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
     // other spin labels since: the operand copies have other sizes now
     if (A->blocked && (!adjoint_blocked(c) || A->spaces != c->spaces_built)) {
-      rebuild_adjoint(c);
+      rebuild_adjoint(c, c->ng);
       A = c->adj;
     }
-    if (A->blocked && (low_product(c, 3, 3) || low_product(c, 4, 2) ||
-                       low_product(c, 2, 4)))
-      ensure_lowp(c, A);
     for (int y = 0; y < c->ng;) {
       const double *t1 = A->T1 + y * VO, *t2 = A->T2 + y * S2;
       const bool kept = y < A->cache.n;
       const int nb = std::min(A->nb, (kept ? A->cache.n : c->ng) - y);
       const AdjSlice s = kept ? at_point(c, A, A->cache, y) : A->work;
-      if (!kept) prepare_points(c, A, t1, t2, s, nb);
-      apply_points(c, A, t1, t2, s, Lt1 + y * VO, Lt2 + y * S2, G1 + y * VO,
-                   G2 + y * S2, nb);
+      try {
+        if (A->blocked && (low_product(c, 3, 3) || low_product(c, 4, 2) ||
+                           low_product(c, 2, 4)))
+          ensure_lowp(c, A);
+        if (!kept) prepare_points(c, A, t1, t2, s, nb);
+        apply_points(c, A, t1, t2, s, Lt1 + y * VO, Lt2 + y * S2,
+                     G1 + y * VO, G2 + y * S2, nb);
+      } catch (const Error &e) {
+        // the operand copies and partial sums of nb points do not fit:
+        // these and the following ones in smaller numbers
+        if (e.code != FTCC_ENOMEM || nb == 1) throw;
+        release_scratch(c);
+        (void)hipGetLastError();
+        rebuild_adjoint(c, (nb + 1) / 2);
+        A = c->adj;
+        continue;
+      }
       y += nb;
     }
   });

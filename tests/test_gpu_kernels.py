@@ -385,6 +385,51 @@ def test_adjoint_after_other_labels(cache, monkeypatch):
     eng.close()
 
 
+@pytest.mark.parametrize("cache", ["64", "0"])
+@pytest.mark.parametrize("prec", ["fp64", "bf16x3"])
+def test_adjoint_in_little_memory(prec, cache, monkeypatch):
+    """J^T wherever one grid point at a time has room: with memory between
+    what one point at a time and what all of them take, begin and apply go on
+    with fewer points (the operand copies and partial sums of an application
+    are allocated at its first launch).  Equal to the unbounded result up to
+    the order of sums."""
+    d = dev()
+    ng = 7
+    monkeypatch.setenv("FTCC_ADJOINT_CACHE_GB", cache)
+    monkeypatch.setenv("FTCC_ADJOINT_LOWP_MIN_GFLOP", "0")
+    rng = numpy.random.default_rng(5)
+    no, nv, (F, I, t1, t2, lo, lv) = _run_problem(((6, 6), (12, 12)), ng, rng)
+    v1 = rng.normal(size=t1.shape) * (lv[:, None] == lo[None, :])
+    v2 = antisym(rng.normal(size=t2.shape)) * (
+        (lv[:, None, None, None] + lv[None, :, None, None]) ==
+        (lo[None, None, :, None] + lo[None, None, None, :]))
+    T1, T2, V1, V2 = (torch.as_tensor(x, device=d) for x in (t1, t2, v1, v2))
+
+    def apply():
+        eng = _run_engine(F, I, no, nv, ng, lo, lv, "fp64")
+        eng.adjoint_begin(T1, T2)
+        eng.adjoint_precision(prec)
+        G1, G2 = eng.empty_amplitudes()
+        eng.adjoint_apply(V1, V2, G1, G2)
+        eng.adjoint_apply(V1, V2, G1, G2)
+        held = eng.workspace_bytes()
+        eng.adjoint_end()
+        eng.close()
+        return held, to_np(G1), to_np(G2)
+    every, ref1, ref2 = apply()
+    with monkeypatch.context() as m:
+        m.setenv("FTCC_WORKSPACE_GB", "0.0001")
+        one, g1, g2 = apply()
+    assert one < every
+    for part in (0.001, 0.05, 0.2, 0.4, 0.6, 0.8, 0.9, 0.95, 0.99):
+        with monkeypatch.context() as m:
+            m.setenv("FTCC_CONTEXT_GB",
+                     repr((one + part * (every - one)) / 2.0 ** 30))
+            held, g1, g2 = apply()
+        assert held < every
+        assert rel(g1, ref1) < 1e-13 and rel(g2, ref2) < 1e-13, part
+
+
 @pytest.mark.parametrize("quad", ['lin', 'mid', 'L'])
 @pytest.mark.parametrize("ng", [3, 5, 7, 9, 17, 33])
 def test_adjoint_recurrence_lengths(quad, ng):

@@ -415,7 +415,7 @@ int ftcc_profile_read(ftcc_ctx *ctx, int64_t *launches, double *ms,
                       double *flops);
 /* Launch plan of the generic GEMMs (the O(n^5) terms, and the products of
  * dense FP64/FP32 contexts): tile_policy 0 takes 64x64 tiles (in FP64 as few
- * 16s as hold a side for K of at most 64, in FP32 128x128 for large products
+ * 16s as hold a side for K of at most 64; 128x128 for long K and 1024 of them
  * with little padding), 1 128x128 unless a dimension is at most 64, 2 the best
  * of 128x64, 64x128 and 64x64 by their estimated time (FP32: 1 and 2 where a
  * product has 1024 of those tiles, else 64x64); K is split at most until a

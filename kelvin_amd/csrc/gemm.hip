@@ -713,24 +713,26 @@ __global__ __launch_bounds__(256) void reduce_few_kernel(GemmGroup grp) {
 }
 
 // Tile shape and K splits of a group: 64x64 tiles (policy 0), and the K per
-// split with the least estimated time.  64x64 was the fastest tile at every
-// size measured but one 4096^3 (TFLOP/s FP64, 64x64 | 128x64 | 128x128: 11
-// of 1458^3 51 | 48 | 42; 3249^3 48 | 44 | 43; 15 of 722^3 42 | 36 | 30;
-// 4096^3 54 | 53 | 55), and for the short-K terms, whose groups it shortens
-// by 4% of a step at n = 66; the wider ones are left to the autotuner.  Per
-// CU a workgroup's slab takes the time of its MFMAs, and a CU works through its workgroups of a launch at that rate or
-// at that of the load latency of its resident ones, whichever is longer;
-// partial sums (splits of K, and products of one output) add their write
-// and read.  (Splitting every launch of fewer than 1024 workgroups, as this
-// rule did before, spent half of an FP64 step at n = 54 in the sums of
-// partials: 7.4 of 14.4 ms.)
-//   FP32: 64x64 too, except that one product of at least 1024 128x128 tiles
-// with at most 6% of padding takes those, as policy 1 (2: the narrower one
-// by the aspect) does from 1024 on: a wide tile has no registers for the FP64
-// sums of its accumulators, which at that many tiles run over all of K.
-// (TFLOP/s and error of the result, 128x128 | 64x64: 4096^3 82 1.1e-6 | 76
-// 2.0e-7; 4356^3, 5% of padding, 78 1.2e-6 | 72 2.0e-7; four of 2178^3, 11%,
-// 64 8.3e-7 | 64 2.0e-7; the sums themselves cost a 64x64 tile 2 to 4%.)
+// split with the least estimated time.  64x64 is the fastest tile of launches
+// that do not fill the chip (TFLOP/s FP64, 64x64 | 128x64 | 128x128: 11 of
+// 1458^3 51 | 48 | 42; 15 of 722^3 42 | 36 | 30) and of the short-K terms,
+// whose groups it shortens by 4% of a step at n = 66; the wider ones are left
+// to the autotuner, but for one product of K >= 1024 and at least 1024
+// 128x128 tiles with at most 6% of padding, which takes those (FP64, 64x64 |
+// 128x128: 3 of 3249^3 46 | 51, 4096^3 50 | 55, 4356^3 46 | 48, 6561^3 43 |
+// 51, 8192^3 47 | 55; with 11% of padding, 8 of 1089x2178x2178, 46 | 42).
+//   Per CU a workgroup's slab takes the time of its MFMAs, and a CU works
+// through its workgroups of a launch at that rate or at that of the load
+// latency of its resident ones, whichever is longer; partial sums (splits of
+// K, and products of one output) add their write and read.  (Splitting every
+// launch of fewer than 1024 workgroups, as this rule did before, spent half
+// of an FP64 step at n = 54 in the sums of partials: 7.4 of 14.4 ms.)
+//   FP32: the same; under policies 1 and 2 wide tiles (2: the narrower one by
+// the aspect) only where one product has 1024 of them.  A wide tile has no
+// registers for the FP64 sums of its accumulators, which at that many tiles
+// run over all of K (TFLOP/s and error of the result, 128x128 | 64x64: 4096^3
+// 82 1.1e-6 | 76 2.0e-7; 4356^3 78 1.2e-6 | 72 2.0e-7; four of 2178^3, 11% of
+// padding, 64 8.3e-7 | 64 2.0e-7; the sums cost a 64x64 tile 2 to 4%).
 struct Plan {
   Tile t;
   int kc;   // K of a split, whole slabs
@@ -775,7 +777,7 @@ Plan plan_of(const Gemm *g, const int *cblk, int n, bool f32) {
   }
   const int whole = std::max(1, (K + BK - 1) / BK) * BK;
   Plan best{{64, 64}, whole};
-  if (f32 && n == 1 && M > 64 && N > 64) {
+  if (n == 1 && M > 64 && N > 64 && (pol == 0 ? K >= 1024 : f32)) {
     const Tile t = pol != 2 ? cand[0] : M >= N ? cand[1] : cand[2];
     const int64_t tiles = tiles_of(g[0], t);
     const bool tight = (double)M * N * g[0].nb1 * g[0].nb2 >=

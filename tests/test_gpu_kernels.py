@@ -102,6 +102,29 @@ def test_engine_goes_on_after_a_failed_growth(monkeypatch):
     eng.close()
 
 
+@pytest.mark.parametrize("precision,K", [("fp64", 1023), ("fp64", 1030),
+                                         ("fp32", 1030)])
+@pytest.mark.parametrize("layout", ["nn", "tt"])
+def test_gemm_of_1024_wide_tiles(layout, precision, K):
+    """One product of 1024 128x128 tiles, which long K takes: rounding of
+    two FP64 sums as above; FP32: of the operands and of a sum of K."""
+    from kelvin_amd.engine import FTEngine
+    d = dev()
+    M, N = 4090, 4081
+    A = torch.randn(M, K, dtype=torch.float64, device=d)
+    B = torch.randn(K, N, dtype=torch.float64, device=d)
+    C = torch.randn(M, N, dtype=torch.float64, device=d)
+    ref = 0.75 * (A @ B) - 0.5 * C
+    bound = 0.75 * (A.abs() @ B.abs()) + 0.5 * C.abs()
+    if layout == "tt":
+        A, B = A.t().contiguous().t(), B.t().contiguous().t()
+    eng = FTEngine(2, 2, 1)
+    eng.gemm(A, B, C, alpha=0.75, beta=-0.5, precision=precision)
+    u = 2 * U64 if precision == "fp64" else U32
+    assert bool(((C - ref).abs() <= (K + 3) * u * bound).all())
+    eng.close()
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 2, 2 ** 22 + 5),
                                    (2, 35, 2 ** 22 - 64)])
 def test_split_product_of_long_rows(M, N, K):

@@ -27,8 +27,10 @@
 // tile of at most 192 rows or columns runs fewer MFMAs and comes after the
 // whole tiles in the launch, to fill its last round.
 //
-// Bound: the matrix cores, 66% busy on a CU at work; the rest is the start
-// and the stores of a tile, which one workgroup per CU does not overlap.
+// Bound: the matrix cores, by counters at n = 114 60% (ladders) to 67% (rings)
+// busy on a CU at work and 50 to 55% over a launch, whose CUs work 82 to 86%
+// of the time; the rest is the start and the stores of a tile, which one
+// workgroup per CU does not overlap, and the last round of tiles.
 // The five products of a residual, ms: n = 114 17.65 -> 15.84 (1.21 PFLOP/s
 // of bf16 MFMAs; a library bf16 product reaches 1.36 at its power limit),
 // n = 66 2.32 -> 2.15, against two stages of 32 K.  Tried: the same with

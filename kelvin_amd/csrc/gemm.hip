@@ -782,7 +782,9 @@ Plan plan_of(const Gemm *g, const int *cblk, int n, bool f32) {
     const int64_t tiles = tiles_of(g[0], t);
     const bool tight = (double)M * N * g[0].nb1 * g[0].nb2 >=
                        0.94 * (double)tiles * t.m * t.n;
-    if (tiles >= 1024 && (pol != 0 || tight)) return Plan{t, whole};
+    // (a larger split_target asks FP32 for more partial sums)
+    const int fill = f32 ? std::max(1024, g[0].split_target) : 1024;
+    if (tiles >= fill && (pol != 0 || tight)) return Plan{t, whole};
   }
   double us = 1e300;
   for (const Tile &t : cand) {

@@ -162,10 +162,12 @@ def test_fp32_products_add_up_in_fp64(M, N, K, batch, layout):
         a = torch.ones(batch, c, r, dtype=torch.float64, device=d)
         return a.transpose(1, 2) if t == "t" else a.reshape(batch, r, c)
     eng = FTEngine(2, 2, 1)
-    C = torch.zeros(batch, M, N, dtype=torch.float64, device=d)
-    eng.gemm(ones(M, K, layout[0]), x * ones(K, N, layout[1]), C,
-             precision="fp32")
-    assert bool((C == K * x).all())
+    for plan in ((0, 1024), (1, 1024), (2, 2048)):
+        eng.set_gemm_plan(*plan)
+        C = torch.zeros(batch, M, N, dtype=torch.float64, device=d)
+        eng.gemm(ones(M, K, layout[0]), x * ones(K, N, layout[1]), C,
+                 precision="fp32")
+        assert bool((C == K * x).all()), plan
     eng.close()
 
 

@@ -872,7 +872,8 @@ int64_t level_extent(const PackIdx &l, int n) {
 bool lowp_ok(const ftcc_ctx *c, const Gemm &g) {
   if (c->adj_prec != FTCC_PREC_BF16X3) return false;
   const double flops = 2.0 * g.M * (double)g.N * g.K;
-  return flops >= c->adj_lowp_min_flops && g.nb2 == 1 && !g.mmap && !g.nmap && !g.D && !g.rmap && !g.cmap && g.K >= 1;
+  return flops >= c->adj_lowp_min_flops && g.nb2 == 1 && !g.mmap &&
+         !g.nmap && !g.D && !g.rmap && !g.cmap && g.K >= 1;
 }
 
 // doubles of a block's split operands and of its offset tables in the

@@ -1160,11 +1160,9 @@ bool try_spin(ftcc_ctx *c, const std::vector<int> &lo,
   const int O = c->no, V = c->nv;
   hipStream_t s = c->stream;
   c->spin = 0;
-  if (!c->d_lab_o) {
-    c->d_lab_o = (int *)dalloc(c, (O + 1) / 2 + 1);
-    c->d_lab_v = (int *)dalloc(c, (V + 1) / 2 + 1);
-    c->d_jl = (int *)dalloc(c, (O + 1) / 2 + 1);
-  }
+  if (!c->d_lab_o) c->d_lab_o = (int *)dalloc(c, (O + 1) / 2 + 1);
+  if (!c->d_lab_v) c->d_lab_v = (int *)dalloc(c, (V + 1) / 2 + 1);
+  if (!c->d_jl) c->d_jl = (int *)dalloc(c, (O + 1) / 2 + 1);
   FTCC_CHECK_HIP(hipMemcpyAsync(c->d_lab_o, lo.data(), sizeof(int) * O,
                                 hipMemcpyHostToDevice, s));
   FTCC_CHECK_HIP(hipMemcpyAsync(c->d_lab_v, lv.data(), sizeof(int) * V,
@@ -1274,30 +1272,33 @@ bool try_spin(ftcc_ctx *c, const std::vector<int> &lo,
 }
 
 void ensure_integrals(ftcc_ctx *c) {
-  if (c->F[0]) return;
   const int O = c->no, V = c->nv;
   const int64_t VO = (int64_t)V * O, VV = (int64_t)V * V, OO = (int64_t)O * O;
   const int64_t S2 = VV * OO;
-  c->F[0] = dalloc(c, OO);
-  c->F[1] = dalloc(c, VO);
-  c->F[2] = dalloc(c, VO);
-  c->F[3] = dalloc(c, VV);
+  // (each by itself: one that failed is taken by the next call)
+  auto take = [&](double *&p, int64_t n) {
+    if (!p) p = dalloc(c, n);
+  };
+  take(c->F[0], OO);
+  take(c->F[1], VO);
+  take(c->F[2], VO);
+  take(c->F[3], VV);
   const int64_t isz[9] = {VV * VV, VV * VO, VO * VV, S2, S2,
                           S2,      V * OO * O, OO * VO, OO * OO};
-  for (int k = 0; k < 9; ++k) c->I[k] = dalloc(c, isz[k]);
-  c->oovv_ring = dalloc(c, S2);
-  c->oovvT = dalloc(c, S2);
-  c->oovv_mefn = dalloc(c, S2);
-  c->vovv_aefm = dalloc(c, VO * VV);
-  c->ovvo_ring = dalloc(c, S2);
-  c->ovvo_ringT = dalloc(c, S2);
-  c->ooov_p1 = dalloc(c, OO * VO);
-  c->ooov_iemn = dalloc(c, OO * VO);
-  c->ooov_emnj = dalloc(c, OO * VO);
-  c->vovv_embf = dalloc(c, VO * VV);
-  c->fovT = dalloc(c, VO);
-  c->eo = dalloc(c, O);
-  c->ev = dalloc(c, V);
+  for (int k = 0; k < 9; ++k) take(c->I[k], isz[k]);
+  take(c->oovv_ring, S2);
+  take(c->oovvT, S2);
+  take(c->oovv_mefn, S2);
+  take(c->vovv_aefm, VO * VV);
+  take(c->ovvo_ring, S2);
+  take(c->ovvo_ringT, S2);
+  take(c->ooov_p1, OO * VO);
+  take(c->ooov_iemn, OO * VO);
+  take(c->ooov_emnj, OO * VO);
+  take(c->vovv_embf, VO * VV);
+  take(c->fovT, VO);
+  take(c->eo, O);
+  take(c->ev, V);
 }
 
 // Residual workspace: as many grid points per chunk as fit the budget
@@ -1355,22 +1356,28 @@ void ensure_workspace(ftcc_ctx *c) {
   c->nb = nb;
   c->nb_alloc = nb;
   c->ws_prec = c->prec;
-  c->aring = dalloc(c, S2 * nb);
-  c->wr = dalloc(c, S2 * nb);
-  c->z = dalloc(c, S2 * nb);
-  c->s1 = dalloc(c, S2 * nb);
-  c->s2 = dalloc(c, S2 * nb);
-  c->wmnij = dalloc(c, OO * OO * nb);
-  c->wabef = dalloc(c, VV * VV * nb);
-  c->u = dalloc(c, OO * VO * nb);
-  c->t1T = dalloc(c, VO * nb);
-  c->Fme = dalloc(c, VO * nb);
-  c->FmeT = dalloc(c, VO * nb);
-  c->Fae = dalloc(c, VV * nb);
-  c->Fmi = dalloc(c, OO * nb);
-  c->Fbe = dalloc(c, VV * nb);
-  c->Fmj = dalloc(c, OO * nb);
-  c->ytmp = dalloc(c, sm * nb);
+  try {
+    c->aring = dalloc(c, S2 * nb);
+    c->wr = dalloc(c, S2 * nb);
+    c->z = dalloc(c, S2 * nb);
+    c->s1 = dalloc(c, S2 * nb);
+    c->s2 = dalloc(c, S2 * nb);
+    c->wmnij = dalloc(c, OO * OO * nb);
+    c->wabef = dalloc(c, VV * VV * nb);
+    c->u = dalloc(c, OO * VO * nb);
+    c->t1T = dalloc(c, VO * nb);
+    c->Fme = dalloc(c, VO * nb);
+    c->FmeT = dalloc(c, VO * nb);
+    c->Fae = dalloc(c, VV * nb);
+    c->Fmi = dalloc(c, OO * nb);
+    c->Fbe = dalloc(c, VV * nb);
+    c->Fmj = dalloc(c, OO * nb);
+    c->ytmp = dalloc(c, sm * nb);
+  } catch (const Error &) {
+    free_workspace(c);   // none of it half made
+    (void)hipGetLastError();
+    throw;
+  }
 }
 
 // Release the residual workspace and the operand copies sized by it (they
@@ -1467,10 +1474,8 @@ void residual_chunk(ftcc_ctx *c, const double *t1, const double *t2,
   } else {
     // dense layout (also a spin-blocked system's rare dense fallback):
     // tau and t2r are formed whole
-    if (!c->tau) {
-      c->tau = dalloc(c, S2 * c->nb_alloc);
-      c->t2r = dalloc(c, S2 * c->nb_alloc);
-    }
+    if (!c->tau) c->tau = dalloc(c, S2 * c->nb_alloc);
+    if (!c->t2r) c->t2r = dalloc(c, S2 * c->nb_alloc);
     PrepOut po{c->tau, c->t2r, c->aring};
     prep_amplitudes(t1, t2, V, O, nb, po, s);
     put_operand(c, OP_TAU_A, c->tau, OO, 1, S2, nb);
@@ -2610,11 +2615,8 @@ int ftcc_td_step(ftcc_ctx *c, int order, double h, int singles, double *T1,
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
     const int64_t len[2] = {VO * c->ng, S2 * c->ng};
     for (int k = 0; k < 2; ++k)
-      if (!c->td_var[k]) {
-        c->td_var[k] = dalloc(c, len[k]);
-        c->td_acc[k] = dalloc(c, len[k]);
-        c->td_k[k] = dalloc(c, len[k]);
-      }
+      for (double **p : {&c->td_var[k], &c->td_acc[k], &c->td_k[k]})
+        if (!*p) *p = dalloc(c, len[k]);
     // kelvin/propagation.py:5-52: rk1 (Euler), rk2 (Heun), rk4 (classical)
     static const double b1[1] = {1.0}, b2[2] = {0.5, 0.5},
                         b4[4] = {1.0 / 6, 1.0 / 3, 1.0 / 3, 1.0 / 6};
@@ -2650,14 +2652,10 @@ int ftcc_td_implicit_step(ftcc_ctx *c, int scheme, double h, int max_iter,
     hipStream_t s = c->stream;
     const int64_t VO = (int64_t)c->nv * c->no, S2 = VO * VO;
     const int64_t len[2] = {VO * c->ng, S2 * c->ng};
-    for (int k = 0; k < 2; ++k) {
-      if (!c->td_var[k]) {
-        c->td_var[k] = dalloc(c, len[k]);
-        c->td_acc[k] = dalloc(c, len[k]);
-        c->td_k[k] = dalloc(c, len[k]);
-      }
-      if (!c->td_k1[k]) c->td_k1[k] = dalloc(c, len[k]);
-    }
+    for (int k = 0; k < 2; ++k)
+      for (double **p : {&c->td_var[k], &c->td_acc[k], &c->td_k[k],
+                         &c->td_k1[k]})
+        if (!*p) *p = dalloc(c, len[k]);
     double *T[2] = {T1, T2};
     auto pass = [&](int k, int mode) {
       UpdateArgs a = upd(c);

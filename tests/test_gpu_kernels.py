@@ -125,6 +125,53 @@ def test_gemm_of_1024_wide_tiles(layout, precision, K):
     eng.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "bf16x3"])
+@pytest.mark.parametrize("spin", [True, False])
+def test_engine_goes_on_after_any_failed_allocation(spin, precision,
+                                                    monkeypatch):
+    """Integrals, residual and a propagation step with memory that ends
+    somewhere on the way, then again with enough: what was allocated before
+    the failure is complete or taken again."""
+    from kelvin_amd._lib import FTCCError
+    from kelvin_amd.engine import FTEngine
+    from kelvin_amd.ov_blocks import one_e_blocks, two_e_blocks
+    d = dev()
+    ng = 3
+    rng = numpy.random.default_rng(8)
+    no, nv, (F, I, t1, t2, lo, lv) = _run_problem(((2, 3), (5, 4)), ng, rng)
+    T1, T2 = (torch.as_tensor(x, device=d) for x in (t1, t2))
+    one = one_e_blocks(**{k: F[k] for k in ('oo', 'ov', 'vo', 'vv')})
+    two = two_e_blocks(**{k: I[k] for k in I})
+
+    def use(eng):
+        eng.set_blocks(one, two)
+        eng.set_denominators(numpy.ones((nv, no)),
+                             numpy.ones((nv, nv, no, no)))
+        eng.set_grid(numpy.zeros(ng), numpy.zeros((ng, ng)))
+        if spin:
+            eng.set_spin(lo, lv)
+        out = [torch.empty_like(T1), torch.empty_like(T2)]
+        eng.residual(T1, T2, *out)
+        out += [T1.clone(), T2.clone()]
+        eng.td_step(out[2], out[3], 0.01, order=4)
+        return [to_np(x) for x in out]
+    eng = FTEngine(no, nv, ng, precision=precision)
+    least = eng.workspace_bytes()
+    ref = use(eng)
+    most = eng.workspace_bytes()
+    eng.close()
+    for part in numpy.linspace(0.01, 0.99, 25):
+        eng = FTEngine(no, nv, ng, precision=precision)
+        with monkeypatch.context() as m:
+            m.setenv("FTCC_CONTEXT_GB",
+                     repr((least + part * (most - least)) / 2.0 ** 30))
+            with pytest.raises(FTCCError, match="FTCC_CONTEXT_GB"):
+                use(eng)
+        for x, y in zip(use(eng), ref):
+            assert rel(x, y) < 1e-13, part
+        eng.close()
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 2, 2 ** 22 + 5),
                                    (2, 35, 2 ** 22 - 64)])
 def test_split_product_of_long_rows(M, N, K):

@@ -67,6 +67,17 @@ void dfree(ftcc_ctx *c, void *p) {
 }
 
 
+// p holds at least n doubles (the grid of a context may grow)
+void ensure_len(ftcc_ctx *c, double *&p, int64_t n) {
+  if (p && c->alloc_doubles.at(p) >= n) return;
+  if (p) {
+    FTCC_CHECK_HIP(hipStreamSynchronize(c->stream));
+    dfree(c, p);
+    p = nullptr;
+  }
+  p = dalloc(c, n);
+}
+
 int64_t p4(int a, int b, int c, int d) {
   return (int64_t)a * b * c * d;
 }
@@ -2616,7 +2627,7 @@ int ftcc_td_step(ftcc_ctx *c, int order, double h, int singles, double *T1,
     const int64_t len[2] = {VO * c->ng, S2 * c->ng};
     for (int k = 0; k < 2; ++k)
       for (double **p : {&c->td_var[k], &c->td_acc[k], &c->td_k[k]})
-        if (!*p) *p = dalloc(c, len[k]);
+        ensure_len(c, *p, len[k]);
     // kelvin/propagation.py:5-52: rk1 (Euler), rk2 (Heun), rk4 (classical)
     static const double b1[1] = {1.0}, b2[2] = {0.5, 0.5},
                         b4[4] = {1.0 / 6, 1.0 / 3, 1.0 / 3, 1.0 / 6};
@@ -2655,7 +2666,7 @@ int ftcc_td_implicit_step(ftcc_ctx *c, int scheme, double h, int max_iter,
     for (int k = 0; k < 2; ++k)
       for (double **p : {&c->td_var[k], &c->td_acc[k], &c->td_k[k],
                          &c->td_k1[k]})
-        if (!*p) *p = dalloc(c, len[k]);
+        ensure_len(c, *p, len[k]);
     double *T[2] = {T1, T2};
     auto pass = [&](int k, int mode) {
       UpdateArgs a = upd(c);

@@ -304,6 +304,24 @@ def test_blocked_residual_at_class_and_run_edges(prec, tol, runs, workspace,
     eng.close()
 
 
+def test_propagation_after_a_longer_grid():
+    """Propagation steps with one slice and then, on the same engine, with
+    five: every slice like the single one, to rounding."""
+    d = dev()
+    rng = numpy.random.default_rng(2)
+    no, nv, (F, I, t1, t2, lo, lv) = _run_problem(((2, 3), (5, 4)), 1, rng)
+    eng = _run_engine(F, I, no, nv, 1, lo, lv, "fp64")
+    one = [torch.as_tensor(x, device=d) for x in (t1, t2)]
+    five = [torch.cat([x] * 5) for x in one]
+    eng.td_step(*one, 0.01, order=4)
+    eng.set_grid(numpy.zeros(5), numpy.zeros((5, 5)))
+    eng.td_step(*five, 0.01, order=4)
+    for x, y in zip(one, five):
+        for k in range(5):
+            assert rel(to_np(y[k]), to_np(x[0])) < 1e-13
+    eng.close()
+
+
 # compositions of one (no, nv): the classes of the second need longer operand
 # slots than those of the first, a longer operand set in the third pair
 _RELABEL = [[((3, 4), (11, 8)), ((3, 4), (10, 9))],
